@@ -334,6 +334,7 @@ struct EngineOptions {
   int window = kDefaultWindow;           // DSM_OPT_WINDOW
   int graph = 0;                         // DSM_OPT_GRAPH
   int wide_pair = 1;                     // DSM_OPT_WIDE_PAIR
+  int lane = 1;                          // DSM_OPT_LANE
 };
 
 struct dsm_engine {
@@ -379,6 +380,9 @@ struct dsm_engine {
   int* d_work = nullptr;
   int d_work_cap = 0;
   int* d_cnt = nullptr;     // [kNumLists] list counts, then [kNumLists] queues
+  float* d_rec = nullptr;  // lane form: one record per strand slot
+  int64_t d_rec_cap = 0;
+  float* d_lane_tab = nullptr;
   unsigned long long* d_counters = nullptr;
   int* d_corr_cnt = nullptr;
   int d_corr_cnt_cap = 0;
@@ -572,6 +576,77 @@ int ensure_stage(dsm_engine* e) {
   return DSM_OK;
 }
 
+// The lane form (dsm_lane.h) covers everything but flow, whose affine step changes every
+// rate of a chain at every jump.
+bool lane_capable(const Ens& E) { return !E.P.flow && E.P.sample_mode != kSampleFlow; }
+
+// Quads per chain with which a batched pass over these ensembles runs in the lane form, or
+// 0 when it runs in the others.  The chains have to fit the largest size, 128 positions,
+// with five standard deviations of the equilibrium Z (binomial) to spare (one that outgrows
+// the size chosen finishes in the wave form).
+int lane_quads(const dsm_engine* e, const std::vector<int>& ids) {
+  if (e->opt.lane == 0 || ids.empty()) return 0;
+  double n = 0.0, zcap = 0.0;
+  for (int id : ids) {
+    const Ens& E = e->ens[id];
+    if (!lane_capable(E)) return 0;
+    const double b = E.P.beta, nk = E.nmax;
+    n += E.n;
+    zcap = std::max(zcap, std::min(nk, (nk + b) / (1.0 + b) + 5.0 * std::sqrt((nk - 1.0) * b) / (1.0 + b)));
+  }
+  int quads = 0;
+  for (int q : kLaneQuads)
+    if (4 * q > zcap) { quads = q; break; }
+  // A wave's step costs nearly the same for one chain as for 64, so the form needs chains:
+  // it passes the row form (four chains a wave) at about 32,000 chains (one 16 tau_K window,
+  // Nk 100: 3.36 against 3.38 ms; 24,000: 3.14 / 2.72; 48,000: 3.63 / 4.58; Nk 50 at about
+  // 38,000, Nk 25 at 30,000) and the pair form (two a wave, from Z = 64 on) at about 14,000
+  // (Nk 150: 4.38 against 4.90 ms at 16,000).
+  if (e->opt.lane == 1 && n < (quads >= 24 ? 14000 : 36000)) return 0;
+  return quads;
+}
+
+// Its working memory: a record per strand slot, allocated when a pass first can use it,
+// and its rate tables for short strands.  It gives way to anything else: not taken beyond
+// a quarter of the free device memory, and given back when an allocation fails (the other
+// forms then run).
+void release_lane(dsm_engine* e) {
+  if (!e->d_rec) return;
+  e->gen++;
+  (void)hipStreamSynchronize(e->st);
+  (void)hipFree(e->d_rec);
+  e->d_rec = nullptr;
+  e->d_rec_cap = 0;
+}
+int ensure_lane(dsm_engine* e, const std::vector<int>& ids) {
+  if (!lane_quads(e, ids)) return DSM_OK;
+  if (!e->d_lane_tab) {
+    std::vector<float> t, out((size_t)kLaneTabFloats, 0.0f);
+    build_tables(t, kLaneN, 1.0f, 0, 0.0f);
+    const int n = kLaneN + 2;
+    for (int N = 1; N < kLaneN; ++N)
+      for (int q = 0; q < 4; ++q) out[4 * N + q] = t[(size_t)q * n + N];
+    for (int x = 1; x < kLaneFR; ++x) out[4 * kLaneN + x] = t[(size_t)kNumTables * n + x];
+    int rc = dev_alloc(&e->d_lane_tab, out.size());
+    if (rc) return rc;
+    HIPCHK(hipMemcpy(e->d_lane_tab, out.data(), sizeof(float) * out.size(), hipMemcpyHostToDevice));
+  }
+  if (e->nstr > e->d_rec_cap) {
+    release_lane(e);
+    const size_t bytes = sizeof(float) * kLaneRecFloats * (size_t)e->nstr;
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || bytes > free_b / 4) return DSM_OK;
+    if (hipMalloc((void**)&e->d_rec, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      e->d_rec = nullptr;
+      return DSM_OK;
+    }
+    e->gen++;
+    e->d_rec_cap = e->nstr;
+  }
+  return DSM_OK;
+}
+
 Ens* get_ens(dsm_engine* e, int id) {
   if (!e || id < 0 || id >= (int)e->ens.size() || !e->ens[id].live) return nullptr;
   return &e->ens[id];
@@ -647,6 +722,8 @@ KmcArgs base_args(dsm_engine* e) {
   a.stage = e->d_stage;
   a.use_ev_stop = 0;
   a.lds_floats = 0;
+  a.rec = e->d_rec;
+  a.lane_tab = e->d_lane_tab;
   return a;
 }
 
@@ -668,6 +745,8 @@ int chain_totals(dsm_engine* e, const std::vector<int>& ids, unsigned long long 
 struct Pass {
   int n0 = 0;  // entries of the bin-0 list
   int bin_max = 0;
+  int lane_quads = 0;       // > 0: the lane form with this many quads per chain
+  int nmax = 0;
   bool concurrent = false;  // batched passes only: split by Z, geometries side by side
   int n_ens = 0;
   int n_live = 0;           // chains of the pass
@@ -695,11 +774,15 @@ int pass_setup(dsm_engine* e, const std::vector<int>& ids, bool use_ev_stop, Pas
   ps.bin_max = bin_max;
   ps.n_ens = (int)ids.size();
   ps.n_live = (int)n_all;
+  ps.lane_quads = batched && e->d_rec_cap >= e->nstr ? lane_quads(e, ids) : 0;
+  ps.nmax = 0;
+  for (int id : ids) ps.nmax = std::max(ps.nmax, e->ens[id].nmax);
   // geometries side by side when chains beyond the first wave-form geometry can occur
   // (their runs are long and few) or when many chains are expected above the row form's
   // 63 positions (the pair form then carries the bulk)
   ps.concurrent = e->opt.concurrent >= 0 ? (e->opt.concurrent > 0 && bin_max >= 1)
                                          : (bin_max >= 3 || (bin_max >= 1 && z_est >= 56.0 * n_all));
+  if (ps.lane_quads) ps.concurrent = false;
   if (n0 == 0) return DSM_OK;
   ps.range = batched && !ps.concurrent && ids.size() == 1;
   ps.first = e->ens[ids[0]].chain0;
@@ -850,16 +933,19 @@ int pass_bins(dsm_engine* e, Pass& ps, bool plain, bool timed, dsm_run_stats* rs
   // (1.79 us per jump against 2.84 us per row-form step of four chains).  Measured:
   // 1000 chains of Nk 25 +15%, of Nk 100 +92%; 4096 chains of Nk 25 -14%.
   const bool small = !plain && ps.n_live <= e->opt.small_per_cu * e->n_cu;
-  const bool zorder = !plain && (ps.n_ens == 1 || small);
+  const bool lane = !plain && ps.lane_quads > 0 && !small;
+  const bool zorder = !plain && (ps.n_ens == 1 || small || lane);
   constexpr int kZList = kNumLists - 1;
   if (zorder)
     HIPCHK(launch_z_order(ps.range ? nullptr : e->d_work, ps.first, ps.range ? ps.n_live : ps.n0, e->ch.Z,
-                          e->ch.stall, cnt + 2 * kNumLists, e->d_work + (size_t)kZList * e->d_work_cap,
+                          e->ch.stall, lane ? (ps.lane_quads + 3) / 4 : 4, cnt + 2 * kNumLists, e->d_work + (size_t)kZList * e->d_work_cap,
                           cnt + kZList, e->st));
   if (small) {  // the compact ordered list feeds the wave form directly
     ns = 0;
     for (int b = kLateFirst; b <= late_last(ps.bin_max); ++b) seq[ns++] = b;
   }
+  // lane form first, then the wave form for chains that outgrew it, if their length allows
+  if (lane && ps.nmax < 4 * ps.lane_quads) ns = 1;
   for (int k = 0; k < ns; ++k) {
     const int b = seq[k], nb = k + 1 < ns ? seq[k + 1] : b + 1;
     const int in = (k == 0 && zorder) ? kZList : b;
@@ -868,9 +954,16 @@ int pass_bins(dsm_engine* e, Pass& ps, bool plain, bool timed, dsm_run_stats* rs
     a.queue = cnt + kNumLists + in;
     a.overflow = e->d_work + (size_t)nb * e->d_work_cap;
     a.n_overflow = cnt + nb;
-    const int grid = device_blocks(e, b, plain, a.lds_floats, a.ext != 0);
     if (timed) HIPCHK(hipEventRecord(e->lev[2 * k], e->st));
-    HIPCHK(launch_kmc(a, b, plain, grid, e->st));
+    if (k == 0 && lane) {
+      // one workgroup per CU; as many lanes as give every wave the same number of rounds
+      const int most = lane_max_lanes(ps.lane_quads), waves = kLaneWaves * e->n_cu;
+      const int rounds = (ps.n_live + waves * most - 1) / (waves * most);
+      a.lanes = std::max(1, (ps.n_live + waves * rounds - 1) / (waves * rounds));
+      HIPCHK(launch_kmc_lane(a, ps.lane_quads, e->n_cu, e->st));
+    } else {
+      HIPCHK(launch_kmc(a, b, plain, device_blocks(e, b, plain, a.lds_floats, a.ext != 0), e->st));
+    }
     if (timed) HIPCHK(hipEventRecord(e->lev[2 * k + 1], e->st));
     rs->kmc_launches++;
     if (k == 0) rs->first_launches++;
@@ -1087,7 +1180,14 @@ int advance_impl(dsm_engine* e, const std::vector<int>& ids, const std::vector<d
         if (s <= 0) s = (int)std::ceil(std::log(te / E.P.delta / E.p) / std::log((double)E.m)) + 1;
         if (s < 1) s = 1;
         if (s > 40) return fail(DSM_ERR_ARG, "correlator needs %d levels (max 40)", s);
-        if ((rc = corr_alloc(e, E, s))) return rc;
+        if ((rc = corr_alloc(e, E, s))) {
+          if (rc != DSM_ERR_MEMORY || !e->d_rec) return rc;
+          release_lane(e);
+          if (E.dD) (void)hipFree(E.dD);
+          if (E.dA) (void)hipFree(E.dA);
+          E.dD = E.dA = E.dC = nullptr;
+          if ((rc = corr_alloc(e, E, s))) return rc;
+        }
       }
     } else if (E.P.sample_mode == kSampleFlow) {
       k_target[q] = (int64_t)std::ceil(te / E.P.delta - 1e-12) + 1;
@@ -1095,6 +1195,7 @@ int advance_impl(dsm_engine* e, const std::vector<int>& ids, const std::vector<d
   }
   const double t0_prog = 0.0;
   (void)t0_prog;
+  if (mode == DSM_MODE_BATCHED && (rc = ensure_lane(e, ids))) return rc;
   std::vector<char> reached(ids.size(), 0);
   for (;;) {
     // next window: each ensemble advances to its window end, the last one to t_end
@@ -1312,7 +1413,7 @@ int dsm_destroy(dsm_engine* e) {
   ChainArrays& c = e->ch;
   void* ptrs[] = {c.Z, c.nk, c.ens, c.cap, c.stall, c.cid, c.local, c.base, c.t, c.ev, c.dt_prev, c.next_sample, c.ev_stop, c.zsum, c.R1,
                   c.Qx, c.Qy, c.Qz, c.N, c.w, e->d_ens, e->d_tabs, e->d_stage, e->d_work, e->d_cnt, e->d_counters,
-                  e->d_corr_cnt, e->d_red, e->d_rows, e->d_healthy, e->d_part};
+                  e->d_corr_cnt, e->d_red, e->d_rows, e->d_healthy, e->d_part, e->d_rec, e->d_lane_tab};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (auto& ev : e->evs)
@@ -1404,6 +1505,12 @@ int dsm_add_ensemble(dsm_engine* e, const dsm_ensemble_desc* d, int32_t* ens_id)
   P.s_At = pc.s_At; P.s_Ct = pc.s_Ct; P.s_Dt = pc.s_Dt; P.s_Adt = pc.s_Adt; P.s_Bdt = pc.s_Bdt;
   P.s_Cdt = pc.s_Cdt; P.s_Ddt = pc.s_Ddt; P.s_taud_inv = pc.s_taud_inv; P.s_one_minus_g = pc.s_one_minus_g;
   {
+    const float ft[5] = {pc.s_At, pc.s_Ct, pc.s_Dt, pc.s_taud_inv, pc.s_one_minus_g};
+    const float fdt[5] = {pc.s_Adt, pc.s_Bdt, pc.s_Cdt, pc.s_Ddt, pc.s_taud_inv};
+    std::copy(ft, ft + 5, P.law_ft);
+    std::copy(fdt, fdt + 5, P.law_fdt);
+  }
+  {
     const double pcut = 1.0 / (1.0 + (double)d->beta);
     double Tc = std::floor(pcut * 4294967296.0);
     if (Tc > 4294967295.0) Tc = 4294967295.0;
@@ -1442,14 +1549,22 @@ int dsm_add_ensemble(dsm_engine* e, const dsm_ensemble_desc* d, int32_t* ens_id)
   E.stage_floats = (int64_t)E.window * E.n * E.ncomp;
   P.stage_off = e->stage_space.take(E.stage_floats);
   e->stage_used = std::max(e->stage_used, e->stage_space.end);
-  if ((rc = ensure_stage(e))) return rc;
+  if ((rc = ensure_stage(e))) {
+    if (rc != DSM_ERR_MEMORY || !e->d_rec) return rc;
+    release_lane(e);
+    if ((rc = ensure_stage(e))) return rc;
+  }
   // chains
   E.chain0 = (int)e->chain_space.take(E.n);
   E.nstrand = 0;
   for (int i = 0; i < E.n; ++i) E.nstrand += cap_of(E.nk[i]);
   P.chain0 = E.chain0;
   E.strand0 = e->strand_space.take(E.nstrand);
-  if ((rc = grow_chains(e, (int)e->chain_space.end, e->strand_space.end))) return rc;
+  if ((rc = grow_chains(e, (int)e->chain_space.end, e->strand_space.end))) {
+    if (rc != DSM_ERR_MEMORY || !e->d_rec) return rc;
+    release_lane(e);
+    if ((rc = grow_chains(e, (int)e->chain_space.end, e->strand_space.end))) return rc;
+  }
   {
     const int id = (int)e->ens.size();
     std::vector<int> hnk(E.n), hens(E.n, id), hcap(E.n), hzero(E.n, 0), hloc(E.n);
@@ -1665,6 +1780,7 @@ int dsm_advance_events(dsm_engine* e, int32_t ens, int64_t n_events, int32_t mod
   if (rc) return rc;
   Timer T;
   dsm_run_stats rs{};
+  if (mode == DSM_MODE_BATCHED && (rc = ensure_lane(e, {ens}))) return rc;
   unsigned long long before[2];
   if ((rc = chain_totals(e, {ens}, before))) return rc;
   E->P.t_end = INFINITY;
@@ -1737,6 +1853,7 @@ int dsm_set_option(dsm_engine* e, int32_t key, int32_t value) {
     case DSM_OPT_BLOCKS_PER_CU: if (value < 0) break; o.blocks_per_cu = value; return DSM_OK;
     case DSM_OPT_WINDOW: if (value < 1) break; o.window = value; return DSM_OK;
     case DSM_OPT_GRAPH: if (value < 0 || value > 1) break; o.graph = value; return DSM_OK;
+    case DSM_OPT_LANE: if (value < 0 || value > 2) break; o.lane = value; return DSM_OK;
     case DSM_OPT_WIDE_PAIR: if (value < 0 || value > 1) break; o.wide_pair = value; return DSM_OK;
     default: return fail(DSM_ERR_ARG, "unknown option %d", key);
   }
@@ -1755,6 +1872,7 @@ int dsm_get_option(dsm_engine* e, int32_t key, int32_t* value) {
     case DSM_OPT_BLOCKS_PER_CU: *value = o.blocks_per_cu; return DSM_OK;
     case DSM_OPT_WINDOW: *value = o.window; return DSM_OK;
     case DSM_OPT_GRAPH: *value = o.graph; return DSM_OK;
+    case DSM_OPT_LANE: *value = o.lane; return DSM_OK;
     case DSM_OPT_WIDE_PAIR: *value = o.wide_pair; return DSM_OK;
     default: return fail(DSM_ERR_ARG, "unknown option %d", key);
   }

@@ -151,12 +151,12 @@ __global__ void split_geoms_kernel(const int* src, int n, const int* Z, const in
   }
 }
 
-// Row-form work list in decreasing Z (16 buckets of four; Z >= 64 first, stalled chains
-// last): the chains started last, at the end of a pass, are the shortest ones.
-__device__ __forceinline__ int zbucket(const int* Z, const int* stall, int c) {
+// Work list in decreasing Z (16 buckets of `width` positions; Z >= 16 * width first,
+// stalled chains last): the chains started last, at the end of a pass, are the shortest.
+__device__ __forceinline__ int zbucket(const int* Z, const int* stall, int width, int c) {
   if (stall[c] != 0) return 16;
   const int z = Z[c];
-  return z >= 64 ? 0 : 15 - (z >> 2);
+  return z >= 16 * width ? 0 : 15 - z / width;
 }
 constexpr int kZBuckets = 17;
 
@@ -164,13 +164,13 @@ constexpr int kZBuckets = 17;
 // global atomic on 17 counters serialises in L2).  Grid-stride over the elements.
 // src == null: the chains first .. first+n-1 (one ensemble's range)
 __global__ void __launch_bounds__(1024) zhist_kernel(const int* src, int first, int n, const int* Z, const int* stall,
-                                                     int* hist) {
+                                                     int width, int* hist) {
   __shared__ int lh[kZBuckets];
   if (threadIdx.x < kZBuckets) lh[threadIdx.x] = 0;
   __syncthreads();
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     const int c = src ? src[i] : first + i;
-    if (c >= 0) atomicAdd(lh + zbucket(Z, stall, c), 1);
+    if (c >= 0) atomicAdd(lh + zbucket(Z, stall, width, c), 1);
   }
   __syncthreads();
   if (threadIdx.x < kZBuckets && lh[threadIdx.x]) atomicAdd(hist + threadIdx.x, lh[threadIdx.x]);
@@ -187,13 +187,13 @@ __global__ void zscan_kernel(int* hist, int* n_out) {
 // Each block reserves its range of every bucket with one atomic, then places its
 // elements with LDS atomics (order within a bucket is arbitrary).
 __global__ void __launch_bounds__(1024) zscatter_kernel(const int* src, int first, int n, const int* Z,
-                                                        const int* stall, int* cursor, int* dst) {
+                                                        const int* stall, int width, int* cursor, int* dst) {
   __shared__ int lh[kZBuckets], base[kZBuckets];
   if (threadIdx.x < kZBuckets) lh[threadIdx.x] = 0;
   __syncthreads();
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     const int c = src ? src[i] : first + i;
-    if (c >= 0) atomicAdd(lh + zbucket(Z, stall, c), 1);
+    if (c >= 0) atomicAdd(lh + zbucket(Z, stall, width, c), 1);
   }
   __syncthreads();
   if (threadIdx.x < kZBuckets) {
@@ -204,7 +204,7 @@ __global__ void __launch_bounds__(1024) zscatter_kernel(const int* src, int firs
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     const int c = src ? src[i] : first + i;
     if (c >= 0) {
-      const int b = zbucket(Z, stall, c);
+      const int b = zbucket(Z, stall, width, c);
       dst[base[b] + atomicAdd(lh + b, 1)] = c;
     }
   }
@@ -880,13 +880,13 @@ hipError_t launch_init_counts(int* cnt, int n, int n0, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t launch_z_order(const int* src, int first, int n, const int* Z, const int* stall, int* scratch17, int* dst,
-                          int* n_out, hipStream_t st) {
+hipError_t launch_z_order(const int* src, int first, int n, const int* Z, const int* stall, int width, int* scratch17,
+                          int* dst, int* n_out, hipStream_t st) {
   if (n <= 0) return hipSuccess;
   const int blocks = n > 64 * 1024 * 4 ? 256 : (n + 4095) / 4096 + 1;  // a few elements per thread
-  hipLaunchKernelGGL(zhist_kernel, dim3(blocks), dim3(1024), 0, st, src, first, n, Z, stall, scratch17);
+  hipLaunchKernelGGL(zhist_kernel, dim3(blocks), dim3(1024), 0, st, src, first, n, Z, stall, width, scratch17);
   hipLaunchKernelGGL(zscan_kernel, dim3(1), dim3(64), 0, st, scratch17, n_out);
-  hipLaunchKernelGGL(zscatter_kernel, dim3(blocks), dim3(1024), 0, st, src, first, n, Z, stall, scratch17, dst);
+  hipLaunchKernelGGL(zscatter_kernel, dim3(blocks), dim3(1024), 0, st, src, first, n, Z, stall, width, scratch17, dst);
   return hipGetLastError();
 }
 

@@ -40,14 +40,29 @@ DSM_DECLARE_GEOM(7)
 // if row2, else the pair form) in one batched launch
 hipError_t launch_kmc_rowpair(const KmcArgs& row, const KmcArgs& pair, bool row2, int grid, hipStream_t st);
 int kmc_rowpair_occupancy(int lds_floats, bool ext, bool row2);
+// The lane form (one chain per lane, quads * 4 positions): persistent workgroups of
+// kLaneWaves waves that share the tables {SP, SM, PP, PM}[kLaneN], FR[kLaneFR].
+constexpr int kLaneN = 64, kLaneFR = 256;
+constexpr int kLaneTabFloats = 4 * kLaneN + kLaneFR;
+constexpr int kLaneRecFloats = 3;  // working memory per strand slot
+constexpr int kLaneWaves = 8;
+constexpr int kLaneQuads[] = {8, 12, 16, 19, 24, 28, 32};
+constexpr int kLaneLdsBytes = 160 * 1024;
+// most lanes of a wave whose columns (an odd number of them) fit the workgroup's LDS
+constexpr int lane_max_lanes(int quads) {
+  const int s = ((int)(kLaneLdsBytes / sizeof(float)) - kLaneTabFloats) / (kLaneWaves * 4 * quads);
+  const int odd = (s & 1) ? s : s - 1;
+  return odd > 64 ? 64 : odd;
+}
+hipError_t launch_kmc_lane(const KmcArgs& a, int quads, int grid, hipStream_t st);
 hipError_t launch_init_eq(const ChainArrays& ch, const EnsParams* ens, const float* tabs, const int* chains, int n,
                           hipStream_t st);
 hipError_t launch_fill_u32(void* p, uint32_t v, int64_t n, hipStream_t st);
 hipError_t launch_iota(int* p, int start, int n, hipStream_t st);
 // the chains of src (entries < 0 skipped; src == null: chains first .. first+n-1) into
-// dst in decreasing Z; *n_out = their count.  scratch17 (17 ints) must be zero.
-hipError_t launch_z_order(const int* src, int first, int n, const int* Z, const int* stall, int* scratch17, int* dst,
-                          int* n_out, hipStream_t st);
+// dst in decreasing Z (buckets of `width` positions, the first from 16 * width on); *n_out = their count.  scratch17 (17 ints) must be zero.
+hipError_t launch_z_order(const int* src, int first, int n, const int* Z, const int* stall, int width, int* scratch17,
+                          int* dst, int* n_out, hipStream_t st);
 // cnt[0] = n0, cnt[1..n) = 0
 hipError_t launch_init_counts(int* cnt, int n, int n0, hipStream_t st);
 hipError_t launch_split_geoms(const int* src, int n, const int* Z, const int* stall, int* lists, int cap,

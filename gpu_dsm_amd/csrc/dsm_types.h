@@ -11,6 +11,7 @@
 // Strand i of a chain is read by lane i%64 of slot i/64 of the wave that owns
 // the chain, so a load of one slot is a contiguous 256-byte access per array.
 #pragma once
+#include <hip/hip_runtime.h>
 #include <stdint.h>
 
 namespace dsm {
@@ -34,6 +35,9 @@ struct EnsParams {
   float kappa[9];
   float c_create;
   float s_At, s_Ct, s_Dt, s_Adt, s_Bdt, s_Cdt, s_Ddt, s_taud_inv, s_one_minus_g;
+  // the CD lifetime samplers' constants in the order of a partner table entry: s_At s_Ct
+  // s_Dt s_taud_inv s_one_minus_g and s_Adt s_Bdt s_Cdt s_Ddt s_taud_inv
+  float law_ft[5], law_fdt[5];
   uint32_t cut_threshold;
   uint32_t key0, key1;
   int tab_off;       // float offset of SP in the table arena
@@ -96,6 +100,9 @@ struct KmcArgs {
   int lds_floats;       // per-wave LDS table copy size (0: tables read from global memory)
   int ext;              // an ensemble of the pass samples MSD(t), has a polydisperse CD background or flows
   int plain_jumps;      // plain form: jumps per chain per launch
+  float* rec;           // lane form: a record {|Q|^2, w, N} per strand slot
+  const float* lane_tab;  // lane form: the rate tables that depend on N alone, for short strands
+  int lanes;            // lane form: lanes of a wave that take chains (1..64)
 };
 
 }  // namespace dsm

@@ -109,6 +109,8 @@ int dsm_mem_info(int32_t device_id, size_t* free_bytes, size_t* total_bytes);
 #define DSM_OPT_WIDE_PAIR 9         /* concurrent pass of one ensemble: chains with 128 <= Z < 240 run two
                                        per wave and those with 64 <= Z < 128 four (1), or one and two (0)
                                        (1) */
+#define DSM_OPT_LANE 10             /* batched equilibrium passes whose chains stay short enough run one chain
+                                       per lane: 1 by the pass's chain count, 0 never, 2 always (1) */
 int dsm_set_option(dsm_engine* e, int32_t key, int32_t value);
 int dsm_get_option(dsm_engine* e, int32_t key, int32_t* value);
 
