@@ -387,10 +387,9 @@ struct dsm_engine {
   int* d_corr_cnt = nullptr;
   int d_corr_cnt_cap = 0;
   double* d_red = nullptr;
-  int d_red_cap = 0;
+  int64_t d_red_cap = 0;
   double* d_rows = nullptr;  // flow rows of one window, all ensembles
   int64_t d_rows_cap = 0;
-  int* d_healthy = nullptr;
   double* d_part = nullptr;  // per-block partial sums of dsm_stress
   hipEvent_t evs[4] = {nullptr, nullptr, nullptr, nullptr};
   std::vector<int> host_work;
@@ -673,11 +672,6 @@ int corr_alloc(dsm_engine* e, Ens& E, int s) {
     if (e->d_corr_cnt) HIPCHK(hipFree(e->d_corr_cnt));
     if ((rc = dev_alloc(&e->d_corr_cnt, (size_t)3 * s))) return rc;
     e->d_corr_cnt_cap = 3 * s;
-  }
-  if (s * E.p > e->d_red_cap) {
-    if (e->d_red) HIPCHK(hipFree(e->d_red));
-    if ((rc = dev_alloc(&e->d_red, (size_t)s * E.p))) return rc;
-    e->d_red_cap = s * E.p;
   }
   HIPCHK(hipStreamSynchronize(e->st));
   return DSM_OK;
@@ -1383,7 +1377,7 @@ int dsm_create(int32_t device_id, dsm_engine** out) {
   for (auto& ev : e->ev_bin) HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
   int rc;
   if ((rc = dev_alloc(&e->d_cnt, 2 * kNumLists + 32)) || (rc = dev_alloc(&e->d_counters, kNumCounters)) ||
-      (rc = dev_alloc(&e->d_healthy, 1)) || (rc = dev_alloc(&e->d_part, (size_t)kStressBlocks * 9))) {
+      (rc = dev_alloc(&e->d_part, (size_t)kStressBlocks * 9))) {
     dsm_destroy(e);
     return rc;
   }
@@ -1413,7 +1407,7 @@ int dsm_destroy(dsm_engine* e) {
   ChainArrays& c = e->ch;
   void* ptrs[] = {c.Z, c.nk, c.ens, c.cap, c.stall, c.cid, c.local, c.base, c.t, c.ev, c.dt_prev, c.next_sample, c.ev_stop, c.zsum, c.R1,
                   c.Qx, c.Qy, c.Qz, c.N, c.w, e->d_ens, e->d_tabs, e->d_stage, e->d_work, e->d_cnt, e->d_counters,
-                  e->d_corr_cnt, e->d_red, e->d_rows, e->d_healthy, e->d_part, e->d_rec, e->d_lane_tab};
+                  e->d_corr_cnt, e->d_red, e->d_rows, e->d_part, e->d_rec, e->d_lane_tab};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (auto& ev : e->evs)
@@ -1910,12 +1904,22 @@ int dsm_correlator_range(dsm_engine* e, int32_t ens, int32_t first, int32_t coun
   int rc = set_device(e);
   if (rc) return rc;
   const int s = E->s, p = E->p, m = E->m;
-  HIPCHK(launch_corr_reduce(E->dC, E->n, e->ch.stall, E->chain0, first, count, s * p, e->d_red, e->d_healthy, e->st));
-  std::vector<double> sums(s * p);
-  int healthy = 0;
-  HIPCHK(hipMemcpyAsync(sums.data(), e->d_red, sizeof(double) * s * p, hipMemcpyDeviceToHost, e->st));
-  HIPCHK(hipMemcpyAsync(&healthy, e->d_healthy, sizeof(int), hipMemcpyDeviceToHost, e->st));
-  HIPCHK(hipStreamSynchronize(e->st));
+  std::vector<double> sums((size_t)s * p + 1, 0.0);
+  if (g && max_pts > 0) {
+    const int64_t npt = (int64_t)s * p + 1, need = npt * (1 + corr_reduce_parts(count));
+    if (need > e->d_red_cap) {
+      if (e->d_red) HIPCHK(hipFree(e->d_red));
+      e->d_red = nullptr;
+      e->d_red_cap = 0;
+      if ((rc = dev_alloc(&e->d_red, (size_t)need))) return rc;
+      e->d_red_cap = need;
+    }
+    HIPCHK(launch_corr_reduce(E->dC, E->n, e->ch.stall, E->chain0, first, count, p, m, s, E->nins.data(),
+                              e->d_red + npt, e->d_red, e->st));
+    HIPCHK(hipMemcpyAsync(sums.data(), e->d_red, sizeof(double) * npt, hipMemcpyDeviceToHost, e->st));
+    HIPCHK(hipStreamSynchronize(e->st));
+  }
+  const int healthy = (int)sums[(size_t)s * p];
   int im = 0;
   double mk = 1.0;
   for (int k = 0; k < s; ++k) {

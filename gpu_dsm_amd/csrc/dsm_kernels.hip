@@ -331,82 +331,8 @@ __device__ __forceinline__ void corr_insert_from(const CorrArgs& a, int c, int l
   }
 }
 
-// As corr_insert_from for p = P, with the lag loop in groups of four lags whose shift
-// register values and lag sums are loaded together: the loads of a group are in flight
-// at once instead of one lag after another (the lag sums and the shift register are
-// distinct arrays, which the compiler cannot assume).  Same operations in the same order.
-template <int P>
-__device__ __forceinline__ void corr_insert_from_p(const CorrArgs& a, int c, int lvl, double vx, double vy, double vz,
-                                                   int* ins, int* macc, int* nins) {
-  const int64_t nch = a.nch;
-  const int m = a.m;
-  for (;;) {
-    if (lvl == a.s) break;
-    const int in = ins[lvl];
-    const int nin = nins[lvl];
-    double* __restrict__ D = a.D + (int64_t)(lvl * P) * 3 * nch + c;
-    double* __restrict__ A = a.A + (int64_t)(lvl * 3) * nch + c;
-    double* __restrict__ Cc = a.C + (int64_t)(lvl * P) * nch + c;
-    const int jmin = (lvl == 0) ? 0 : P / m;
-    // lag j pairs v with the value inserted j steps before it (j = 0: v itself)
-#pragma unroll
-    for (int j0 = 0; j0 < P; j0 += 4) {
-      if (j0 + 3 < jmin || j0 > nin) continue;
-      double dx[4], dy[4], dz[4], cv[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int j = j0 + k;
-        int idx = in - j;
-        if (idx < 0) idx += P;
-        const bool use = j >= jmin && j <= nin;
-        dx[k] = vx; dy[k] = vy; dz[k] = vz; cv[k] = 0.0;
-        if (use && j > 0) {
-          dx[k] = D[(int64_t)(idx * 3 + 0) * nch];
-          dy[k] = D[(int64_t)(idx * 3 + 1) * nch];
-          dz[k] = D[(int64_t)(idx * 3 + 2) * nch];
-        }
-        if (use) cv[k] = Cc[(int64_t)j * nch];
-      }
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int j = j0 + k;
-        if (!(j >= jmin && j <= nin)) continue;
-        if (a.type == 0) {
-          cv[k] += vx * dx[k] + vy * dy[k] + vz * dz[k];
-        } else {
-          const double ex = vx - dx[k], ey = vy - dy[k], ez = vz - dz[k];
-          cv[k] += ex * ex + ey * ey + ez * ez;
-        }
-        Cc[(int64_t)j * nch] = cv[k];
-      }
-    }
-    D[(int64_t)(in * 3 + 0) * nch] = vx;
-    D[(int64_t)(in * 3 + 1) * nch] = vy;
-    D[(int64_t)(in * 3 + 2) * nch] = vz;
-    // MSD carries the first value of each block up unaveraged
-    // (common/eq_ensemble_kernel.cu:181-189)
-    double ax = A[0], ay = A[nch], az = A[2 * nch];
-    if (a.type == 0 || macc[lvl] == 0) { ax += vx; ay += vy; az += vz; }
-    macc[lvl]++;
-    const bool push = macc[lvl] == m;
-    double ux = 0.0, uy = 0.0, uz = 0.0;
-    if (push) {
-      if (a.type == 0) { ux = ax / m; uy = ay / m; uz = az / m; }
-      else { ux = ax; uy = ay; uz = az; }
-      ax = 0.0; ay = 0.0; az = 0.0;
-      macc[lvl] = 0;
-    }
-    A[0] = ax; A[nch] = ay; A[2 * nch] = az;
-    ins[lvl] = (in + 1 == P) ? 0 : in + 1;
-    nins[lvl] = nin < P ? nin + 1 : P;
-    if (!push) break;
-    ++lvl;
-    vx = ux; vy = uy; vz = uz;
-  }
-}
-
-// Any p: every level in device memory.
-__global__ void __launch_bounds__(256) corr_update_kernel(CorrArgs a) {
+// p too large for the kernel below: thread per chain, every level in device memory.
+__global__ void __launch_bounds__(256) corr_update_serial_kernel(CorrArgs a) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= a.nch) return;
   int ins[40], macc[40], nins[40];
@@ -418,105 +344,156 @@ __global__ void __launch_bounds__(256) corr_update_kernel(CorrArgs a) {
   }
 }
 
-// p = P (16 in every reference input): level 0, which takes every sample row, is held
-// in registers for the whole window -- its P slots in age order (h[0] the newest), its P
-// lag sums and its block accumulator -- and written back once; the levels above take
-// the block pushes in device memory as before.  Every sum is formed in the same order
-// as in corr_update_kernel, so both give identical results.
-template <int P>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) corr_update_reg_kernel(CorrArgs a) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= a.nch) return;
-  int ins[40], macc[40], nins[40];
-  for (int k = 1; k < a.s; ++k) { ins[k] = a.cnt[k]; macc[k] = a.cnt[a.s + k]; nins[k] = a.cnt[2 * a.s + k]; }
-  int in0 = a.cnt[0], macc0 = a.cnt[a.s], nins0 = a.cnt[2 * a.s];
+
+// A window's samples into the correlator, level by level: kCorrChains chains per block
+// (chain fastest in the thread index and in LDS, as in device memory) by up to 16 lag
+// threads.  A level's values of a chunk of rows lie in LDS behind the last p before them,
+// so every lag of every chain sums its products on its own, in row order as a sample by
+// sample update does, and the accumulators and shift register of a level are read and
+// written once per chunk.  The block averages (first values for MSD) handed up are the
+// next level's values.
+// One thread per chain with the lags in turn was bound by its serial chain of device-memory
+// accesses: 64 rows of 20,011 chains with p = 64 took 2,909 us, of 1000 chains with p = 16
+// 231 us.
+template <int CH>
+__global__ void __launch_bounds__(16 * CH) corr_update_kernel(CorrArgs a, int chunk) {
+  extern __shared__ double corr_lds[];
+  const int p = a.p, m = a.m, LT = blockDim.x / CH;
+  double* cur = corr_lds;                            // [p older values, oldest first; chunk new ones][3][CH]
+  double* nxt = cur + (int64_t)(p + chunk) * 3 * CH;  // [chunk / m + 1][3][CH]
+  const int ch = threadIdx.x % CH, lt = threadIdx.x / CH;
+  const int c0 = blockIdx.x * CH, c = c0 + ch;
+  const bool on = c < a.nch;
   const int64_t nch = a.nch;
-  const int m = a.m;
-  double* D = a.D + c;
-  double* A = a.A + c;
-  double* Cc = a.C + c;
-  double hx[P], hy[P], hz[P], cs[P];
-#pragma unroll
-  for (int k = 0; k < P; ++k) {
-    const int slot = (in0 - 1 - k + 2 * P) % P;
-    hx[k] = D[(int64_t)(slot * 3 + 0) * nch];
-    hy[k] = D[(int64_t)(slot * 3 + 1) * nch];
-    hz[k] = D[(int64_t)(slot * 3 + 2) * nch];
-    cs[k] = Cc[(int64_t)k * nch];
-  }
-  double ax = A[0], ay = A[nch], az = A[2 * nch];
-  for (int row = 0; row < a.nrows; ++row) {
-    const float* o = a.stage + ((int64_t)row * nch + c) * 3;
-    const double vx = o[0], vy = o[1], vz = o[2];
-    if (a.type == 0 || macc0 == 0) { ax += vx; ay += vy; az += vz; }
-    ++macc0;
-    const bool push = macc0 == m;
-    double ux = 0.0, uy = 0.0, uz = 0.0;
-    if (push) {
-      if (a.type == 0) { ux = ax / m; uy = ay / m; uz = az / m; }
-      else { ux = ax; uy = ay; uz = az; }
-      ax = 0.0; ay = 0.0; az = 0.0;
-      macc0 = 0;
+  for (int row0 = 0; row0 < a.nrows; row0 += chunk) {
+    int n = min(chunk, a.nrows - row0);
+    const int live = min(CH, a.nch - c0);
+    for (int e = threadIdx.x; e < n * 3 * live; e += blockDim.x) {
+      const int r = e / (3 * live), x = e - r * 3 * live;
+      cur[((p + r) * 3 + x % 3) * CH + x / 3] = (double)a.stage[((int64_t)(row0 + r) * nch + c0) * 3 + x];
     }
-    // lag j pairs the new value with the one inserted j steps before it (h[j-1])
+    int done = row0;  // values this level took in earlier chunks of the window
+    for (int lvl = 0; lvl < a.s && n > 0; ++lvl) {
+      const int ins = (int)((a.cnt[lvl] + (int64_t)done) % p);
+      const int macc = (int)((a.cnt[a.s + lvl] + (int64_t)done) % m);
+      const int nins = min(p, a.cnt[2 * a.s + lvl] + done);
+      double* D = a.D + (int64_t)(lvl * p) * 3 * nch + c;
+      for (int i = lt; i < p; i += LT) {
+        const int age = p - i;
+        if (on && age <= nins) {
+          const int slot = ins >= age ? ins - age : ins - age + p;
 #pragma unroll
-    for (int j = 0; j < P; ++j) {
-      const double dx = j == 0 ? vx : hx[j - 1 < 0 ? 0 : j - 1];
-      const double dy = j == 0 ? vy : hy[j - 1 < 0 ? 0 : j - 1];
-      const double dz = j == 0 ? vz : hz[j - 1 < 0 ? 0 : j - 1];
-      double add;
-      if (a.type == 0) {
-        add = vx * dx + vy * dy + vz * dz;
-      } else {
-        const double ex = vx - dx, ey = vy - dy, ez = vz - dz;
-        add = ex * ex + ey * ey + ez * ez;
+          for (int q = 0; q < 3; ++q) cur[(i * 3 + q) * CH + ch] = D[(int64_t)(slot * 3 + q) * nch];
+        }
       }
-      if (j <= nins0) cs[j] += add;
-    }
+      __syncthreads();
+      // lag sums: four lags of a thread share the reads of the new value
+      const int jmin = lvl == 0 ? 0 : p / m;
+      for (int j0 = lt; j0 < p; j0 += 4 * LT) {
+        double cs[4];
 #pragma unroll
-    for (int k = P - 1; k > 0; --k) { hx[k] = hx[k - 1]; hy[k] = hy[k - 1]; hz[k] = hz[k - 1]; }
-    hx[0] = vx; hy[0] = vy; hz[0] = vz;
-    in0 = (in0 + 1 == P) ? 0 : in0 + 1;
-    nins0 = nins0 < P ? nins0 + 1 : P;
-    if (push) corr_insert_from_p<P>(a, c, 1, ux, uy, uz, ins, macc, nins);
-  }
-  // write back: the slots of this window's values (the newest min(nrows, P)), the lag
-  // sums and the block accumulator
+        for (int k = 0; k < 4; ++k) {
+          const int j = j0 + k * LT;
+          cs[k] = on && j >= jmin && j < p ? a.C[(int64_t)(lvl * p + j) * nch + c] : 0.0;
+        }
+        if (on) {
+          for (int r = 0; r < n; ++r) {
+            const double vx = cur[((p + r) * 3 + 0) * CH + ch], vy = cur[((p + r) * 3 + 1) * CH + ch],
+                         vz = cur[((p + r) * 3 + 2) * CH + ch];
 #pragma unroll
-  for (int k = 0; k < P; ++k) {
-    if (k < a.nrows) {
-      const int slot = (in0 - 1 - k + 2 * P) % P;
-      D[(int64_t)(slot * 3 + 0) * nch] = hx[k];
-      D[(int64_t)(slot * 3 + 1) * nch] = hy[k];
-      D[(int64_t)(slot * 3 + 2) * nch] = hz[k];
+            for (int k = 0; k < 4; ++k) {
+              const int j = j0 + k * LT;
+              if (j < p && nins + r >= j) {
+                const double* d = cur + (p + r - j) * 3 * CH + ch;
+                const double dx = d[0], dy = d[CH], dz = d[2 * CH];
+                if (a.type == 0) {
+                  cs[k] += vx * dx + vy * dy + vz * dz;
+                } else {
+                  const double ex = vx - dx, ey = vy - dy, ez = vz - dz;
+                  cs[k] += ex * ex + ey * ey + ez * ez;
+                }
+              }
+            }
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int j = j0 + k * LT;
+          if (on && j >= jmin && j < p) a.C[(int64_t)(lvl * p + j) * nch + c] = cs[k];
+        }
+      }
+      // block accumulators, one component a thread; MSD carries the first value of each
+      // block up unaveraged (common/eq_ensemble_kernel.cu:181-189)
+      if (on) {
+        for (int q = lt; q < 3; q += LT) {
+          double acc = a.A[(int64_t)(lvl * 3 + q) * nch + c];
+          int mc = macc, k = 0;
+          for (int r = 0; r < n; ++r) {
+            const double v = cur[((p + r) * 3 + q) * CH + ch];
+            if (a.type == 0 || mc == 0) acc += v;
+            if (++mc == m) {
+              nxt[(k * 3 + q) * CH + ch] = a.type == 0 ? acc / m : acc;
+              acc = 0.0;
+              mc = 0;
+              ++k;
+            }
+          }
+          a.A[(int64_t)(lvl * 3 + q) * nch + c] = acc;
+        }
+        for (int r = max(0, n - p) + lt; r < n; r += LT) {
+          const int slot = (ins + r) % p;
+#pragma unroll
+          for (int q = 0; q < 3; ++q) D[(int64_t)(slot * 3 + q) * nch] = cur[((p + r) * 3 + q) * CH + ch];
+        }
+      }
+      __syncthreads();
+      const int up = (macc + n) / m;
+      for (int e = threadIdx.x; e < up * 3 * CH; e += blockDim.x) cur[p * 3 * CH + e] = nxt[e];
+      done = (int)((a.cnt[a.s + lvl] + (int64_t)done) / m);
+      n = up;
+      __syncthreads();
     }
-    Cc[(int64_t)k * nch] = cs[k];
   }
-  A[0] = ax; A[nch] = ay; A[2 * nch] = az;
 }
 
-// G(level, lag) = sum over healthy chains of C / (3 * n_pairs * n_healthy); the chains
-// are first .. first+count-1 of an ensemble of ld chains (C is [point][ld])
+// G(level, lag) = sum over healthy chains of C / (3 * n_pairs * n_healthy); the chains are
+// first .. first+count-1 of an ensemble of ld chains (C is [point][ld]).  Block (point,
+// part) sums one of gridDim.y parts of the chains; points without a pair yet, and the lags
+// below p/m of the upper levels, are left out.  The parts are added in order by
+// corr_parts_kernel, so the result does not depend on timing.  Row npts counts the chains.
+// (One block a point: 345 us for 192 points of 131,072 chains; 40 us in 32 parts.)
+struct CorrPoints {
+  int p, m, s;
+  int nins[40];  // values each level has taken, clamped to p
+};
 __global__ void __launch_bounds__(256) corr_reduce_kernel(const double* C, int ld, const int* stall, int chain0,
-                                                            int first, int count, int npts, double* out_sum,
-                                                            int* out_healthy) {
-  const int pt = blockIdx.x;
-  if (pt >= npts) return;
-  __shared__ double red[256];
-  __shared__ int cnt[256];
-  double acc = 0.0;
-  int h = 0;
-  for (int c = first + threadIdx.x; c < first + count; c += blockDim.x) {
-    if (stall[chain0 + c] == 0) { acc += C[(int64_t)pt * ld + c]; ++h; }
+                                                            int first, int count, CorrPoints P, double* part) {
+  const int pt = blockIdx.x, npts = P.s * P.p;
+  const int lvl = pt / P.p, lag = pt - lvl * P.p;
+  if (pt < npts && (lag >= P.nins[lvl] || (lvl > 0 && lag < P.p / P.m))) {
+    if (threadIdx.x == 0) part[(int64_t)pt * gridDim.y + blockIdx.y] = 0.0;
+    return;
   }
+  const int per = (count + gridDim.y - 1) / gridDim.y;
+  const int lo = first + blockIdx.y * per, hi = min(first + count, lo + per);
+  double acc = 0.0;
+  for (int c = lo + threadIdx.x; c < hi; c += blockDim.x)
+    if (stall[chain0 + c] == 0) acc += pt < npts ? C[(int64_t)pt * ld + c] : 1.0;
+  __shared__ double red[256];
   red[threadIdx.x] = acc;
-  cnt[threadIdx.x] = h;
   __syncthreads();
   for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) { red[threadIdx.x] += red[threadIdx.x + s]; cnt[threadIdx.x] += cnt[threadIdx.x + s]; }
+    if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
     __syncthreads();
   }
-  if (threadIdx.x == 0) { out_sum[pt] = red[0]; if (pt == 0) *out_healthy = cnt[0]; }
+  if (threadIdx.x == 0) part[(int64_t)pt * gridDim.y + blockIdx.y] = red[0];
+}
+__global__ void __launch_bounds__(256) corr_parts_kernel(const double* part, int parts, int npts, double* out) {
+  const int pt = blockIdx.x * blockDim.x + threadIdx.x;
+  if (pt >= npts) return;
+  double acc = 0.0;
+  for (int k = 0; k < parts; ++k) acc += part[(int64_t)pt * parts + k];
+  out[pt] = acc;
 }
 
 // ------------------------------------------------------------------ captured passes
@@ -907,18 +884,38 @@ hipError_t launch_corr_update(const float* stage, double* D, double* A, double* 
                               int nch, int p, int m, int s, int nrows, const int* cnt, int type, hipStream_t st) {
   if (nrows <= 0 || nch <= 0) return hipSuccess;
   CorrArgs a{stage, D, A, C, stall, chain0, nch, p, m, s, nrows, cnt, type};
-  if (p == 16)
-    hipLaunchKernelGGL(corr_update_reg_kernel<16>, dim3((nch + 255) / 256), dim3(256), 0, st, a);
-  else
-    hipLaunchKernelGGL(corr_update_kernel, dim3((nch + 255) / 256), dim3(256), 0, st, a);
+  // 16 chains a block: 128-byte rows of the [...][chain] arrays.  An ensemble of few chains
+  // takes four, so that its blocks are not all on a few CUs.
+  const int chunk = nrows < 64 ? nrows : 64, lt = p < 16 ? (p < 4 ? 4 : p) : 16;
+  const size_t per_chain = sizeof(double) * 3 * (size_t)(p + chunk + chunk / m + 1);
+  const int ch = nch <= 4096 || 16 * per_chain > 64 * 1024 ? 4 : 16;
+  const size_t lds = per_chain * ch;
+  if (lds <= 64 * 1024) {
+    const dim3 grid((nch + ch - 1) / ch), block(ch * lt);
+    if (ch == 4) hipLaunchKernelGGL(corr_update_kernel<4>, grid, block, lds, st, a, chunk);
+    else hipLaunchKernelGGL(corr_update_kernel<16>, grid, block, lds, st, a, chunk);
+  } else {
+    hipLaunchKernelGGL(corr_update_serial_kernel, dim3((nch + 255) / 256), dim3(256), 0, st, a);
+  }
   return hipGetLastError();
 }
 
-hipError_t launch_corr_reduce(const double* C, int ld, const int* stall, int chain0, int first, int count, int npts,
-                              double* out_sum, int* out_healthy, hipStream_t st) {
-  if (npts <= 0) return hipSuccess;
-  hipLaunchKernelGGL(corr_reduce_kernel, dim3(npts), dim3(256), 0, st, C, ld, stall, chain0, first, count, npts,
-                     out_sum, out_healthy);
+int corr_reduce_parts(int count) {
+  const int parts = (count + 4095) / 4096;
+  return parts < 1 ? 1 : parts > 64 ? 64 : parts;
+}
+hipError_t launch_corr_reduce(const double* C, int ld, const int* stall, int chain0, int first, int count, int p, int m,
+                              int s, const int64_t* nins, double* part, double* out, hipStream_t st) {
+  CorrPoints P{};
+  P.p = p;
+  P.m = m;
+  P.s = s;
+  for (int k = 0; k < s && k < 40; ++k) P.nins[k] = (int)(nins[k] < p ? nins[k] : p);
+  const int parts = corr_reduce_parts(count), npts = s * p;
+  hipLaunchKernelGGL(corr_reduce_kernel, dim3(npts + 1, parts), dim3(256), 0, st, C, ld, stall, chain0, first, count, P,
+                     parts > 1 ? part : out);
+  if (parts > 1)
+    hipLaunchKernelGGL(corr_parts_kernel, dim3((npts + 256) / 256), dim3(256), 0, st, part, parts, npts + 1, out);
   return hipGetLastError();
 }
 

@@ -76,8 +76,11 @@ hipError_t launch_flow_reduce(const float* stage, int nch, int nrows, double* ou
                               hipStream_t st);
 hipError_t launch_corr_update(const float* stage, double* D, double* A, double* C, const int* stall, int chain0,
                               int nch, int p, int m, int s, int nrows, const int* cnt, int type, hipStream_t st);
-hipError_t launch_corr_reduce(const double* C, int ld, const int* stall, int chain0, int first, int count, int npts,
-                              double* out_sum, int* out_healthy, hipStream_t st);
+// out[0..s*p): sums of C over the healthy chains, out[s*p]: their count; nins: values each
+// level has taken; part: (s*p + 1) * corr_reduce_parts(count) doubles
+int corr_reduce_parts(int count);
+hipError_t launch_corr_reduce(const double* C, int ld, const int* stall, int chain0, int first, int count, int p, int m,
+                              int s, const int64_t* nins, double* part, double* out, hipStream_t st);
 // ensemble stress of the current state: kStressBlocks partial sums of 9 doubles
 // (xx yy zz xy yz zx Lpp Z count over the chains that have not stalled)
 constexpr int kStressBlocks = 256;
