@@ -519,23 +519,25 @@ __global__ void __launch_bounds__(256) stage_window_kernel(const WinParam* __res
 // sum_i |Q_i| and Z, in FP64 from the stored FP32 strands, after the deformation still
 // pending from the chain's last jump (dt_prev; the reference applies it with olddt).
 // Chains that have stalled are left out.  A fixed grid of kStressBlocks blocks strides
-// over the chains; block b writes its partial sums to part[9b .. 9b+8] (xx yy zz xy yz zx
-// Lpp Z count), which the host adds in block order, so the result does not depend on
-// timing.
-__global__ void __launch_bounds__(256) chain_stress_kernel(ChainArrays ch, int chain0, int n, KappaArg K,
-                                                           double* part) {
-  __shared__ double red[9][256];
+// over the chains, one wave a chain, one lane a strand (the arrays are read in whole
+// lines; one thread a chain took 85 us for 20,011 chains of Z ~ 100); block b writes its
+// partial sums to part[9b .. 9b+8] (xx yy zz xy yz zx Lpp Z count), which the host adds in
+// block order, so the result does not depend on timing.
+constexpr int kStressWaves = 16;
+__global__ void __launch_bounds__(64 * kStressWaves) chain_stress_kernel(ChainArrays ch, int chain0, int n, KappaArg K,
+                                                                         double* part) {
+  __shared__ double red[9][kStressWaves];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   double acc[9];
 #pragma unroll
   for (int q = 0; q < 9; ++q) acc[q] = 0.0;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+  for (int i = blockIdx.x * kStressWaves + wave; i < n; i += gridDim.x * kStressWaves) {
     const int c = chain0 + i;
     if (ch.stall[c] != 0) continue;
     const int Z = ch.Z[c];
     const int64_t b = ch.base[c];
     const double dt = (double)ch.dt_prev[c];
-    double s[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int k = 0; k < Z; ++k) {
+    for (int k = lane; k < Z; k += 64) {
       double x = ch.Qx[b + k], y = ch.Qy[b + k], z = ch.Qz[b + k];
       if (dt != 0.0) {
         const double x1 = x + dt * ((double)K.k[0] * x + (double)K.k[1] * y + (double)K.k[2] * z);
@@ -544,28 +546,25 @@ __global__ void __launch_bounds__(256) chain_stress_kernel(ChainArrays ch, int c
         x = x1; y = y1; z = z1;
       }
       const double t3 = 3.0 / (double)ch.N[b + k];
-      s[0] -= t3 * x * x; s[1] -= t3 * y * y; s[2] -= t3 * z * z;
-      s[3] -= t3 * x * y; s[4] -= t3 * y * z; s[5] -= t3 * x * z;
-      s[6] += sqrt(x * x + y * y + z * z);
+      acc[0] -= t3 * x * x; acc[1] -= t3 * y * y; acc[2] -= t3 * z * z;
+      acc[3] -= t3 * x * y; acc[4] -= t3 * y * z; acc[5] -= t3 * x * z;
+      acc[6] += sqrt(x * x + y * y + z * z);
     }
-#pragma unroll
-    for (int q = 0; q < 7; ++q) acc[q] += s[q];
-    acc[7] += (double)Z;
-    acc[8] += 1.0;
+    if (lane == 0) {
+      acc[7] += (double)Z;
+      acc[8] += 1.0;
+    }
   }
 #pragma unroll
-  for (int q = 0; q < 9; ++q) red[q][threadIdx.x] = acc[q];
+  for (int q = 0; q < 9; ++q) {
+    for (int d = 32; d > 0; d >>= 1) acc[q] += __shfl_down(acc[q], d, 64);
+    if (lane == 0) red[q][wave] = acc[q];
+  }
   __syncthreads();
-  for (int h = blockDim.x / 2; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h) {
-#pragma unroll
-      for (int q = 0; q < 9; ++q) red[q][threadIdx.x] += red[q][threadIdx.x + h];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int q = 0; q < 9; ++q) part[blockIdx.x * 9 + q] = red[q][0];
+  if (threadIdx.x < 9) {
+    double s = 0.0;
+    for (int w = 0; w < kStressWaves; ++w) s += red[threadIdx.x][w];
+    part[blockIdx.x * 9 + threadIdx.x] = s;
   }
 }
 
@@ -574,39 +573,43 @@ __global__ void __launch_bounds__(256) chain_stress_kernel(ChainArrays ch, int c
 // (App. A.1 of the chain state): out[0] Z outside 1..Nk, out[1] a strand with N < 1,
 // out[2] sum of N != Nk, out[3] an end strand (index 0 or Z-1, Z > 1) with Q != 0,
 // out[4] a non-finite Q or CD rate, out[5] stalled chains, out[6] chains whose clock is
-// below t_min.  The counters (7 x uint64) must be zero on entry.
+// below t_min.  The counters (7 x uint64) must be zero on entry.  One wave a chain, one lane
+// a strand (one thread a chain took 121 us for 20,011 chains of Z ~ 100).
 __global__ void __launch_bounds__(256) check_state_kernel(ChainArrays ch, int chain0, int n, double t_min,
                                                           unsigned long long* out) {
-  unsigned long long v[7] = {0, 0, 0, 0, 0, 0, 0};
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+  __shared__ unsigned int tot[7];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (threadIdx.x < 7) tot[threadIdx.x] = 0;
+  __syncthreads();
+  unsigned int v[7] = {0, 0, 0, 0, 0, 0, 0};  // the same on every lane of a wave
+  for (int i = blockIdx.x * 4 + wave; i < n; i += gridDim.x * 4) {
     const int c = chain0 + i;
     const int Z = ch.Z[c], nk = ch.nk[c];
     if (ch.stall[c] != 0) v[5]++;
     if (!(ch.t[c] >= t_min)) v[6]++;
     if (Z < 1 || Z > nk || Z > ch.cap[c]) { v[0]++; continue; }
     const int64_t b = ch.base[c];
-    int64_t sum = 0;
-    bool bad_n = false, bad_f = false;
-    for (int k = 0; k < Z; ++k) {
+    long long all = 0;
+    bool bad_n = false, bad_f = false, bad_e = false;
+    for (int k = lane; k < Z; k += 64) {
       const int N = ch.N[b + k];
       bad_n = bad_n || N < 1;
-      sum += N;
+      all += N;
       const float x = ch.Qx[b + k], y = ch.Qy[b + k], z = ch.Qz[b + k];
       bad_f = bad_f || !isfinite(x) || !isfinite(y) || !isfinite(z) || (k < Z - 1 && !isfinite(ch.w[b + k]));
+      if (Z > 1 && (k == 0 || k == Z - 1)) bad_e = bad_e || x != 0.f || y != 0.f || z != 0.f;
     }
-    if (bad_n) v[1]++;
-    if (sum != nk) v[2]++;
-    if (Z > 1) {
-      const int64_t e0 = b, e1 = b + Z - 1;
-      if (ch.Qx[e0] != 0.f || ch.Qy[e0] != 0.f || ch.Qz[e0] != 0.f || ch.Qx[e1] != 0.f || ch.Qy[e1] != 0.f ||
-          ch.Qz[e1] != 0.f)
-        v[3]++;
-    }
-    if (bad_f) v[4]++;
+    for (int d = 32; d > 0; d >>= 1) all += __shfl_xor(all, d, 64);
+    if (__ballot(bad_n)) v[1]++;
+    if (all != nk) v[2]++;
+    if (__ballot(bad_e)) v[3]++;
+    if (__ballot(bad_f)) v[4]++;
   }
 #pragma unroll
   for (int q = 0; q < 7; ++q)
-    if (v[q]) atomicAdd(out + q, v[q]);
+    if (lane == 0 && v[q]) atomicAdd(tot + q, v[q]);
+  __syncthreads();
+  if (threadIdx.x < 7 && tot[threadIdx.x]) atomicAdd(out + threadIdx.x, (unsigned long long)tot[threadIdx.x]);
 }
 
 // ------------------------------------------------------------------ copy probe (bandwidth)
@@ -929,14 +932,14 @@ hipError_t launch_chain_stress(const ChainArrays& ch, int chain0, int n, const f
                                hipStream_t st) {
   KappaArg K;
   for (int i = 0; i < 9; ++i) K.k[i] = kappa[i];
-  hipLaunchKernelGGL(chain_stress_kernel, dim3(kStressBlocks), dim3(256), 0, st, ch, chain0, n, K, part);
+  hipLaunchKernelGGL(chain_stress_kernel, dim3(kStressBlocks), dim3(64 * kStressWaves), 0, st, ch, chain0, n, K, part);
   return hipGetLastError();
 }
 
 hipError_t launch_check_state(const ChainArrays& ch, int chain0, int n, double t_min, unsigned long long* out,
                               hipStream_t st) {
   if (n <= 0) return hipSuccess;
-  const int grid = std::min(1024, (n + 255) / 256);
+  const int grid = std::min(2048, (n + 3) / 4);
   hipLaunchKernelGGL(check_state_kernel, dim3(grid), dim3(256), 0, st, ch, chain0, n, t_min, out);
   return hipGetLastError();
 }
