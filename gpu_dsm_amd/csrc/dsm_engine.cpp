@@ -390,6 +390,8 @@ struct dsm_engine {
   int64_t d_red_cap = 0;
   double* d_rows = nullptr;  // flow rows of one window, all ensembles
   int64_t d_rows_cap = 0;
+  double* d_row_part = nullptr;  // partial sums of one ensemble's rows
+  int64_t d_row_part_cap = 0;
   double* d_part = nullptr;  // per-block partial sums of dsm_stress
   hipEvent_t evs[4] = {nullptr, nullptr, nullptr, nullptr};
   std::vector<int> host_work;
@@ -1069,7 +1071,7 @@ int window_launches(dsm_engine* e, const std::vector<int>& act, const std::vecto
       HIPCHK(launch_corr_update(e->d_stage + E.P.stage_off, E.dD, E.dA, E.dC, e->ch.stall, E.chain0, E.n, E.p, E.m,
                                 E.s, rows, e->d_corr_cnt + cnt_off[q], E.P.sample_mode == kSampleMsd ? 1 : 0, e->st));
     else
-      HIPCHK(launch_flow_reduce(e->d_stage + E.P.stage_off, E.n, rows, e->d_rows + row_off[q], e->st));
+      HIPCHK(launch_flow_reduce(e->d_stage + E.P.stage_off, E.n, rows, e->d_row_part, e->d_rows + row_off[q], e->st));
   }
   return DSM_OK;
 }
@@ -1218,7 +1220,7 @@ int advance_impl(dsm_engine* e, const std::vector<int>& ids, const std::vector<d
     // the window's sample consumers: level counters set before the pass
     std::vector<int> cnt;
     std::vector<int64_t> cnt_off(act.size(), -1), row_off(act.size(), -1);
-    int64_t flow_doubles = 0;
+    int64_t flow_doubles = 0, row_parts = 0;
     for (size_t q = 0; q < act.size(); ++q) {
       const Ens& E = e->ens[act[q]];
       if (E.P.k_end <= E.P.k0) continue;
@@ -1230,6 +1232,7 @@ int advance_impl(dsm_engine* e, const std::vector<int>& ids, const std::vector<d
       } else {
         row_off[q] = flow_doubles;
         flow_doubles += (E.P.k_end - E.P.k0) * 9;
+        row_parts = std::max(row_parts, (E.P.k_end - E.P.k0) * 9 * flow_reduce_parts(E.n));
       }
     }
     if ((int)cnt.size() > e->d_corr_cnt_cap) {
@@ -1243,6 +1246,14 @@ int advance_impl(dsm_engine* e, const std::vector<int>& ids, const std::vector<d
       if (e->d_rows) HIPCHK(hipFree(e->d_rows));
       if ((rc = dev_alloc(&e->d_rows, (size_t)flow_doubles))) return rc;
       e->d_rows_cap = flow_doubles;
+    }
+    if (row_parts > e->d_row_part_cap) {
+      e->gen++;
+      if (e->d_row_part) HIPCHK(hipFree(e->d_row_part));
+      e->d_row_part = nullptr;
+      e->d_row_part_cap = 0;
+      if ((rc = dev_alloc(&e->d_row_part, (size_t)row_parts))) return rc;
+      e->d_row_part_cap = row_parts;
     }
     Pass timed;
     bool graph_timed = false;
@@ -1407,7 +1418,7 @@ int dsm_destroy(dsm_engine* e) {
   ChainArrays& c = e->ch;
   void* ptrs[] = {c.Z, c.nk, c.ens, c.cap, c.stall, c.cid, c.local, c.base, c.t, c.ev, c.dt_prev, c.next_sample, c.ev_stop, c.zsum, c.R1,
                   c.Qx, c.Qy, c.Qz, c.N, c.w, e->d_ens, e->d_tabs, e->d_stage, e->d_work, e->d_cnt, e->d_counters,
-                  e->d_corr_cnt, e->d_red, e->d_rows, e->d_part, e->d_rec, e->d_lane_tab};
+                  e->d_corr_cnt, e->d_red, e->d_rows, e->d_row_part, e->d_part, e->d_rec, e->d_lane_tab};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (auto& ev : e->evs)
@@ -1540,7 +1551,7 @@ int dsm_add_ensemble(dsm_engine* e, const dsm_ensemble_desc* d, int32_t* ens_id)
   E.p = d->corr_p > 0 ? d->corr_p : 64;
   E.m = d->corr_m > 0 ? d->corr_m : 8;
   if (E.p % E.m != 0 && eq_sampling(d->sample_mode)) return fail(DSM_ERR_ARG, "corr_p must be a multiple of corr_m");
-  E.stage_floats = (int64_t)E.window * E.n * E.ncomp;
+  E.stage_floats = ((int64_t)E.window * E.n * E.ncomp + 3) & ~(int64_t)3;  // rows start on 16 bytes
   P.stage_off = e->stage_space.take(E.stage_floats);
   e->stage_used = std::max(e->stage_used, e->stage_space.end);
   if ((rc = ensure_stage(e))) {
@@ -1617,9 +1628,7 @@ int dsm_init_equilibrium(dsm_engine* e, int32_t ens) {
   if (!E) return fail(DSM_ERR_ARG, "no ensemble %d", ens);
   int rc = set_device(e);
   if (rc) return rc;
-  HIPCHK(launch_iota(e->d_work, E->chain0, E->n, e->st));
-  HIPCHK(launch_init_eq(e->ch, e->d_ens, e->d_tabs, e->d_work, E->n, e->st));
-  HIPCHK(hipMemsetAsync(e->ch.R1 + 3 * (int64_t)E->chain0, 0, 12 * (size_t)E->n, e->st));  // common/chain.cu:207
+  HIPCHK(launch_init_eq(e->ch, e->d_ens, e->d_tabs, E->chain0, E->n, e->st));
   HIPCHK(hipStreamSynchronize(e->st));
   E->k_cur = E->P.sample_mode == kSampleFlow ? 1 : 0;
   E->flow_rows.clear();

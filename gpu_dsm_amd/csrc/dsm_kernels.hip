@@ -25,62 +25,104 @@
 namespace dsm {
 
 // ------------------------------------------------------------------ equilibrium init
-// Thread per chain.  Inner Kuhn-step boundary i (1 <= i < nk) carries an
-// entanglement iff Philox word (i-1) < 2^32/(1+beta): Z-1 ~ Binomial(nk-1, 1/(1+beta))
-// and N|Z uniform over compositions (the laws of common/chain.cu:38-88).
-// Internal strands get Q ~ N(0, N/3) per component (common/chain.cu:90-102),
-// links get CD rates from f_t (common/chain.cu:155-158), with the partner length of
-// each link drawn from the background distribution when there is one (:141-149).
+// A 16-lane row per chain of first .. first+n-1.  Inner Kuhn-step boundary i (1 <= i < nk)
+// carries an entanglement iff Philox word (i-1) < 2^32/(1+beta): Z-1 ~ Binomial(nk-1,
+// 1/(1+beta)) and N|Z uniform over compositions (the laws of common/chain.cu:38-88).
+// Internal strands get Q ~ N(0, N/3) per component (common/chain.cu:90-102), links get CD
+// rates from f_t (common/chain.cu:155-158), with the partner length of each link drawn from
+// the background distribution when there is one (:141-149).  A lane has the four words of
+// one Philox call in each part; a cut's strand index is the count of cuts before it, and
+// the cut positions are kept in the strand-length array until the lengths are their
+// differences.  (One thread a chain, all of it in turn: 66 us for 16,384 chains of Nk 50,
+// 3,379 us for the 262,144-chain melt.)
 __global__ void __launch_bounds__(256) init_eq_kernel(ChainArrays ch, const EnsParams* ens, const float* tabs,
-                                                        const int* chains, int n) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= n) return;
-  const int c = chains[idx];
+                                                        int first, int n) {
+  const int rl = threadIdx.x & 15;
+  const int idx = blockIdx.x * 16 + (threadIdx.x >> 4);
+  const bool on = idx < n;  // rows past the end run along, without a store
+  const int c = first + (on ? idx : 0);
   const EnsParams& P = ens[ch.ens[c]];
   const uint32_t k0 = P.key0, k1 = P.key1;
   const int nk = ch.nk[c];
   const uint32_t cid = ch.cid[c];
   const int64_t b = ch.base[c];
-  int Z = 0, len = 0;
-  uint4 x = make_uint4(0, 0, 0, 0);
-  for (int i = 1; i <= nk; ++i) {
-    ++len;
-    if (i == nk) { ch.N[b + Z] = len; ++Z; break; }
-    const int wi = i - 1;
-    if ((wi & 3) == 0) x = philox4x32_10(make_uint4((uint32_t)(wi >> 2), 0u, cid, kPurposeInitCut), k0, k1);
-    const uint32_t word = (wi & 3) == 0 ? x.x : (wi & 3) == 1 ? x.y : (wi & 3) == 2 ? x.z : x.w;
-    if (word < P.cut_threshold) { ch.N[b + Z] = len; ++Z; len = 0; }
-  }
-  for (int k = 0; k < Z; ++k) {
-    float qx = 0.0f, qy = 0.0f, qz = 0.0f;
-    if (k > 0 && k < Z - 1) {
-      const uint4 g = philox4x32_10(make_uint4((uint32_t)k, 0u, cid, kPurposeInitQ), k0, k1);
-      float g0, g1, g2, g3;
-      boxmuller(g.x, g.y, g0, g1);
-      boxmuller(g.z, g.w, g2, g3);
-      const float sig = sqrtf((float)ch.N[b + k] / 3.0f);
-      qx = g0 * sig; qy = g1 * sig; qz = g2 * sig;
+  int Z = 0;
+  for (int w0 = 0; __ballot(w0 < nk); w0 += 64) {
+    const int wi = w0 + 4 * rl;  // words wi..wi+3: boundaries wi+1..wi+4; boundary nk always ends a strand
+    uint4 x = make_uint4(0, 0, 0, 0);
+    if (wi < nk - 1) x = philox4x32_10(make_uint4((uint32_t)(wi >> 2), 0u, cid, kPurposeInitCut), k0, k1);
+    const uint32_t word[4] = {x.x, x.y, x.z, x.w};
+    int cut[4], cnt = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int i = wi + k + 1;
+      cut[k] = i == nk || (i < nk && word[k] < P.cut_threshold) ? 1 : 0;
+      cnt += cut[k];
     }
-    ch.Qx[b + k] = qx; ch.Qy[b + k] = qy; ch.Qz[b + k] = qz;
-    ch.w[b + k] = 0.0f;
-  }
-  if (P.cd) {
-    const float* pd = tabs + P.pd_off;
-    uint4 y = make_uint4(0, 0, 0, 0);
-    for (int k = 0; k < Z - 1; ++k) {
-      if ((k & 3) == 0) x = philox4x32_10(make_uint4((uint32_t)(k >> 2), 0u, cid, kPurposeInitTau), k0, k1);
-      const uint32_t word = (k & 3) == 0 ? x.x : (k & 3) == 1 ? x.y : (k & 3) == 2 ? x.z : x.w;
-      if (P.partner) {
-        if ((k & 3) == 0) y = philox4x32_10(make_uint4((uint32_t)(k >> 2), 0u, cid, kPurposeInitPartner), k0, k1);
-        const uint32_t pw = (k & 3) == 0 ? y.x : (k & 3) == 1 ? y.y : (k & 3) == 2 ? y.z : y.w;
-        ch.w[b + k] = rate_ft_partner(pd, (int)(pw >> (32 - kPartnerBits)), u01(word));
-      } else {
-        ch.w[b + k] = rate_ft(&P, u01(word));
+    int before = cnt;  // inclusive count over the row
+    before += dppi<kRowShr1>(before, 0);
+    before += dppi<kRowShr2>(before, 0);
+    before += dppi<kRowShr4>(before, 0);
+    before += dppi<kRowShr8>(before, 0);
+    const int total = row_last(before);
+    int at = Z + before - cnt;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (cut[k]) {
+        if (on) ch.N[b + at] = wi + k + 1;
+        ++at;
       }
+    Z += total;
+  }
+  // The lanes' cut positions are complete (same wave, in issue order); lengths from the
+  // last block of 16 strands down, each read before the strand below is rewritten
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  const int zmax = Z;
+  for (int s0 = (zmax - 1) & ~15; __ballot(s0 >= 0); s0 -= 16) {
+    const int k = s0 + rl;
+    const bool in = s0 >= 0 && k < Z;
+    int N = 0;
+    if (in) N = ch.N[b + k] - (k > 0 ? ch.N[b + k - 1] : 0);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (in && on) {
+      float qx = 0.0f, qy = 0.0f, qz = 0.0f;
+      if (k > 0 && k < Z - 1) {
+        const uint4 g = philox4x32_10(make_uint4((uint32_t)k, 0u, cid, kPurposeInitQ), k0, k1);
+        float g0, g1, g2, g3;
+        boxmuller(g.x, g.y, g0, g1);
+        boxmuller(g.z, g.w, g2, g3);
+        const float sig = sqrtf((float)N / 3.0f);
+        qx = g0 * sig; qy = g1 * sig; qz = g2 * sig;
+      }
+      ch.Qx[b + k] = qx; ch.Qy[b + k] = qy; ch.Qz[b + k] = qz;
+      ch.N[b + k] = N;
     }
   }
-  ch.Z[c] = Z; ch.stall[c] = 0; ch.t[c] = 0.0; ch.ev[c] = 0; ch.dt_prev[c] = 0.0f; ch.zsum[c] = 0;
-  ch.next_sample[c] = (P.sample_mode == kSampleFlow) ? 1 : 0;
+  const float* pd = tabs + P.pd_off;
+  for (int s0 = 0; __ballot(s0 < Z); s0 += 64) {
+    const int k = s0 + 4 * rl;
+    if (k >= Z || !on) continue;
+    uint4 x = make_uint4(0, 0, 0, 0), y = x;
+    if (P.cd && k < Z - 1) {
+      x = philox4x32_10(make_uint4((uint32_t)(k >> 2), 0u, cid, kPurposeInitTau), k0, k1);
+      if (P.partner) y = philox4x32_10(make_uint4((uint32_t)(k >> 2), 0u, cid, kPurposeInitPartner), k0, k1);
+    }
+    const uint32_t word[4] = {x.x, x.y, x.z, x.w}, pw[4] = {y.x, y.y, y.z, y.w};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (k + q >= Z) continue;
+      float w = 0.0f;
+      if (P.cd && k + q < Z - 1)
+        w = P.partner ? rate_ft_partner(pd, (int)(pw[q] >> (32 - kPartnerBits)), u01(word[q])) : rate_ft(&P, u01(word[q]));
+      ch.w[b + k + q] = w;
+    }
+  }
+  if (on && rl == 0) {
+    ch.Z[c] = Z; ch.stall[c] = 0; ch.t[c] = 0.0; ch.ev[c] = 0; ch.dt_prev[c] = 0.0f; ch.zsum[c] = 0;
+    ch.next_sample[c] = (P.sample_mode == kSampleFlow) ? 1 : 0;
+    float* r1 = ch.R1 + 3 * (int64_t)c;  // common/chain.cu:207
+    r1[0] = 0.0f; r1[1] = 0.0f; r1[2] = 0.0f;
+  }
 }
 
 // ------------------------------------------------------------------ utility kernels
@@ -229,15 +271,21 @@ __global__ void iota_kernel(int* p, int start, int n) {
 // NaN, so a chain that stalls mid-window keeps the rows it recorded before, as the
 // reference excludes a stalled chain only from the outputs after its stall
 // (common/ensemble_call_block.cu:471-491, per output step).
-__global__ void __launch_bounds__(256) flow_reduce_kernel(const float* stage, int nchains, int nrows, double* out) {
+// Block (row, part) sums one of gridDim.y parts of the chains into part[row][part][9]; with
+// one part that is the row's result, otherwise flow_parts_kernel adds the parts in order.
+// (One block a row: 87 us for 8 rows of 16,384 chains, four parts in flight a row.)
+__global__ void __launch_bounds__(256) flow_reduce_kernel(const float* stage, int nchains, double* part) {
   const int row = blockIdx.x;
-  if (row >= nrows) return;
-  __shared__ double red[9][256];
+  const int per = (nchains + gridDim.y - 1) / gridDim.y;
+  const int lo = blockIdx.y * per, hi = min(nchains, lo + per);
+  __shared__ double red[9][4];
   double acc[9];
 #pragma unroll
   for (int q = 0; q < 9; ++q) acc[q] = 0.0;
-  for (int c = threadIdx.x; c < nchains; c += blockDim.x) {
-    const float* o = stage + ((int64_t)row * nchains + c) * 8;
+  for (int c = lo + threadIdx.x; c < hi; c += blockDim.x) {
+    const float4* o4 = (const float4*)(stage + ((int64_t)row * nchains + c) * 8);
+    const float4 a = o4[0], b = o4[1];
+    const float o[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
     bool ok = o[7] > 0.0f;
 #pragma unroll
     for (int q = 0; q < 8; ++q) ok = ok && (o[q] == o[q]);
@@ -248,19 +296,22 @@ __global__ void __launch_bounds__(256) flow_reduce_kernel(const float* stage, in
     }
   }
 #pragma unroll
-  for (int q = 0; q < 9; ++q) red[q][threadIdx.x] = acc[q];
+  for (int q = 0; q < 9; ++q) {
+    for (int d = 32; d > 0; d >>= 1) acc[q] += __shfl_down(acc[q], d, 64);
+    if ((threadIdx.x & 63) == 0) red[q][threadIdx.x >> 6] = acc[q];
+  }
   __syncthreads();
-  for (int h = blockDim.x / 2; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h) {
-#pragma unroll
-      for (int q = 0; q < 9; ++q) red[q][threadIdx.x] += red[q][threadIdx.x + h];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int q = 0; q < 9; ++q) out[(int64_t)row * 9 + q] = red[q][0];
-  }
+  if (threadIdx.x < 9)
+    part[((int64_t)row * gridDim.y + blockIdx.y) * 9 + threadIdx.x] =
+        ((red[threadIdx.x][0] + red[threadIdx.x][1]) + red[threadIdx.x][2]) + red[threadIdx.x][3];
+}
+__global__ void __launch_bounds__(256) flow_parts_kernel(const double* part, int parts, int nrows, double* out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nrows * 9) return;
+  const int row = i / 9, q = i - 9 * row;
+  double acc = 0.0;
+  for (int k = 0; k < parts; ++k) acc += part[((int64_t)row * parts + k) * 9 + q];
+  out[i] = acc;
 }
 
 // ------------------------------------------------------------------ multi-tau correlator
@@ -819,10 +870,10 @@ int kmc_max_blocks_per_cu(int geom, bool plain, int lds_floats, bool ext) {
 }
 
 
-hipError_t launch_init_eq(const ChainArrays& ch, const EnsParams* ens, const float* tabs, const int* chains, int n,
+hipError_t launch_init_eq(const ChainArrays& ch, const EnsParams* ens, const float* tabs, int first, int n,
                           hipStream_t st) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(init_eq_kernel, dim3((n + 255) / 256), dim3(256), 0, st, ch, ens, tabs, chains, n);
+  hipLaunchKernelGGL(init_eq_kernel, dim3((n + 15) / 16), dim3(256), 0, st, ch, ens, tabs, first, n);
   return hipGetLastError();
 }
 
@@ -876,10 +927,16 @@ hipError_t launch_iota(int* p, int start, int n, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t launch_flow_reduce(const float* stage, int nch, int nrows, double* out,
-                              hipStream_t st) {
+int flow_reduce_parts(int nch) {
+  const int parts = (nch + 1023) / 1024;
+  return parts < 1 ? 1 : parts > 64 ? 64 : parts;
+}
+hipError_t launch_flow_reduce(const float* stage, int nch, int nrows, double* part, double* out, hipStream_t st) {
   if (nrows <= 0) return hipSuccess;
-  hipLaunchKernelGGL(flow_reduce_kernel, dim3(nrows), dim3(256), 0, st, stage, nch, nrows, out);
+  const int parts = flow_reduce_parts(nch);
+  hipLaunchKernelGGL(flow_reduce_kernel, dim3(nrows, parts), dim3(256), 0, st, stage, nch, parts > 1 ? part : out);
+  if (parts > 1)
+    hipLaunchKernelGGL(flow_parts_kernel, dim3((nrows * 9 + 255) / 256), dim3(256), 0, st, part, parts, nrows, out);
   return hipGetLastError();
 }
 

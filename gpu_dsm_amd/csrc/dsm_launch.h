@@ -55,7 +55,8 @@ constexpr int lane_max_lanes(int quads) {
   return odd > 64 ? 64 : odd;
 }
 hipError_t launch_kmc_lane(const KmcArgs& a, int quads, int grid, hipStream_t st);
-hipError_t launch_init_eq(const ChainArrays& ch, const EnsParams* ens, const float* tabs, const int* chains, int n,
+// chains first .. first+n-1
+hipError_t launch_init_eq(const ChainArrays& ch, const EnsParams* ens, const float* tabs, int first, int n,
                           hipStream_t st);
 hipError_t launch_fill_u32(void* p, uint32_t v, int64_t n, hipStream_t st);
 hipError_t launch_iota(int* p, int start, int n, hipStream_t st);
@@ -72,8 +73,9 @@ hipError_t launch_sum_counters(const uint64_t* ev, const uint64_t* zsum, int cha
                                hipStream_t st);
 hipError_t launch_set_ev_stop(const uint64_t* ev, uint64_t* ev_stop, int chain0, int n, uint64_t add,
                               hipStream_t st);
-hipError_t launch_flow_reduce(const float* stage, int nch, int nrows, double* out,
-                              hipStream_t st);
+// out[row][9]; part: nrows * flow_reduce_parts(nch) * 9 doubles
+int flow_reduce_parts(int nch);
+hipError_t launch_flow_reduce(const float* stage, int nch, int nrows, double* part, double* out, hipStream_t st);
 hipError_t launch_corr_update(const float* stage, double* D, double* A, double* C, const int* stall, int chain0,
                               int nch, int p, int m, int s, int nrows, const int* cnt, int type, hipStream_t st);
 // out[0..s*p): sums of C over the healthy chains, out[s*p]: their count; nins: values each
