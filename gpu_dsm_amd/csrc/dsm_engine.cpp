@@ -335,6 +335,7 @@ struct EngineOptions {
   int graph = 0;                         // DSM_OPT_GRAPH
   int wide_pair = 1;                     // DSM_OPT_WIDE_PAIR
   int lane = 1;                          // DSM_OPT_LANE
+  int solo = 1;                          // DSM_OPT_SOLO
 };
 
 struct dsm_engine {
@@ -607,6 +608,16 @@ int lane_quads(const dsm_engine* e, const std::vector<int>& ids) {
   return quads;
 }
 
+// The solo form (dsm_solo.h) takes the place of the wave forms (bins 2 and up) wherever no
+// chain flows: a jump costs it the same at any length, so it gains most on the long chains
+// (Nk 1000: 2.7 times; Nk 600: 1.8; Nk 300, against the two-chain form: 1.08) and is level
+// with the G = 1 form on short ones.
+bool solo_capable(const dsm_engine* e, const std::vector<int>& ids) {
+  for (int id : ids)
+    if (!lane_capable(e->ens[id])) return false;
+  return e->opt.solo != 0;
+}
+
 // Its working memory: a record per strand slot, allocated when a pass first can use it,
 // and its rate tables for short strands.  It gives way to anything else: not taken beyond
 // a quarter of the free device memory, and given back when an allocation fails (the other
@@ -620,7 +631,7 @@ void release_lane(dsm_engine* e) {
   e->d_rec_cap = 0;
 }
 int ensure_lane(dsm_engine* e, const std::vector<int>& ids) {
-  if (!lane_quads(e, ids)) return DSM_OK;
+  if (!lane_quads(e, ids) && !solo_capable(e, ids)) return DSM_OK;
   if (!e->d_lane_tab) {
     std::vector<float> t, out((size_t)kLaneTabFloats, 0.0f);
     build_tables(t, kLaneN, 1.0f, 0, 0.0f);
@@ -632,7 +643,7 @@ int ensure_lane(dsm_engine* e, const std::vector<int>& ids) {
     if (rc) return rc;
     HIPCHK(hipMemcpy(e->d_lane_tab, out.data(), sizeof(float) * out.size(), hipMemcpyHostToDevice));
   }
-  if (e->nstr > e->d_rec_cap) {
+  if (lane_quads(e, ids) && e->nstr > e->d_rec_cap) {
     release_lane(e);
     const size_t bytes = sizeof(float) * kLaneRecFloats * (size_t)e->nstr;
     size_t free_b = 0, total_b = 0;
@@ -742,6 +753,7 @@ struct Pass {
   int n0 = 0;  // entries of the bin-0 list
   int bin_max = 0;
   int lane_quads = 0;       // > 0: the lane form with this many quads per chain
+  bool solo = false;        // the solo form instead of the wave forms
   int nmax = 0;
   bool concurrent = false;  // batched passes only: split by Z, geometries side by side
   int n_ens = 0;
@@ -771,6 +783,7 @@ int pass_setup(dsm_engine* e, const std::vector<int>& ids, bool use_ev_stop, Pas
   ps.n_ens = (int)ids.size();
   ps.n_live = (int)n_all;
   ps.lane_quads = batched && e->d_rec_cap >= e->nstr ? lane_quads(e, ids) : 0;
+  ps.solo = batched && e->d_lane_tab && solo_capable(e, ids);
   ps.nmax = 0;
   for (int id : ids) ps.nmax = std::max(ps.nmax, e->ens[id].nmax);
   // geometries side by side when chains beyond the first wave-form geometry can occur
@@ -805,6 +818,13 @@ int pass_setup(dsm_engine* e, const std::vector<int>& ids, bool use_ev_stop, Pas
 constexpr int kLateFirst = 2;
 int late_last(int bin_max) { return std::max(bin_max, kLateFirst); }
 
+// Launches bin b >= kLateFirst of a batched pass: the solo form, or the wave form `geom`.
+hipError_t launch_wave(dsm_engine* e, const Pass& ps, const KmcArgs& a, int b, int geom, hipStream_t st) {
+  if (!ps.solo) return launch_kmc(a, geom, false, device_blocks(e, geom, false, a.lds_floats, a.ext != 0), st);
+  const int cap = kmc_geom_capacity(b);
+  return launch_kmc_solo(a, cap, std::min(ps.n0, kmc_solo_occupancy(cap) * e->n_cu), st);
+}
+
 // Batched pass with the geometries side by side: the chains are split by their current
 // Z into one list per geometry and every geometry runs at once, each on its own
 // stream, the largest first (its few long chains take their slots before the bulk fills
@@ -826,7 +846,6 @@ int pass_bins_concurrent(dsm_engine* e, Pass& ps, dsm_run_stats* rs) {
     a.overflow = list(out);
     a.n_overflow = cnt + out;
   };
-  auto grid = [&](int b) { return device_blocks(e, b, false, a.lds_floats, a.ext != 0); };
   auto late_of = [&](int b) { return kLateList + (b < kLateFirst ? kLateFirst : b + 1); };  // bin b's overflow
   const bool timed = !e->capturing;  // a captured pass is timed as a whole, around its replay
   if (timed) HIPCHK(hipEventRecord(e->cev[0], e->st));
@@ -845,7 +864,7 @@ int pass_bins_concurrent(dsm_engine* e, Pass& ps, dsm_run_stats* rs) {
   // launches of the G = 2 and G = 1 bins, which share their work queues, so whichever
   // stream is free first takes the remaining chains (a launch that finds its queue empty
   // exits at once).  The G = 2 runs, longer than the G = 1 ones, start with the pass.
-  // Measured on the 262,144-chain melt, per 16 tau_K window: 111-113 ms; 118-123 ms with
+  // Measured with the wave forms on the 262,144-chain melt, per 16 tau_K window: 111-113 ms; 118-123 ms with
   // the G = 1 bulk at the start and G = 2 behind G = 8; 128-136 ms with both bins in one
   // launch, G = 2 first.  The G = 4 waves (260 registers) find few SIMDs with room beside
   // the bulk's persistent waves and run their chains a few after one another (110 ms for
@@ -870,7 +889,7 @@ int pass_bins_concurrent(dsm_engine* e, Pass& ps, dsm_run_stats* rs) {
     bind(kSplitList + b, late_of(b));
     ++rs->kmc_launches;
     const int geom = (b == 2 && wide) ? kGeomPair2 : b;
-    return launch_kmc(a, geom, false, grid(geom), stream(k));
+    return launch_wave(e, ps, a, b, geom, stream(k));
   };
   HIPCHK(first(5, 0));
   for (int k = 1; k < 4; ++k) HIPCHK(hipStreamWaitEvent(e->xs[k], e->ev_split, 0));
@@ -890,7 +909,7 @@ int pass_bins_concurrent(dsm_engine* e, Pass& ps, dsm_run_stats* rs) {
   // bulk, instead of after the whole first round (118-123 ms per window against 123-126
   // with the earlier stream layout)
   bind(kLateList + kLateFirst, late_of(kLateFirst));
-  HIPCHK(launch_kmc(a, kLateFirst, false, grid(kLateFirst), e->xs[2]));
+  HIPCHK(launch_wave(e, ps, a, kLateFirst, kLateFirst, e->xs[2]));
   rs->kmc_launches += 2;
   HIPCHK(first(3, 0));
   HIPCHK(first(2, 0));
@@ -899,7 +918,7 @@ int pass_bins_concurrent(dsm_engine* e, Pass& ps, dsm_run_stats* rs) {
   // late launches: chains that outgrew their geometry, through the larger ones in order
   for (int b = kLateFirst + 1; b <= late_last(ps.bin_max); ++b) {
     bind(kLateList + b, late_of(b));
-    HIPCHK(launch_kmc(a, b, false, grid(b), e->st));
+    HIPCHK(launch_wave(e, ps, a, b, b, e->st));
   }
   if (timed) HIPCHK(hipEventRecord(e->cev[3], e->st));
   ps.pending = timed ? 2 : 0;  // read by pass_times after the caller's next synchronisation
@@ -957,6 +976,8 @@ int pass_bins(dsm_engine* e, Pass& ps, bool plain, bool timed, dsm_run_stats* rs
       const int rounds = (ps.n_live + waves * most - 1) / (waves * most);
       a.lanes = std::max(1, (ps.n_live + waves * rounds - 1) / (waves * rounds));
       HIPCHK(launch_kmc_lane(a, ps.lane_quads, e->n_cu, e->st));
+    } else if (!plain && b >= kLateFirst) {
+      HIPCHK(launch_wave(e, ps, a, b, b, e->st));
     } else {
       HIPCHK(launch_kmc(a, b, plain, device_blocks(e, b, plain, a.lds_floats, a.ext != 0), e->st));
     }
@@ -1857,6 +1878,7 @@ int dsm_set_option(dsm_engine* e, int32_t key, int32_t value) {
     case DSM_OPT_WINDOW: if (value < 1) break; o.window = value; return DSM_OK;
     case DSM_OPT_GRAPH: if (value < 0 || value > 1) break; o.graph = value; return DSM_OK;
     case DSM_OPT_LANE: if (value < 0 || value > 2) break; o.lane = value; return DSM_OK;
+    case DSM_OPT_SOLO: if (value < 0 || value > 1) break; o.solo = value; return DSM_OK;
     case DSM_OPT_WIDE_PAIR: if (value < 0 || value > 1) break; o.wide_pair = value; return DSM_OK;
     default: return fail(DSM_ERR_ARG, "unknown option %d", key);
   }
@@ -1876,6 +1898,7 @@ int dsm_get_option(dsm_engine* e, int32_t key, int32_t* value) {
     case DSM_OPT_WINDOW: *value = o.window; return DSM_OK;
     case DSM_OPT_GRAPH: *value = o.graph; return DSM_OK;
     case DSM_OPT_LANE: *value = o.lane; return DSM_OK;
+    case DSM_OPT_SOLO: *value = o.solo; return DSM_OK;
     case DSM_OPT_WIDE_PAIR: *value = o.wide_pair; return DSM_OK;
     default: return fail(DSM_ERR_ARG, "unknown option %d", key);
   }

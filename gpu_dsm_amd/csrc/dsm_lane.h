@@ -304,6 +304,34 @@ __device__ __forceinline__ void rec_get4(const LaneRec* r, float (&q)[4], float 
   N[2] = __float_as_int(c.x); q[3] = c.y; w[3] = c.z; N[3] = __float_as_int(c.w);
 }
 
+// Rates of the quad of positions p0 .. p0+3 of a chain of Z strands: of the pair to a
+// position's right, the chain-end rates' sum `ee` at Z-1, zero behind it.  N, q: lengths and
+// |Q|^2 of positions p0 .. p0+4, lengths outside the chain given as 1.
+__device__ __forceinline__ void lane_quad_rates(const LaneCtx& C, int ens, int cd, float cc, int Z, int p0,
+                                                const int (&N)[5], const float (&q)[5], const float (&ww)[4], float ee,
+                                                float (&R)[4]) {
+  LaneStrand t[5];
+#pragma unroll
+  for (int k = 0; k < 5; ++k) t[k] = lane_strand(C, N[k], q[k], p0 + k == 0 || p0 + k == Z - 1);
+  bool slow = false;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int p = p0 + k;
+    float wp, wm;
+    const bool far = lane_pair(C, t[k], t[k + 1], wp, wm) || N[k] + N[k + 1] >= kLaneN;
+    slow = slow || (far && p <= Z - 2);
+    R[k] = p <= Z - 2 ? lane_total(cd, cc, N[k], wp, wm, ww[k]) : (p == Z - 1 ? ee : 0.0f);
+  }
+  if (slow) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      float wp, wm;
+      if (p0 + k <= Z - 2)
+        lane_pair_any(ens, cd, N[k], N[k + 1], q[k], q[k + 1], ww[k], p0 + k == 0, p0 + k + 2 == Z, wp, wm, R[k]);
+    }
+  }
+}
+
 // Load the chains of lanes `m` from the chain arrays: rates into LDS, records into `rec`.
 template <int NQ>
 __device__ __forceinline__ void lane_load(const LaneCtx& C, const KmcArgs& a, const LaneChain& H, uint64_t m) {
@@ -333,26 +361,7 @@ __device__ __forceinline__ void lane_load(const LaneCtx& C, const KmcArgs& a, co
         const float q[5] = {q2_of(x.x, y.x, z.x), q2_of(x.y, y.y, z.y), q2_of(x.z, y.z, z.z), q2_of(x.w, y.w, z.w),
                             q2_of(x4, y4, z4)};
         const float ww[4] = {w.x, w.y, w.z, w.w};
-        LaneStrand t[5];
-#pragma unroll
-        for (int k = 0; k < 5; ++k) t[k] = lane_strand(C, N[k], q[k], p0 + k == 0 || p0 + k == Z - 1);
-        bool slow = false;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const int p = p0 + k;
-          float wp, wm;
-          const bool far = lane_pair(C, t[k], t[k + 1], wp, wm) || N[k] + N[k + 1] >= kLaneN;
-          slow = slow || (far && p <= Z - 2);
-          R[k] = p <= Z - 2 ? lane_total(cd, cc, N[k], wp, wm, ww[k]) : (p == Z - 1 ? ee : 0.0f);
-        }
-        if (slow) {
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            float wp, wm;
-            if (p0 + k <= Z - 2)
-              lane_pair_any(ens, cd, N[k], N[k + 1], q[k], q[k + 1], ww[k], p0 + k == 0, p0 + k + 2 == Z, wp, wm, R[k]);
-          }
-        }
+        lane_quad_rates(C, ens, cd, cc, Z, p0, N, q, ww, ee, R);
         const int ns[4] = {N[0] | p0 << 16, N[1] | (p0 + 1) << 16, N[2] | (p0 + 2) << 16, N[3] | (p0 + 3) << 16};
         rec_put4(C.rec + o, q, ww, ns);
         C.rq[(p0 >> 2) * C.S + src] = vf4{R[0], R[1], R[2], R[3]};
@@ -530,67 +539,152 @@ __device__ __forceinline__ uint4 lane_step_words(const LaneChain& H, uint64_t ev
   return lane_philox(make_uint4((uint32_t)ev, (uint32_t)(ev >> 32), H.cid, kPurposeStep), H.key0, H.key1);
 }
 
+// The header of chain H.c of H.Z strands.
+__device__ __forceinline__ void lane_begin(const KmcArgs& a, LaneChain& H) {
+  const double kNever = __longlong_as_double(0x7ff0000000000000ll);
+  const int c = H.c;
+  const ChainArrays& ch = a.ch;
+  H.ens = ch.ens[c]; H.stall = 0; H.cid = ch.cid[c];
+  H.base = ch.base[c]; H.t = ch.t[c]; H.next_sample = ch.next_sample[c]; H.ev = ch.ev[c]; H.zsum = 0;
+  H.dt_prev = ch.dt_prev[c];
+  const uint64_t stop = a.use_ev_stop ? ch.ev_stop[c] : ~0ull;
+  H.left = stop <= H.ev ? 0 : (stop - H.ev > 0x7fffffffull ? 0x7fffffff : (int)(stop - H.ev));
+  const EnsParams* P = a.ens + H.ens;
+  H.key0 = P->key0; H.key1 = P->key1; H.beta = P->beta; H.cd = P->cd; H.exp_wait = P->exp_wait;
+  H.cc = P->cd ? P->c_create : 0.0f;
+  H.t_end = P->t_end;
+  H.t_next = H.next_sample < P->k_end && P->sample_mode != kSampleNone ? (double)H.next_sample * P->delta : kNever;
+  H.N0 = ch.N[H.base]; H.N1 = ch.N[H.base + (H.Z > 1 ? 1 : 0)];
+  H.Nz = ch.N[H.base + H.Z - 1]; H.Nz2 = ch.N[H.base + (H.Z > 1 ? H.Z - 2 : 0)];
+  lane_end_rates(H);
+  H.rnd = lane_step_words(H, H.ev);
+  H.msd = P->sample_mode == kSampleMsd;
+  H.pd = P->partner ? P->pd_off : -1;
+  H.kind = kEvNone;
+}
+
+// A chain's total rate and, once W*u is known, the quad of the first position whose
+// inclusive sum exceeds it, from its quad sums.
+template <int NQ>
+struct LanePick {
+  float X0[16], I0[16], X1[16], I1[16], B0;
+  float Xl, Gl, cin;  // sums before the quad: within its block, over the chain; before the block
+  __device__ __forceinline__ float total(const float (&lf)[NQ], int Z) {
+    B0 = lane_tree<NQ, 0>(lf, X0, I0);
+    float B1 = 0.0f;
+    if constexpr (NQ > 16) B1 = lane_tree<NQ, 1>(lf, X1, I1);
+    return NQ > 16 && Z > 64 ? B0 + B1 : B0;
+  }
+  // (block 1 adds block 0's total; 4 * NQ: none)
+  __device__ __forceinline__ int quad(float pr) {
+    int qp = 4 * NQ;
+    Xl = 0.0f;
+    Gl = 0.0f;
+#pragma unroll
+    for (int k = NQ - 1; k >= 16; --k) {
+      const int l = k - 16;
+      const bool g = B0 + I1[l] > pr;
+      qp = g ? k : qp;
+      Xl = g ? X1[l] : Xl;
+      Gl = g ? (l > 0 ? B0 + I1[l > 0 ? l - 1 : 0] : B0) : Gl;
+    }
+#pragma unroll
+    for (int k = (NQ < 16 ? NQ : 16) - 1; k >= 0; --k) {
+      const bool g = I0[k] > pr;
+      qp = g ? k : qp;
+      Xl = g ? X0[k] : Xl;
+      Gl = g ? (k > 0 ? I0[k > 0 ? k - 1 : 0] : 0.0f) : Gl;
+    }
+    cin = NQ > 16 && qp >= 16 ? B0 : 0.0f;
+    return qp;
+  }
+  // the position in the quad with rates R (0..3) and the sum before it
+  __device__ __forceinline__ int slot(const float (&R)[4], float pr, float& before) const {
+    const float s0 = R[0], s1 = s0 + R[1], s2 = s1 + R[2];
+    const float g0 = cin + (Xl + s0), g1 = cin + (Xl + s1), g2 = cin + (Xl + s2);
+    const int k = g0 > pr ? 0 : (g1 > pr ? 1 : (g2 > pr ? 2 : 3));
+    before = k == 0 ? Gl : (k == 1 ? g0 : (k == 2 ? g1 : g2));
+    return k;
+  }
+};
+
+// Waiting time and clock of a jump with total rate W; false: the chain stalls.
+__device__ __forceinline__ bool lane_clock(LaneChain& H, float W, const uint4& rnd) {
+  float dt;
+  if (H.exp_wait) dt = (-dlogf(u01(rnd.y))) / W;
+  else dt = 1.0f / W;
+  if (__builtin_amdgcn_classf(dt, 0x263)) {  // zero, NaN or +infinity
+    H.stall = dt == 0.0f ? 1 : (dt != dt ? 2 : 3);
+    return false;
+  }
+  H.t += (double)dt;
+  H.dt_prev = dt;
+  H.ev += 1;
+  H.zsum += (uint64_t)H.Z;
+  --H.left;
+  return true;
+}
+
+// The sub-event of position p in the reference order: of a pair, from its CD and shift
+// rates; at the end position, from the chain-end rates.  r becomes what is left of it.
+__device__ __forceinline__ int lane_kind(const LaneChain& H, bool pair, float w, float wp, float wm, int N, float& r) {
+  float v0 = H.cd ? w : 0.0f, v1 = wp, v2 = wm, v3 = H.cc * (float)(N - 1), v4 = 0.0f;
+  if (!pair) {
+    const EndRates er = lane_ends(H);
+    v0 = er.cdcz; v1 = er.sdc1; v2 = er.sdcz; v3 = er.sdd1; v4 = er.sddz;
+  }
+  const float x = r;
+  const bool t0 = v0 > 0.0f && x < v0;
+  const float x1 = x - v0;
+  const bool t1 = v1 > 0.0f && x1 < v1;
+  const float x2 = x1 - v1;
+  const bool t2 = v2 > 0.0f && x2 < v2;
+  const float x3 = x2 - v2;
+  const bool t3 = v3 > 0.0f && x3 < v3;
+  const float x4 = x3 - v3;
+  const bool t4 = v4 > 0.0f && x4 < v4;
+  const int m = t0 ? 0 : (t1 ? 1 : (t2 ? 2 : (t3 ? 3 : (t4 ? 4 : 5))));
+  r = t0 ? x : (t1 ? x1 : (t2 ? x2 : (t3 ? x3 : x4)));
+  // four bits a kind
+  constexpr uint32_t kPair = kEvCDd | kEvShiftP << 4 | kEvShiftM << 8 | kEvCDc << 12;
+  constexpr uint32_t kEnd = kEvCDcTail | kEvSDcHead << 4 | kEvSDcTail << 8 | kEvSDdHead << 12 | kEvSDdTail << 16;
+  static_assert(kEvNone == 0, "what is not listed");
+  return (int)(((pair ? kPair : kEnd) >> (4 * m)) & 15);
+}
+
+// Lengths at the chain's ends after a shift that left N at p and M at p + 1; true when one
+// of them changed.
+__device__ __forceinline__ bool lane_shift_ends(LaneChain& H, int p, int N, int M) {
+  const int Z = H.Z;
+  if (p == 0) { H.N0 = N; H.N1 = M; }
+  if (p == 1) H.N1 = N;
+  if (p == Z - 2) { H.Nz2 = N; H.Nz = M; }
+  if (p == Z - 3) H.Nz2 = M;
+  return p <= 1 || p >= Z - 3;
+}
+
 // Picks the event, applies it when it is a shift of one Kuhn step across a link, and
 // leaves a split or merge in (kind, p, r) for lane_rare.
 template <int NQ>
 __device__ __forceinline__ void lane_jump(const LaneCtx& C, LaneChain& H, float (&lf)[NQ]) {
   const uint4 rnd = H.rnd;
   const int Z = H.Z;
-  float X0[16], I0[16], X1[16], I1[16], W;
-  const float B0 = lane_tree<NQ, 0>(lf, X0, I0);
-  float B1 = 0.0f;
-  if constexpr (NQ > 16) B1 = lane_tree<NQ, 1>(lf, X1, I1);
-  W = NQ > 16 && Z > 64 ? B0 + B1 : B0;
-  float dt;
-  if (H.exp_wait) dt = (-dlogf(u01(rnd.y))) / W;
-  else dt = 1.0f / W;
+  LanePick<NQ> K;
+  const float W = K.total(lf, Z);
+  if (!lane_clock(H, W, rnd)) return;
   const float pr = W * u01(rnd.x);
-  int stl = 0;
-  if (dt == 0.0f) stl = 1;
-  if (dt != dt) stl = 2;
-  if (__float_as_uint(dt) == 0x7f800000u) stl = 3;
-  if (stl) {
-    H.stall = stl;
-    return;
-  }
-  H.t += (double)dt;
-  H.dt_prev = dt;
-  H.ev += 1;
-  H.zsum += (uint64_t)Z;
-  --H.left;
-  // the quad of the first position whose inclusive sum exceeds pr; Xl, Gl: sums before it
-  // within its block and over the chain (block 1 adds block 0's total)
-  int qp = 4 * NQ;
-  float Xl = 0.0f, Gl = 0.0f;
-#pragma unroll
-  for (int k = NQ - 1; k >= 16; --k) {
-    const int l = k - 16;
-    const bool g = B0 + I1[l] > pr;
-    qp = g ? k : qp;
-    Xl = g ? X1[l] : Xl;
-    Gl = g ? (l > 0 ? B0 + I1[l > 0 ? l - 1 : 0] : B0) : Gl;
-  }
-#pragma unroll
-  for (int k = (NQ < 16 ? NQ : 16) - 1; k >= 0; --k) {
-    const bool g = I0[k] > pr;
-    qp = g ? k : qp;
-    Xl = g ? X0[k] : Xl;
-    Gl = g ? (k > 0 ? I0[k > 0 ? k - 1 : 0] : 0.0f) : Gl;
-  }
+  const int qp = K.quad(pr);
   if (qp > (Z - 1) >> 2) {  // no position: the clock moves, the chain does not
     H.rnd = lane_step_words(H, H.ev);
     return;
   }
   const int p4 = 4 * qp;
-  const float cin = NQ > 16 && qp >= 16 ? B0 : 0.0f;
   const vf4 Rv = C.rq[qp * C.S + C.lane];
   float R[4] = {Rv.x, Rv.y, Rv.z, Rv.w};
-  const float s0 = R[0], s1 = s0 + R[1], s2 = s1 + R[2];
-  const float g0 = cin + (Xl + s0), g1 = cin + (Xl + s1), g2 = cin + (Xl + s2);
-  const int k = g0 > pr ? 0 : (g1 > pr ? 1 : (g2 > pr ? 2 : 3));
-  const float Gprev = k == 0 ? Gl : (k == 1 ? g0 : (k == 2 ? g1 : g2));
+  float before;
+  const int k = K.slot(R, pr, before);
   const int p = p4 + k;
-  float r = p == 0 ? pr : pr - Gprev;
+  float r = p == 0 ? pr : pr - before;
   // the window p-1 .. p+2 (clamped into the chain)
   LaneRec* rb = C.rec + H.base;
   const int pm1 = max(p - 1, 0), pp1 = min(p + 1, Z - 1), pp2 = min(p + 2, Z - 1);
@@ -601,38 +695,12 @@ __device__ __forceinline__ void lane_jump(const LaneCtx& C, LaneChain& H, float 
   const float q[4] = {c0.q2, c1.q2, c2.q2, c3.q2}, w[3] = {c0.w, c1.w, c2.w};
   N[2] = p + 1 < Z ? N[2] : 1;
   N[3] = p + 2 < Z ? N[3] : 1;
-  int kind = kEvNone;
   const bool pair = p < Z - 1;
-  {
-    float v0, v1, v2, v3, v4 = 0.0f;
-    float wp, wm, rr;
-    const bool far = lane_pair(C, lane_strand(C, N[1], q[1], p == 0), lane_strand(C, N[2], q[2], p + 2 == Z), wp, wm);
-    if ((far || N[1] + N[2] >= kLaneN) && pair)
-      lane_pair_any(H.ens, H.cd, N[1], N[2], q[1], q[2], w[1], p == 0, p + 2 == Z, wp, wm, rr);
-    v0 = H.cd ? w[1] : 0.0f;
-    v1 = wp;
-    v2 = wm;
-    v3 = H.cc * (float)(N[1] - 1);
-    if (!pair) {
-      const EndRates er = lane_ends(H);
-      v0 = er.cdcz; v1 = er.sdc1; v2 = er.sdcz; v3 = er.sdd1; v4 = er.sddz;
-    }
-    const float x = r;
-    const bool t0 = v0 > 0.0f && x < v0;
-    const float x1 = x - v0;
-    const bool t1 = v1 > 0.0f && x1 < v1;
-    const float x2 = x1 - v1;
-    const bool t2 = v2 > 0.0f && x2 < v2;
-    const float x3 = x2 - v2;
-    const bool t3 = v3 > 0.0f && x3 < v3;
-    const float x4 = x3 - v3;
-    const bool t4 = v4 > 0.0f && x4 < v4;
-    const int m = t0 ? 0 : (t1 ? 1 : (t2 ? 2 : (t3 ? 3 : (t4 ? 4 : -1))));
-    r = t0 ? x : (t1 ? x1 : (t2 ? x2 : (t3 ? x3 : x4)));
-    if (pair) kind = m == 0 ? kEvCDd : m == 1 ? kEvShiftP : m == 2 ? kEvShiftM : m == 3 ? kEvCDc : kEvNone;
-    else kind = m == 0 ? kEvCDcTail : m == 1 ? kEvSDcHead : m == 2 ? kEvSDcTail : m == 3 ? kEvSDdHead
-              : m == 4 ? kEvSDdTail : kEvNone;
-  }
+  float wp, wm, rr;
+  const bool far = lane_pair(C, lane_strand(C, N[1], q[1], p == 0), lane_strand(C, N[2], q[2], p + 2 == Z), wp, wm);
+  if ((far || N[1] + N[2] >= kLaneN) && pair)
+    lane_pair_any(H.ens, H.cd, N[1], N[2], q[1], q[2], w[1], p == 0, p + 2 == Z, wp, wm, rr);
+  const int kind = lane_kind(H, pair, w[1], wp, wm, N[1], r);
   if (kind != kEvShiftP && kind != kEvShiftM) {
     H.kind = kind;
     H.p = p;
@@ -647,11 +715,7 @@ __device__ __forceinline__ void lane_jump(const LaneCtx& C, LaneChain& H, float 
   N[2] -= dn;
   rb[p].ns = c1.ns + dn;
   rb[p + 1].ns = c2.ns - dn;
-  if (p == 0) { H.N0 = N[1]; H.N1 = N[2]; }
-  if (p == 1) H.N1 = N[1];
-  if (p == Z - 2) { H.Nz2 = N[1]; H.Nz = N[2]; }
-  if (p == Z - 3) H.Nz2 = N[2];
-  const bool ends = p <= 1 || p >= Z - 3;
+  const bool ends = lane_shift_ends(H, p, N[1], N[2]);
   float Rn[3];
   lane_pairs3(C, H, p - 1, Z, N, q, w, Rn);
   float eend = 0.0f;
@@ -787,84 +851,62 @@ struct RowShift {
 // tail, e = Z-1).  The lane computes the new values, the rows shift the arrays by one
 // position behind the event, the lane writes its values, and the rows rebuild the quad
 // sums.
-template <int NQ>
-__device__ __forceinline__ void lane_rare(const LaneCtx& C, const KmcArgs& a, LaneChain& H, float (&lf)[NQ],
-                                          uint64_t m) {
-  const bool on = (m >> C.lane) & 1;
-  int e = 0, dir = 0, zold = 1;
-  float x0 = 0.f, y0 = 0.f, z0 = 0.f, x1 = 0.f, y1 = 0.f, z1 = 0.f, q0 = 0.f, q1 = 0.f, w0 = 0.f, w1 = 0.f;
-  int n0 = 0, n1 = 0, sl0 = 0, sl1 = 0;
-  if (on) {
+struct LaneEvent {
+  int e, dir;              // strand; +1 split, -1 merge
+  int n0, n1;              // lengths at e and (split) e + 1
+  float x0, y0, z0, x1, y1, z1, w0, w1;
+  // The strand the waiting event acts on.
+  __device__ __forceinline__ void place(const LaneChain& H) {
+    const uint32_t k = 1u << H.kind;
+    e = k & (1u << kEvSDcHead | 1u << kEvSDdHead) ? 0 : H.p;
+    e = k & (1u << kEvSDdTail) ? H.Z - 2 : e;
+    dir = k & (1u << kEvCDd | 1u << kEvSDdHead | 1u << kEvSDdTail) ? -1 : 1;
+  }
+  // New strands from the old lengths at e-1 .. e+2 (m), CD rates (we, we1) and vectors
+  // (a, b) at e and e+1; the header follows.
+  __device__ __forceinline__ void apply(const KmcArgs& A, LaneChain& H, int m0, int m1, int m2, int m3, float we,
+                                        float we1, float ax, float ay, float az, float bx, float by, float bz) {
     const int Z = H.Z, kind = H.kind;
-    zold = Z;
-    const bool merge = kind == kEvCDd || kind == kEvSDdHead || kind == kEvSDdTail;
     const bool tail = kind == kEvCDcTail || kind == kEvSDcTail;
     const bool sd = kind == kEvSDcHead || kind == kEvSDcTail;
-    e = kind == kEvSDcHead || kind == kEvSDdHead ? 0 : (kind == kEvSDdTail ? Z - 2 : H.p);
-    // the old values at e-1 .. e+2, clamped into the chain, and the constants of the
-    // lifetime law of a new link; the random numbers while they are on their way
-    const LaneRec* rb = C.rec + H.base;
-    const LaneRec o0 = rb[max(e - 1, 0)], o1 = rb[e], o2 = rb[min(e + 1, Z - 1)], o3 = rb[min(e + 2, Z - 1)];
-    const EnsParams* P = a.ens + H.ens;
-    const float* law = H.pd >= 0 ? a.tabs + H.pd + 5 * ((sd ? 0 : kPartnerK) + (int)(H.rw >> (32 - kPartnerBits)))
-                                 : (sd ? P->law_ft : P->law_fdt);
-    const float l0 = law[0], l1 = law[1], l2 = law[2], l3 = law[3], l4 = law[4];
-    float g0 = 0.f, g1 = 0.f, g2 = 0.f, wn = 0.f;
-    if (!merge) {
-      const uint64_t evj = H.ev - 1;
-      const uint4 gr = lane_philox(make_uint4((uint32_t)evj, (uint32_t)(evj >> 32), H.cid, kPurposeGauss), H.key0, H.key1);
-      float g3;
-      boxmuller(gr.x, gr.y, g0, g1);
-      boxmuller(gr.z, gr.w, g2, g3);
-      // rate_ft (s_At s_Ct s_Dt s_taud_inv s_one_minus_g) or rate_fdt (s_Adt s_Bdt s_Cdt
-      // s_Ddt s_taud_inv)
-      const float u = u01(H.rz);
-      const float thr = sd ? l4 : l1, A = l0, D = sd ? l2 : l3, ex = sd ? l1 : l2, slow = sd ? l3 : l4;
-      wn = u < thr ? dpowf(__builtin_fmaf(u, A, D), ex) : slow;
-    }
-    const int64_t v1 = H.base + o1.slot(), v2 = H.base + o2.slot();
-    const float ax = a.ch.Qx[v1], ay = a.ch.Qy[v1], az = a.ch.Qz[v1];
-    const float bx = a.ch.Qx[v2], by = a.ch.Qy[v2], bz = a.ch.Qz[v2];
-    const int m0 = o0.N(), m1 = o1.N(), m2 = o2.N(), m3 = o3.N();
-    sl0 = o1.slot();
-    int N[4];
-    float q[4], w[3];
-    N[0] = e > 0 ? m0 : 1;
-    q[0] = o0.q2;
-    w[0] = o0.w;
-    if (merge) {
-      dir = -1;
+    x0 = y0 = z0 = x1 = y1 = z1 = 0.0f;
+    w1 = 0.0f;
+    n1 = 0;
+    if (dir < 0) {
       n0 = m1 + m2;
-      if (kind == kEvCDd && !(e == 0 || e == Z - 2)) {
-        x0 = ax + bx; y0 = ay + by; z0 = az + bz;
-      }
+      if (kind == kEvCDd && !(e == 0 || e == Z - 2)) { x0 = ax + bx; y0 = ay + by; z0 = az + bz; }
       if (H.msd && e == 0 && kind != kEvSDdTail) {  // the first entanglement goes: R1 moves forward by the old Q_1
-        float* r1 = a.ch.R1 + 3 * (int64_t)H.c;
+        float* r1 = A.ch.R1 + 3 * (int64_t)H.c;
         r1[0] = r1[0] + bx; r1[1] = r1[1] + by; r1[2] = r1[2] + bz;
       }
-      const int s1 = o2.slot();
-#pragma unroll
-      for (int k = 0; k < (NQ + 7) / 8; ++k) H.used[k] &= (s1 >> 5) == k ? ~(1u << (s1 & 31)) : ~0u;
-      q0 = q2_of(x0, y0, z0);
-      w0 = kind == kEvSDdTail ? 0.0f : o2.w;
+      w0 = kind == kEvSDdTail ? 0.0f : we1;
       H.Z = Z - 1;
-      N[1] = n0;
-      N[2] = e + 2 < Z ? m3 : 1;
-      N[3] = 1;
-      q[1] = q0; q[2] = o3.q2; q[3] = 0.0f;
-      w[1] = w0; w[2] = 0.0f;
-      if (e == 0) { H.N0 = n0; H.N1 = N[2]; }
+      if (e == 0) { H.N0 = n0; H.N1 = e + 2 < Z ? m3 : 1; }
       if (e == 1) H.N1 = n0;
-      if (e == Z - 2) { H.Nz = n0; H.Nz2 = N[0]; }
+      if (e == Z - 2) { H.Nz = n0; H.Nz2 = e > 0 ? m0 : 1; }
       if (e == Z - 3) H.Nz2 = n0;
     } else {
-      dir = 1;
+      // the lifetime law's constants (on their way during the random numbers): rate_ft
+      // (s_At s_Ct s_Dt s_taud_inv s_one_minus_g) or rate_fdt (s_Adt s_Bdt s_Cdt s_Ddt
+      // s_taud_inv)
+      const EnsParams* P = A.ens + H.ens;
+      const float* law = H.pd >= 0 ? A.tabs + H.pd + 5 * ((sd ? 0 : kPartnerK) + (int)(H.rw >> (32 - kPartnerBits)))
+                                   : (sd ? P->law_ft : P->law_fdt);
+      const float l0 = law[0], l1 = law[1], l2 = law[2], l3 = law[3], l4 = law[4];
+      const uint64_t evj = H.ev - 1;
+      const uint4 gr = lane_philox(make_uint4((uint32_t)evj, (uint32_t)(evj >> 32), H.cid, kPurposeGauss), H.key0, H.key1);
+      float g0, g1, g2, g3;
+      boxmuller(gr.x, gr.y, g0, g1);
+      boxmuller(gr.z, gr.w, g2, g3);
+      const float u = u01(H.rz);
+      const float thr = sd ? l4 : l1, D = sd ? l2 : l3, ex = sd ? l1 : l2, slow = sd ? l3 : l4;
+      const float wn = u < thr ? dpowf(__builtin_fmaf(u, l0, D), ex) : slow;
       const int Ne = m1;
       const float wc = H.cc * (float)(Ne - 1);
       n0 = kind == kEvSDcHead ? 1 : (kind == kEvSDcTail ? Ne - 1 : split_newn(H.r, Ne, wc));
       n1 = Ne - n0;
       w0 = sd && !H.cd ? 0.0f : wn;
-      w1 = tail ? 0.0f : o1.w;
+      w1 = tail ? 0.0f : we;
       // the vectors: all zero but the new strand's at the ends
       const float num = tail ? (float)n0 : (e == 0 ? (float)n1 : (float)n0 * (float)n1);
       const float den = tail || e == 0 ? 3.0f : 3.0f * (float)Ne;
@@ -883,32 +925,63 @@ __device__ __forceinline__ void lane_rare(const LaneCtx& C, const KmcArgs& a, La
         x1 = ax - x0; y1 = ay - y0; z1 = az - z0;
       }
       if (H.msd && ((kind == kEvCDc && e == 0) || kind == kEvSDcHead)) {  // a new first one: back by the new Q_1
-        float* r1 = a.ch.R1 + 3 * (int64_t)H.c;
+        float* r1 = A.ch.R1 + 3 * (int64_t)H.c;
         r1[0] = r1[0] - x1; r1[1] = r1[1] - y1; r1[2] = r1[2] - z1;
       }
-      // the first free slot
-      sl1 = 0;
-#pragma unroll
-      for (int k = (NQ + 7) / 8 - 1; k >= 0; --k) sl1 = ~H.used[k] ? 32 * k + __builtin_ctz(~H.used[k]) : sl1;
-#pragma unroll
-      for (int k = 0; k < (NQ + 7) / 8; ++k) H.used[k] |= (sl1 >> 5) == k ? 1u << (sl1 & 31) : 0u;
-      q0 = q2_of(x0, y0, z0);
-      q1 = q2_of(x1, y1, z1);
       H.Z = Z + 1;
-      N[1] = n0;
-      N[2] = n1;
-      N[3] = e + 1 < Z ? m2 : 1;
-      q[1] = q0; q[2] = q1; q[3] = o2.q2;
-      w[1] = w0; w[2] = w1;
       if (e == 0) { H.N0 = n0; H.N1 = n1; }
       if (e == 1) H.N1 = n0;
       if (e == Z - 1) { H.Nz2 = n0; H.Nz = n1; }
       if (e == Z - 2) H.Nz2 = n1;
     }
     H.kind = kEvNone;
+    lane_end_rates(H);
+  }
+};
+
+template <int NQ>
+__device__ __forceinline__ void lane_rare(const LaneCtx& C, const KmcArgs& a, LaneChain& H, float (&lf)[NQ],
+                                          uint64_t m) {
+  const bool on = (m >> C.lane) & 1;
+  LaneEvent E;
+  E.e = 0;
+  E.dir = 0;
+  int zold = 1, sl0 = 0, sl1 = 0;
+  float q0 = 0.f, q1 = 0.f;
+  if (on) {
+    const int Z = H.Z;
+    zold = Z;
+    E.place(H);
+    const int e = E.e;
+    // the old values at e-1 .. e+2, clamped into the chain
+    const LaneRec* rb = C.rec + H.base;
+    const LaneRec o0 = rb[max(e - 1, 0)], o1 = rb[e], o2 = rb[min(e + 1, Z - 1)], o3 = rb[min(e + 2, Z - 1)];
+    const int64_t v1 = H.base + o1.slot(), v2 = H.base + o2.slot();
+    const float ax = a.ch.Qx[v1], ay = a.ch.Qy[v1], az = a.ch.Qz[v1];
+    const float bx = a.ch.Qx[v2], by = a.ch.Qy[v2], bz = a.ch.Qz[v2];
+    E.apply(a, H, o0.N(), o1.N(), o2.N(), o3.N(), o1.w, o2.w, ax, ay, az, bx, by, bz);
+    q0 = q2_of(E.x0, E.y0, E.z0);
+    q1 = q2_of(E.x1, E.y1, E.z1);
+    sl0 = o1.slot();
+    const bool split = E.dir > 0;
+    // a merge frees the slot of e+1, a split takes the first free one
+    if (split) {
+#pragma unroll
+      for (int k = (NQ + 7) / 8 - 1; k >= 0; --k) sl1 = ~H.used[k] ? 32 * k + __builtin_ctz(~H.used[k]) : sl1;
+    }
+    const int sx = split ? sl1 : o2.slot();
+#pragma unroll
+    for (int k = 0; k < (NQ + 7) / 8; ++k) {
+      const uint32_t bit = (sx >> 5) == k ? 1u << (sx & 31) : 0u;
+      H.used[k] = split ? H.used[k] | bit : H.used[k] & ~bit;
+    }
+    const int N[4] = {e > 0 ? o0.N() : 1, E.n0, split ? E.n1 : (e + 2 < Z ? o3.N() : 1),
+                      split && e + 1 < Z ? o2.N() : 1};
+    const float q[4] = {o0.q2, q0, split ? q1 : o3.q2, split ? o2.q2 : 0.0f};
+    const float w[3] = {o0.w, E.w0, E.w1};
+    const int dir = E.dir;
     float Rn[3];
     lane_pairs3(C, H, e - 1, H.Z, N, q, w, Rn);
-    lane_end_rates(H);
     // the rates behind the event move by one position in the lane's own column: position
     // p > e+1 takes the old p-1 (split), position p > e the old p+1 (merge; a zero follows
     // the last rate)
@@ -949,7 +1022,7 @@ __device__ __forceinline__ void lane_rare(const LaneCtx& C, const KmcArgs& a, La
   constexpr int NB = (NQ + 15) / 16;
   for (uint64_t mm = m; mm;) {
     RowShift row;
-    row.take(C, mm, e, dir, zold, H.base);
+    row.take(C, mm, E.e, E.dir, zold, H.base);
 #pragma unroll 1
     for (int i = 0; i < NB; ++i) {
       row.load(C, i, NB);
@@ -957,15 +1030,14 @@ __device__ __forceinline__ void lane_rare(const LaneCtx& C, const KmcArgs& a, La
     }
   }
   wave_lds_sync();
-  // the lane's new strands
-  if (on) {
-    const int64_t o = H.base + e, v = H.base + sl0;
-    C.rec[o] = LaneRec{q0, w0, n0 | sl0 << 16};
-    a.ch.Qx[v] = x0; a.ch.Qy[v] = y0; a.ch.Qz[v] = z0;
-    if (dir > 0) {
+  if (on) {  // the lane's new strands
+    const int64_t o = H.base + E.e, v = H.base + sl0;
+    C.rec[o] = LaneRec{q0, E.w0, E.n0 | sl0 << 16};
+    a.ch.Qx[v] = E.x0; a.ch.Qy[v] = E.y0; a.ch.Qz[v] = E.z0;
+    if (E.dir > 0) {
       const int64_t v1 = H.base + sl1;
-      C.rec[o + 1] = LaneRec{q1, w1, n1 | sl1 << 16};
-      a.ch.Qx[v1] = x1; a.ch.Qy[v1] = y1; a.ch.Qz[v1] = z1;
+      C.rec[o + 1] = LaneRec{q1, E.w1, E.n1 | sl1 << 16};
+      a.ch.Qx[v1] = E.x1; a.ch.Qy[v1] = E.y1; a.ch.Qz[v1] = E.z1;
     }
   }
 }
@@ -1071,30 +1143,12 @@ __global__ void __launch_bounds__(64 * kLaneWaves) __attribute__((amdgpu_waves_p
           break;
         }
         if (H.c >= 0) {
-          const int c = H.c;
-          const ChainArrays& ch = a.ch;
-          H.ens = ch.ens[c]; H.stall = 0; H.cid = ch.cid[c];
-          H.base = ch.base[c]; H.t = ch.t[c]; H.next_sample = ch.next_sample[c]; H.ev = ch.ev[c]; H.zsum = 0;
-          H.dt_prev = ch.dt_prev[c];
-          const uint64_t stop = a.use_ev_stop ? ch.ev_stop[c] : ~0ull;
-          H.left = stop <= H.ev ? 0 : (stop - H.ev > 0x7fffffffull ? 0x7fffffff : (int)(stop - H.ev));
-          const EnsParams* P = a.ens + H.ens;
-          H.key0 = P->key0; H.key1 = P->key1; H.beta = P->beta; H.cd = P->cd; H.exp_wait = P->exp_wait;
-          H.cc = P->cd ? P->c_create : 0.0f;
-          H.t_end = P->t_end;
-          H.t_next = H.next_sample < P->k_end && P->sample_mode != kSampleNone ? (double)H.next_sample * P->delta : kNever;
-          H.N0 = ch.N[H.base]; H.N1 = ch.N[H.base + (H.Z > 1 ? 1 : 0)];
-          H.Nz = ch.N[H.base + H.Z - 1]; H.Nz2 = ch.N[H.base + (H.Z > 1 ? H.Z - 2 : 0)];
-          lane_end_rates(H);
-          H.rnd = lane_step_words(H, H.ev);
-          H.msd = P->sample_mode == kSampleMsd;
-          H.pd = P->partner ? P->pd_off : -1;
+          lane_begin(a, H);
 #pragma unroll
           for (int k = 0; k < (NQ + 7) / 8; ++k) {
             const int z = H.Z - 32 * k;
             H.used[k] = z >= 32 ? ~0u : (z > 0 ? (1u << z) - 1u : 0u);
           }
-          H.kind = kEvNone;
         }
       }
       const uint64_t ml = __ballot(need && H.c >= 0);

@@ -55,6 +55,10 @@ constexpr int lane_max_lanes(int quads) {
   return odd > 64 ? 64 : odd;
 }
 hipError_t launch_kmc_lane(const KmcArgs& a, int quads, int grid, hipStream_t st);
+// The solo form (one chain per wave, `cap` positions in LDS, a multiple of 4): waves per CU,
+// and a launch of `grid` waves.
+int kmc_solo_occupancy(int cap);
+hipError_t launch_kmc_solo(const KmcArgs& a, int cap, int grid, hipStream_t st);
 // chains first .. first+n-1
 hipError_t launch_init_eq(const ChainArrays& ch, const EnsParams* ens, const float* tabs, int first, int n,
                           hipStream_t st);

@@ -1,0 +1,29 @@
+// dsm_solo_inst.hip -- instantiates the solo form of the KMC kernels (dsm_solo.h).
+#include "dsm_solo.h"
+
+namespace dsm {
+
+namespace {
+size_t solo_lds(int cap) { return sizeof(float) * (kLaneTabFloats + 4 * (size_t)cap); }
+}  // namespace
+
+int kmc_solo_occupancy(int cap) {
+  int n = 0;
+  const hipError_t rc =
+      cap > 256 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kmc_solo_kernel<true>, 64, solo_lds(cap))
+                : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kmc_solo_kernel<false>, 64, solo_lds(cap));
+  if (rc != hipSuccess) return 1;
+  return n < 1 ? 1 : n;
+}
+
+hipError_t launch_kmc_solo(const KmcArgs& a, int cap, int grid, hipStream_t st) {
+  if (grid <= 0) return hipSuccess;
+  if (cap <= 0 || (cap & 3)) return hipErrorInvalidValue;
+  KmcArgs b = a;
+  b.cap = cap;
+  if (cap > 256) hipLaunchKernelGGL((kmc_solo_kernel<true>), dim3(grid), dim3(64), solo_lds(cap), st, b);
+  else hipLaunchKernelGGL((kmc_solo_kernel<false>), dim3(grid), dim3(64), solo_lds(cap), st, b);
+  return hipGetLastError();
+}
+
+}  // namespace dsm

@@ -102,6 +102,7 @@ struct KmcArgs {
   int plain_jumps;      // plain form: jumps per chain per launch
   float* rec;           // lane form: a record {|Q|^2, w, N} per strand slot
   const float* lane_tab;  // lane form: the rate tables that depend on N alone, for short strands
+  int cap;              // solo form: positions of a chain in LDS (a multiple of 4)
   int lanes;            // lane form: lanes of a wave that take chains (1..64)
 };
 
