@@ -301,6 +301,7 @@ struct Ens {
   int64_t strand0 = 0, nstrand = 0;
   EnsParams P{};
   int bin_max = 0;      // largest geometry bin a chain of this ensemble can need
+  int n_lane = 0;          // its chains that stay within the lane form's largest columns
   double z_sum_est = 0.0;  // sum over its chains of the equilibrium mean Z, (Nk + beta) / (1 + beta)
   // sampling
   int ncomp = 0;        // floats per sample per chain (3 G(t), 8 flow)
@@ -608,6 +609,25 @@ int lane_quads(const dsm_engine* e, const std::vector<int>& ids) {
   return quads;
 }
 
+// Chains of a pass of mixed lengths that run in the lane form before the longer ones start
+// (its workgroups take whole CUs), or 0.  Beside them the pass loses the time in which its
+// longest chains' serial runs would overlap the rest: measured with nothing above 256
+// positions (Nk 200, 8 tau_K) 3.54 ms without against 4.29 ms with 15,000 such chains, 6.24 /
+// 4.81 with 30,000, 11.2 / 5.5 with 60,000; with longer ones (the polydisperse melt, 16
+// tau_K) 18.4 / 22.8 with 46,000, 26.1 / 27.0 with 69,000, 33.8 / 32.4 with 92,000, 64 / 58
+// with 184,000.
+int lane_share(const dsm_engine* e, const std::vector<int>& ids) {
+  if (e->opt.lane == 0) return 0;
+  int64_t n = 0;
+  bool longer = false;
+  for (int id : ids) {
+    if (!lane_capable(e->ens[id])) return 0;
+    n += e->ens[id].n_lane;
+    longer = longer || e->ens[id].bin_max >= 3;
+  }
+  return e->opt.lane == 2 || n >= (longer ? 80000 : 22000) ? (int)n : 0;
+}
+
 // The solo form (dsm_solo.h) takes the place of the wave forms (bins 2 and up) wherever no
 // chain flows: a jump costs it the same at any length, so it gains most on the long chains
 // (Nk 1000: 2.7 times; Nk 600: 1.8; Nk 300, against the two-chain form: 1.08) and is level
@@ -631,7 +651,8 @@ void release_lane(dsm_engine* e) {
   e->d_rec_cap = 0;
 }
 int ensure_lane(dsm_engine* e, const std::vector<int>& ids) {
-  if (!lane_quads(e, ids) && !solo_capable(e, ids)) return DSM_OK;
+  const bool lanes = lane_quads(e, ids) || lane_share(e, ids);
+  if (!lanes && !solo_capable(e, ids)) return DSM_OK;
   if (!e->d_lane_tab) {
     std::vector<float> t, out((size_t)kLaneTabFloats, 0.0f);
     build_tables(t, kLaneN, 1.0f, 0, 0.0f);
@@ -643,7 +664,7 @@ int ensure_lane(dsm_engine* e, const std::vector<int>& ids) {
     if (rc) return rc;
     HIPCHK(hipMemcpy(e->d_lane_tab, out.data(), sizeof(float) * out.size(), hipMemcpyHostToDevice));
   }
-  if (lane_quads(e, ids) && e->nstr > e->d_rec_cap) {
+  if (lanes && e->nstr > e->d_rec_cap) {
     release_lane(e);
     const size_t bytes = sizeof(float) * kLaneRecFloats * (size_t)e->nstr;
     size_t free_b = 0, total_b = 0;
@@ -753,6 +774,7 @@ struct Pass {
   int n0 = 0;  // entries of the bin-0 list
   int bin_max = 0;
   int lane_quads = 0;       // > 0: the lane form with this many quads per chain
+  int n_lane = 0;           // concurrent: chains that run in the lane form first
   bool solo = false;        // the solo form instead of the wave forms
   int nmax = 0;
   bool concurrent = false;  // batched passes only: split by Z, geometries side by side
@@ -792,6 +814,7 @@ int pass_setup(dsm_engine* e, const std::vector<int>& ids, bool use_ev_stop, Pas
   ps.concurrent = e->opt.concurrent >= 0 ? (e->opt.concurrent > 0 && bin_max >= 1)
                                          : (bin_max >= 3 || (bin_max >= 1 && z_est >= 56.0 * n_all));
   if (ps.lane_quads) ps.concurrent = false;
+  ps.n_lane = ps.concurrent && batched && e->d_rec_cap >= e->nstr ? lane_share(e, ids) : 0;
   if (n0 == 0) return DSM_OK;
   ps.range = batched && !ps.concurrent && ids.size() == 1;
   ps.first = e->ens[ids[0]].chain0;
@@ -825,6 +848,14 @@ hipError_t launch_wave(dsm_engine* e, const Pass& ps, const KmcArgs& a, int b, i
   return launch_kmc_solo(a, cap, std::min(ps.n0, kmc_solo_occupancy(cap) * e->n_cu), st);
 }
 
+// Lanes of a wave for n chains on one workgroup per CU: as many as give every wave the same
+// number of rounds.
+int lane_lanes(const dsm_engine* e, int quads, int n) {
+  const int most = lane_max_lanes(quads), waves = kLaneWaves * e->n_cu;
+  const int rounds = (n + waves * most - 1) / (waves * most);
+  return std::max(1, (n + waves * rounds - 1) / (waves * rounds));
+}
+
 // Batched pass with the geometries side by side: the chains are split by their current
 // Z into one list per geometry and every geometry runs at once, each on its own
 // stream, the largest first (its few long chains take their slots before the bulk fills
@@ -849,9 +880,21 @@ int pass_bins_concurrent(dsm_engine* e, Pass& ps, dsm_run_stats* rs) {
   auto late_of = [&](int b) { return kLateList + (b < kLateFirst ? kLateFirst : b + 1); };  // bin b's overflow
   const bool timed = !e->capturing;  // a captured pass is timed as a whole, around its replay
   if (timed) HIPCHK(hipEventRecord(e->cev[0], e->st));
-  HIPCHK(launch_fill_u32(cnt, 0u, 2 * kNumLists, e->st));
-  HIPCHK(launch_split_geoms(list(0), ps.n0, e->ch.Z, e->ch.stall, list(kSplitList), (int)cap, cnt + kSplitList,
-                            e->opt.split_margin_div, e->st));
+  constexpr int kEmpty = 2 * kNumLists + kZOrderScratch;  // a count that stays zero
+  HIPCHK(launch_fill_u32(cnt, 0u, kEmpty + 1, e->st));
+  if (ps.n_lane) HIPCHK(launch_fill_u32(list(kSplitList), 0xFFFFFFFFu, ps.n0, e->st));
+  HIPCHK(launch_split_geoms(list(0), ps.n0, e->ch, e->d_ens, list(kSplitList), (int)cap, cnt + kSplitList,
+                            e->opt.split_margin_div, ps.n_lane ? 4 * kLaneMaxQuads : 0, e->st));
+  if (ps.n_lane) {
+    // the short chains in the lane form, in decreasing Z (list 0, which has been split); its
+    // workgroups take whole CUs, so the other forms start behind it
+    HIPCHK(launch_z_order(list(kSplitList), 0, ps.n0, e->ch.Z, e->ch.stall, kLaneMaxQuads / 4, cnt + 2 * kNumLists,
+                          list(0), cnt, e->st));
+    bind(0, late_of(0));
+    a.lanes = lane_lanes(e, kLaneMaxQuads, ps.n_lane);
+    HIPCHK(launch_kmc_lane(a, kLaneMaxQuads, e->n_cu, e->st));
+    ++rs->kmc_launches;
+  }
   HIPCHK(hipEventRecord(e->ev_split, e->st));
   // first launches.  A process has four hardware queues on this device, so four streams.
   // The longest chains (G = 8: few chains, a latency-bound run that sets the window's
@@ -899,6 +942,7 @@ int pass_bins_concurrent(dsm_engine* e, Pass& ps, dsm_run_stats* rs) {
   bind(kSplitList + 1, late_of(1));
   const KmcArgs pair_args = a;
   bind(kSplitList, late_of(0));
+  if (ps.n_lane) a.n_work = cnt + kEmpty;
   int nb = kmc_rowpair_occupancy(a.lds_floats, a.ext != 0, wide);
   if (e->opt.blocks_per_cu > 0) nb = std::min(nb, e->opt.blocks_per_cu);
   if (timed) HIPCHK(hipEventRecord(e->cev[1], e->xs[2]));
@@ -934,7 +978,7 @@ int pass_bins_concurrent(dsm_engine* e, Pass& ps, dsm_run_stats* rs) {
 int pass_bins(dsm_engine* e, Pass& ps, bool plain, bool timed, dsm_run_stats* rs) {
   if (!plain && ps.concurrent) return pass_bins_concurrent(e, ps, rs);
   int* cnt = e->d_cnt;
-  HIPCHK(launch_init_counts(cnt, 2 * kNumLists + 17, ps.n0, e->st));  // lists, queues, order scratch
+  HIPCHK(launch_init_counts(cnt, 2 * kNumLists + kZOrderScratch, ps.n0, e->st));  // lists, queues, order scratch
   KmcArgs a = ps.a;
   int seq[kNumBins], ns = 0;
   seq[ns++] = 0;
@@ -971,10 +1015,7 @@ int pass_bins(dsm_engine* e, Pass& ps, bool plain, bool timed, dsm_run_stats* rs
     a.n_overflow = cnt + nb;
     if (timed) HIPCHK(hipEventRecord(e->lev[2 * k], e->st));
     if (k == 0 && lane) {
-      // one workgroup per CU; as many lanes as give every wave the same number of rounds
-      const int most = lane_max_lanes(ps.lane_quads), waves = kLaneWaves * e->n_cu;
-      const int rounds = (ps.n_live + waves * most - 1) / (waves * most);
-      a.lanes = std::max(1, (ps.n_live + waves * rounds - 1) / (waves * rounds));
+      a.lanes = lane_lanes(e, ps.lane_quads, ps.n_live);
       HIPCHK(launch_kmc_lane(a, ps.lane_quads, e->n_cu, e->st));
     } else if (!plain && b >= kLateFirst) {
       HIPCHK(launch_wave(e, ps, a, b, b, e->st));
@@ -1408,7 +1449,7 @@ int dsm_create(int32_t device_id, dsm_engine** out) {
   HIPCHK(hipEventCreateWithFlags(&e->ev_split, hipEventDisableTiming));
   for (auto& ev : e->ev_bin) HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
   int rc;
-  if ((rc = dev_alloc(&e->d_cnt, 2 * kNumLists + 32)) || (rc = dev_alloc(&e->d_counters, kNumCounters)) ||
+  if ((rc = dev_alloc(&e->d_cnt, 2 * kNumLists + kZOrderScratch + 1)) || (rc = dev_alloc(&e->d_counters, kNumCounters)) ||
       (rc = dev_alloc(&e->d_part, (size_t)kStressBlocks * 9))) {
     dsm_destroy(e);
     return rc;
@@ -1479,6 +1520,7 @@ int dsm_add_ensemble(dsm_engine* e, const dsm_ensemble_desc* d, int32_t* ens_id)
     E.nk[i] = nk;
     nmax = std::max(nmax, nk);
     E.z_sum_est += ((double)nk + d->beta) / (1.0 + d->beta);
+    E.n_lane += lane_room((float)nk, d->beta) < 4.0f * kLaneMaxQuads;
   }
   E.nmax = nmax;
   E.bin_max = bin_for(nmax);

@@ -163,34 +163,53 @@ __global__ void set_ev_stop_kernel(const uint64_t* ev, uint64_t* ev_stop, int ch
 // boundaries costs more in the first round than it saves in the late one).  Stalled
 // chains go to geometry 0, which skips them.  Lists are cap entries apart, counts[b]
 // their lengths.
-// One atomic per wave and geometry: the lanes of a geometry get consecutive slots.
+// One global atomic per block and geometry (one per wave took 197 us for 262,144 chains, all
+// on a line of L2): the waves of a geometry get consecutive slots of the block's.
 // margin_div > 0: a chain within capacity/margin_div of a wave-form geometry's capacity
 // starts in the next one (it would likely outgrow it during the pass)
-__global__ void split_geoms_kernel(const int* src, int n, const int* Z, const int* stall, int* lists, int cap,
-                                   int* counts, int margin_div) {
+// lane_cap > 0: list 0 takes the chains that will stay below that many positions (three
+// standard deviations above the equilibrium Z, eight above now) whatever their geometry, the
+// row form's others join list 1.
+__global__ void __launch_bounds__(1024) split_geoms_kernel(const int* src, int n, const ChainArrays ch, const EnsParams* ens, int* lists,
+                                   int cap, int* counts, int margin_div, int lane_cap) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const int c = i < n ? src[i] : -1;
   int b = -1;
   if (c >= 0) {
-    const int z = Z[c];
+    const int z = ch.Z[c];
     b = 0;
-    if (stall[c] == 0)
+    bool fits = false;
+    if (lane_cap > 0) {
+      const float nk = (float)ch.nk[c], beta = ens[ch.ens[c]].beta;
+      fits = z + 8 < lane_cap && lane_room(nk, beta) < (float)lane_cap;
+      b = fits ? 0 : 1;
+    }
+    if (ch.stall[c] == 0 && !fits)
       while (b + 1 < kNumGeoms &&
              z >= kmc_geom_capacity(b) - (b >= 2 && margin_div > 0 ? kmc_geom_capacity(b) / margin_div : 0))
         ++b;
   }
+  __shared__ int num[kNumGeoms], base[kNumGeoms];
+  if (threadIdx.x < kNumGeoms) num[threadIdx.x] = 0;
+  __syncthreads();
   const int lane = (int)__lane_id();
   const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  int at = 0;  // within the block's share of the list
 #pragma unroll
   for (int g = 0; g < kNumGeoms; ++g) {
     const uint64_t m = __ballot(b == g);
     if (m == 0) continue;
     const int leader = (int)__builtin_ctzll(m);
-    int base = 0;
-    if (lane == leader) base = atomicAdd(counts + g, __popcll(m));
-    base = __shfl(base, leader);
-    if (b == g) lists[(int64_t)g * cap + base + __popcll(m & below)] = c;
+    int o = 0;
+    if (lane == leader) o = atomicAdd(num + g, __popcll(m));
+    o = __shfl(o, leader) + __popcll(m & below);
+    at = b == g ? o : at;
   }
+  __syncthreads();
+  if (threadIdx.x < kNumGeoms && num[threadIdx.x] > 0)
+    base[threadIdx.x] = atomicAdd(counts + threadIdx.x, num[threadIdx.x]);
+  __syncthreads();
+  if (b >= 0) lists[(int64_t)b * cap + base[b] + at] = c;
 }
 
 // Work list in decreasing Z (16 buckets of `width` positions; Z >= 16 * width first,
@@ -200,7 +219,7 @@ __device__ __forceinline__ int zbucket(const int* Z, const int* stall, int width
   const int z = Z[c];
   return z >= 16 * width ? 0 : 15 - z / width;
 }
-constexpr int kZBuckets = 17;
+constexpr int kZBuckets = kZOrderScratch;
 
 // Block-local histograms in LDS, one global atomic per block and bucket (a per-element
 // global atomic on 17 counters serialises in L2).  Grid-stride over the elements.
@@ -898,11 +917,11 @@ hipError_t launch_sum_counters(const uint64_t* ev, const uint64_t* zsum, int cha
   return hipGetLastError();
 }
 
-hipError_t launch_split_geoms(const int* src, int n, const int* Z, const int* stall, int* lists, int cap,
-                              int* counts, int margin_div, hipStream_t st) {
+hipError_t launch_split_geoms(const int* src, int n, const ChainArrays& ch, const EnsParams* ens, int* lists, int cap,
+                              int* counts, int margin_div, int lane_cap, hipStream_t st) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(split_geoms_kernel, dim3((n + 255) / 256), dim3(256), 0, st, src, n, Z, stall, lists, cap,
-                     counts, margin_div);
+  hipLaunchKernelGGL(split_geoms_kernel, dim3((n + 1023) / 1024), dim3(1024), 0, st, src, n, ch, ens, lists, cap,
+                     counts, margin_div, lane_cap);
   return hipGetLastError();
 }
 
@@ -911,13 +930,13 @@ hipError_t launch_init_counts(int* cnt, int n, int n0, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t launch_z_order(const int* src, int first, int n, const int* Z, const int* stall, int width, int* scratch17,
+hipError_t launch_z_order(const int* src, int first, int n, const int* Z, const int* stall, int width, int* scratch,
                           int* dst, int* n_out, hipStream_t st) {
   if (n <= 0) return hipSuccess;
   const int blocks = n > 64 * 1024 * 4 ? 256 : (n + 4095) / 4096 + 1;  // a few elements per thread
-  hipLaunchKernelGGL(zhist_kernel, dim3(blocks), dim3(1024), 0, st, src, first, n, Z, stall, width, scratch17);
-  hipLaunchKernelGGL(zscan_kernel, dim3(1), dim3(64), 0, st, scratch17, n_out);
-  hipLaunchKernelGGL(zscatter_kernel, dim3(blocks), dim3(1024), 0, st, src, first, n, Z, stall, width, scratch17, dst);
+  hipLaunchKernelGGL(zhist_kernel, dim3(blocks), dim3(1024), 0, st, src, first, n, Z, stall, width, scratch);
+  hipLaunchKernelGGL(zscan_kernel, dim3(1), dim3(64), 0, st, scratch, n_out);
+  hipLaunchKernelGGL(zscatter_kernel, dim3(blocks), dim3(1024), 0, st, src, first, n, Z, stall, width, scratch, dst);
   return hipGetLastError();
 }
 

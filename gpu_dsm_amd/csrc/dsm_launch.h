@@ -1,5 +1,6 @@
 // dsm_launch.h -- host-callable launchers for the kernels in dsm_kernels.hip.
 #pragma once
+#include <cmath>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -47,12 +48,18 @@ constexpr int kLaneTabFloats = 4 * kLaneN + kLaneFR;
 constexpr int kLaneRecFloats = 3;  // working memory per strand slot
 constexpr int kLaneWaves = 8;
 constexpr int kLaneQuads[] = {8, 12, 16, 19, 24, 28, 32};
+constexpr int kLaneMaxQuads = 32;
 constexpr int kLaneLdsBytes = 160 * 1024;
 // most lanes of a wave whose columns (an odd number of them) fit the workgroup's LDS
 constexpr int lane_max_lanes(int quads) {
   const int s = ((int)(kLaneLdsBytes / sizeof(float)) - kLaneTabFloats) / (kLaneWaves * 4 * quads);
   const int odd = (s & 1) ? s : s - 1;
   return odd > 64 ? 64 : odd;
+}
+// positions a chain of nk Kuhn steps stays below in a window (three standard deviations above
+// its equilibrium Z, a binomial one)
+__host__ __device__ inline float lane_room(float nk, float beta) {
+  return (nk + beta) / (1.0f + beta) + 3.0f * sqrtf((nk - 1.0f) * beta) / (1.0f + beta);
 }
 hipError_t launch_kmc_lane(const KmcArgs& a, int quads, int grid, hipStream_t st);
 // The solo form (one chain per wave, `cap` positions in LDS, a multiple of 4): waves per CU,
@@ -65,13 +72,15 @@ hipError_t launch_init_eq(const ChainArrays& ch, const EnsParams* ens, const flo
 hipError_t launch_fill_u32(void* p, uint32_t v, int64_t n, hipStream_t st);
 hipError_t launch_iota(int* p, int start, int n, hipStream_t st);
 // the chains of src (entries < 0 skipped; src == null: chains first .. first+n-1) into
-// dst in decreasing Z (buckets of `width` positions, the first from 16 * width on); *n_out = their count.  scratch17 (17 ints) must be zero.
-hipError_t launch_z_order(const int* src, int first, int n, const int* Z, const int* stall, int width, int* scratch17,
+// dst in decreasing Z (buckets of `width` positions, the first from 16 * width on); *n_out = their count.  scratch (kZOrderScratch
+// ints) must be zero.
+constexpr int kZOrderScratch = 17;
+hipError_t launch_z_order(const int* src, int first, int n, const int* Z, const int* stall, int width, int* scratch,
                           int* dst, int* n_out, hipStream_t st);
 // cnt[0] = n0, cnt[1..n) = 0
 hipError_t launch_init_counts(int* cnt, int n, int n0, hipStream_t st);
-hipError_t launch_split_geoms(const int* src, int n, const int* Z, const int* stall, int* lists, int cap,
-                              int* counts, int margin_div, hipStream_t st);
+hipError_t launch_split_geoms(const int* src, int n, const ChainArrays& ch, const EnsParams* ens, int* lists, int cap,
+                              int* counts, int margin_div, int lane_cap, hipStream_t st);
 // out[0] += sum ev[chain0..chain0+n), out[1] += sum zsum[...]
 hipError_t launch_sum_counters(const uint64_t* ev, const uint64_t* zsum, int chain0, int n, unsigned long long* out,
                                hipStream_t st);
