@@ -981,9 +981,6 @@ int pass_bins(dsm_engine* e, Pass& ps, bool plain, bool timed, dsm_run_stats* rs
   HIPCHK(launch_init_counts(cnt, 2 * kNumLists + kZOrderScratch, ps.n0, e->st));  // lists, queues, order scratch
   KmcArgs a = ps.a;
   int seq[kNumBins], ns = 0;
-  seq[ns++] = 0;
-  if (ps.bin_max >= 1)
-    for (int b = kLateFirst; b <= late_last(ps.bin_max); ++b) seq[ns++] = b;
   // batched, one ensemble: the row form takes its chains in decreasing Z, so the chains
   // started last, which set the end of the launch, are the shortest (several ensembles
   // keep their order: a wave runs one ensemble at a time)
@@ -994,6 +991,9 @@ int pass_bins(dsm_engine* e, Pass& ps, bool plain, bool timed, dsm_run_stats* rs
   const bool small = !plain && ps.n_live <= e->opt.small_per_cu * e->n_cu;
   const bool lane = !plain && ps.lane_quads > 0 && !small;
   const bool zorder = !plain && (ps.n_ens == 1 || small || lane);
+  seq[ns++] = 0;
+  if (ps.bin_max >= 1 || lane)  // (a lane's columns may be lower than the longest chain)
+    for (int b = kLateFirst; b <= late_last(ps.bin_max); ++b) seq[ns++] = b;
   constexpr int kZList = kNumLists - 1;
   if (zorder)
     HIPCHK(launch_z_order(ps.range ? nullptr : e->d_work, ps.first, ps.range ? ps.n_live : ps.n0, e->ch.Z,

@@ -522,9 +522,10 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(MULTI ?
   S.ns = (lds_i*)(S.w + S.cap);
   S.g = 0; S.X = 0.0f; S.cb = 0.0f; S.P = 0.0f; S.tot = 0.0f; S.nb = 1;
   for (auto& v : S.s) v = 0.0f;
+  const int n_work = *a.n_work;
+  if ((int)blockIdx.x >= n_work) return;  // more waves than chains: nothing is left for it
   for (int i = S.C.lane; i < kLaneTabFloats; i += 64) S.C.tab[i] = a.lane_tab[i];
   wave_lds_sync();
-  const int n_work = *a.n_work;
   const double kNever = __longlong_as_double(0x7ff0000000000000ll);
   LaneChain H;
   for (;;) {
