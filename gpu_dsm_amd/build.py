@@ -25,7 +25,7 @@ COMMON = [
     "-I", os.path.join(ROOT, "include"), "-I", CSRC,
 ]
 DEVICE = ["--offload-arch=" + ARCH, "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
-SOURCES = ["dsm_kernels.hip", "dsm_engine.cpp", "dsm_driver.cpp", "dsm_serve.cpp", "dsm_noalloc.hip", "dsm_lane_inst.hip", "dsm_solo_inst.hip"]
+SOURCES = ["dsm_kernels.hip", "dsm_engine.cpp", "dsm_driver.cpp", "dsm_serve.cpp", "dsm_noalloc.hip", "dsm_lane_inst.hip", "dsm_lane_flow_inst.hip", "dsm_solo_inst.hip"]
 GEOMS = [0, 1, 2, 3, 4, 5, 6, 7]  # KMC chain geometries (one translation unit each; 6 = bins 0 and 1 merged:
                                   # the row form, then the row form with two register groups or the
                                   # pair form; 7 = pair form with two register groups)

@@ -583,6 +583,13 @@ int ensure_stage(dsm_engine* e) {
 // rate of a chain at every jump.
 bool lane_capable(const Ens& E) { return !E.P.flow && E.P.sample_mode != kSampleFlow; }
 
+// Positions that a chain of an ensemble stays below: the equilibrium Z (binomial) and five
+// standard deviations.
+double equilibrium_room(const Ens& E) {
+  const double b = E.P.beta, nk = E.nmax;
+  return std::min(nk, (nk + b) / (1.0 + b) + 5.0 * std::sqrt((nk - 1.0) * b) / (1.0 + b));
+}
+
 // Quads per chain with which a batched pass over these ensembles runs in the lane form, or
 // 0 when it runs in the others.  The chains have to fit the largest size, 128 positions,
 // with five standard deviations of the equilibrium Z (binomial) to spare (one that outgrows
@@ -593,9 +600,8 @@ int lane_quads(const dsm_engine* e, const std::vector<int>& ids) {
   for (int id : ids) {
     const Ens& E = e->ens[id];
     if (!lane_capable(E)) return 0;
-    const double b = E.P.beta, nk = E.nmax;
     n += E.n;
-    zcap = std::max(zcap, std::min(nk, (nk + b) / (1.0 + b) + 5.0 * std::sqrt((nk - 1.0) * b) / (1.0 + b)));
+    zcap = std::max(zcap, equilibrium_room(E));
   }
   int quads = 0;
   for (int q : kLaneQuads)
@@ -607,6 +613,32 @@ int lane_quads(const dsm_engine* e, const std::vector<int>& ids) {
   // (Nk 150: 4.38 against 4.90 ms at 16,000).
   if (e->opt.lane == 1 && n < (quads >= 24 ? 14000 : 36000)) return 0;
   return quads;
+}
+
+// Positions a chain with which a pass of flow ensembles runs in the lane form under flow
+// (dsm_lane_flow.h), or 0: to 40, at 2.75 standard deviations above the equilibrium Z (more
+// room costs lanes: at Nk 50 five per cent of the time each position; a chain that outgrows
+// it finishes in the wave form).  A lane's step costs its wave the same for one chain as for
+// 64, so the form needs chains, the more the longer they are, and more where the row form is
+// at its best, with one ensemble whose chains it takes in decreasing Z: there, 8 tau_K, 65,536
+// chains of Nk 12 0.82 against 1.45 ms (16,384: 0.68 / 0.50), of Nk 25 1.39 / 2.01 (16,384: 1.00 /
+// 0.70), of Nk 35 1.89 / 2.42, of Nk 50 262,144 9.6 / 10.6 and 131,072 6.0 / 5.4.  Of 16
+// ensembles, 16,384 of Nk 25 1.06 / 1.24, 32,768 of Nk 50 2.66 / 3.22, 262,144 of Nk 50 9.6 / 11.8.
+int flow_cap(const dsm_engine* e, const std::vector<int>& ids) {
+  if (e->opt.lane == 0 || ids.empty()) return 0;
+  double n = 0.0, zcap = 0.0;
+  for (int id : ids) {
+    const Ens& E = e->ens[id];
+    if (!E.P.flow || (E.P.sample_mode != kSampleNone && E.P.sample_mode != kSampleFlow)) return 0;
+    n += E.n;
+    zcap = std::max(zcap, std::min((double)E.nmax, (double)lane_room((float)E.nmax, E.P.beta, 2.75f)));
+  }
+  int cap = 0;
+  for (int p : kFlowCaps)
+    if (p > zcap) { cap = p; break; }
+  const double least = ids.size() > 1 ? std::max(16000, 800 * cap)
+                                      : std::max(28000, (cap > 32 ? 5000 : 1500) * cap);
+  return e->opt.lane == 2 || n >= least ? cap : 0;
 }
 
 // Chains of a pass of mixed lengths that run in the lane form before the longer ones start
@@ -652,14 +684,14 @@ void release_lane(dsm_engine* e) {
 }
 int ensure_lane(dsm_engine* e, const std::vector<int>& ids) {
   const bool lanes = lane_quads(e, ids) || lane_share(e, ids);
-  if (!lanes && !solo_capable(e, ids)) return DSM_OK;
+  if (!lanes && !solo_capable(e, ids) && !flow_cap(e, ids)) return DSM_OK;
   if (!e->d_lane_tab) {
     std::vector<float> t, out((size_t)kLaneTabFloats, 0.0f);
     build_tables(t, kLaneN, 1.0f, 0, 0.0f);
     const int n = kLaneN + 2;
     for (int N = 1; N < kLaneN; ++N)
       for (int q = 0; q < 4; ++q) out[4 * N + q] = t[(size_t)q * n + N];
-    for (int x = 1; x < kLaneFR; ++x) out[4 * kLaneN + x] = t[(size_t)kNumTables * n + x];
+    for (int x = 1; x < kLaneFR; ++x) out[4 * kLaneN + x] = 4.0f / (float)x;  // (build_tables' FR)
     int rc = dev_alloc(&e->d_lane_tab, out.size());
     if (rc) return rc;
     HIPCHK(hipMemcpy(e->d_lane_tab, out.data(), sizeof(float) * out.size(), hipMemcpyHostToDevice));
@@ -774,6 +806,7 @@ struct Pass {
   int n0 = 0;  // entries of the bin-0 list
   int bin_max = 0;
   int lane_quads = 0;       // > 0: the lane form with this many quads per chain
+  int flow_cap = 0;         // > 0: the lane form under flow with this many positions a chain
   int n_lane = 0;           // concurrent: chains that run in the lane form first
   bool solo = false;        // the solo form instead of the wave forms
   int nmax = 0;
@@ -813,7 +846,8 @@ int pass_setup(dsm_engine* e, const std::vector<int>& ids, bool use_ev_stop, Pas
   // 63 positions (the pair form then carries the bulk)
   ps.concurrent = e->opt.concurrent >= 0 ? (e->opt.concurrent > 0 && bin_max >= 1)
                                          : (bin_max >= 3 || (bin_max >= 1 && z_est >= 56.0 * n_all));
-  if (ps.lane_quads) ps.concurrent = false;
+  ps.flow_cap = batched && e->d_lane_tab ? flow_cap(e, ids) : 0;
+  if (ps.lane_quads || ps.flow_cap) ps.concurrent = false;
   ps.n_lane = ps.concurrent && batched && e->d_rec_cap >= e->nstr ? lane_share(e, ids) : 0;
   if (n0 == 0) return DSM_OK;
   ps.range = batched && !ps.concurrent && ids.size() == 1;
@@ -848,12 +882,14 @@ hipError_t launch_wave(dsm_engine* e, const Pass& ps, const KmcArgs& a, int b, i
   return launch_kmc_solo(a, cap, std::min(ps.n0, kmc_solo_occupancy(cap) * e->n_cu), st);
 }
 
-// Lanes of a wave for n chains on one workgroup per CU: as many as give every wave the same
-// number of rounds.
-int lane_lanes(const dsm_engine* e, int quads, int n) {
-  const int most = lane_max_lanes(quads), waves = kLaneWaves * e->n_cu;
+// Lanes of each of `waves` waves for n chains: as many, to `most`, as give every wave the
+// same number of rounds.
+int even_lanes(int n, int most, int waves) {
   const int rounds = (n + waves * most - 1) / (waves * most);
   return std::max(1, (n + waves * rounds - 1) / (waves * rounds));
+}
+int lane_lanes(const dsm_engine* e, int quads, int n) {
+  return even_lanes(n, lane_max_lanes(quads), kLaneWaves * e->n_cu);
 }
 
 // Batched pass with the geometries side by side: the chains are split by their current
@@ -989,7 +1025,8 @@ int pass_bins(dsm_engine* e, Pass& ps, bool plain, bool timed, dsm_run_stats* rs
   // (1.79 us per jump against 2.84 us per row-form step of four chains).  Measured:
   // 1000 chains of Nk 25 +15%, of Nk 100 +92%; 4096 chains of Nk 25 -14%.
   const bool small = !plain && ps.n_live <= e->opt.small_per_cu * e->n_cu;
-  const bool lane = !plain && ps.lane_quads > 0 && !small;
+  const bool flow = !plain && ps.flow_cap > 0 && !small;
+  const bool lane = flow || (!plain && ps.lane_quads > 0 && !small);
   const bool zorder = !plain && (ps.n_ens == 1 || small || lane);
   seq[ns++] = 0;
   if (ps.bin_max >= 1 || lane)  // (a lane's columns may be lower than the longest chain)
@@ -997,14 +1034,14 @@ int pass_bins(dsm_engine* e, Pass& ps, bool plain, bool timed, dsm_run_stats* rs
   constexpr int kZList = kNumLists - 1;
   if (zorder)
     HIPCHK(launch_z_order(ps.range ? nullptr : e->d_work, ps.first, ps.range ? ps.n_live : ps.n0, e->ch.Z,
-                          e->ch.stall, lane ? (ps.lane_quads + 3) / 4 : 4, cnt + 2 * kNumLists, e->d_work + (size_t)kZList * e->d_work_cap,
+                          e->ch.stall, flow ? (ps.flow_cap + 15) / 16 : lane ? (ps.lane_quads + 3) / 4 : 4, cnt + 2 * kNumLists, e->d_work + (size_t)kZList * e->d_work_cap,
                           cnt + kZList, e->st));
   if (small) {  // the compact ordered list feeds the wave form directly
     ns = 0;
     for (int b = kLateFirst; b <= late_last(ps.bin_max); ++b) seq[ns++] = b;
   }
   // lane form first, then the wave form for chains that outgrew it, if their length allows
-  if (lane && ps.nmax < 4 * ps.lane_quads) ns = 1;
+  if (lane && ps.nmax < (flow ? ps.flow_cap : 4 * ps.lane_quads)) ns = 1;
   for (int k = 0; k < ns; ++k) {
     const int b = seq[k], nb = k + 1 < ns ? seq[k + 1] : b + 1;
     const int in = (k == 0 && zorder) ? kZList : b;
@@ -1014,7 +1051,10 @@ int pass_bins(dsm_engine* e, Pass& ps, bool plain, bool timed, dsm_run_stats* rs
     a.overflow = e->d_work + (size_t)nb * e->d_work_cap;
     a.n_overflow = cnt + nb;
     if (timed) HIPCHK(hipEventRecord(e->lev[2 * k], e->st));
-    if (k == 0 && lane) {
+    if (k == 0 && flow) {
+      a.lanes = even_lanes(ps.n_live, flow_max_lanes(ps.flow_cap), kFlowWaves * e->n_cu);
+      HIPCHK(launch_kmc_lane_flow(a, ps.flow_cap, e->n_cu, e->st));
+    } else if (k == 0 && lane) {
       a.lanes = lane_lanes(e, ps.lane_quads, ps.n_live);
       HIPCHK(launch_kmc_lane(a, ps.lane_quads, e->n_cu, e->st));
     } else if (!plain && b >= kLateFirst) {

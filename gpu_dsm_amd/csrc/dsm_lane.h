@@ -140,10 +140,10 @@ struct LaneCtx {
   int S;
   int lane, row, rl;
   __device__ __forceinline__ LaneTab pt(int N) const {
-    const vf4 v = *(lds_f4*)(tab + 4 * min(N, kLaneN - 1));
+    const vf4 v = *(lds_f4*)(tab + 4 * N);
     return LaneTab{v.x, v.y, v.z, v.w};
   }
-  __device__ __forceinline__ float fr(int x) const { return tab[4 * kLaneN + min(x, kLaneFR - 1)]; }
+  __device__ __forceinline__ float fr(int x) const { return tab[4 * kLaneN + x]; }
   // rate of position p of lane column c
   __device__ __forceinline__ lds_f* rp(int p, int c) const { return (lds_f*)(rq + ((p >> 2) * S + c)) + (p & 3); }
 };
@@ -158,8 +158,9 @@ struct LaneStrand {
   int xp, xm;
 };
 __device__ __forceinline__ LaneStrand lane_strand(const LaneCtx& X, int N, float q2, bool end) {
-  const LaneTab t = X.pt(N);
-  const int x = end ? 4 * N : 2 * N, d = end ? 1 : 0;
+  const int n = min(N, kLaneN - 1);  // (longer ones take the general form)
+  const LaneTab t = X.pt(n);
+  const int x = end ? 4 * n : 2 * n, d = end ? 1 : 0;
   const float one = N > 1 ? 1.0f : 0.0f;
   return LaneStrand{q2 * t.sp, q2 * t.sm, end ? 1.0f : t.pp, end ? one : t.pm, x + d, x - d};
 }
@@ -169,7 +170,8 @@ __device__ __forceinline__ bool lane_pair(const LaneCtx& X, const LaneStrand& i,
   const float ep = i.a - j.b, em = j.a - i.b;
   wp = ((X.fr(i.xp + j.xm) * i.pp) * j.pm) * lane_exp(ep);
   wm = ((X.fr(i.xm + j.xp) * i.pm) * j.pp) * lane_exp(em);
-  return !(__builtin_fabsf(ep) <= 87.0f) || !(__builtin_fabsf(em) <= 87.0f);
+  // (a NaN |Q|^2 makes both NaN, an infinite one at least one infinite or both NaN)
+  return !(fmaxf(__builtin_fabsf(ep), __builtin_fabsf(em)) <= 87.0f);
 }
 __device__ __forceinline__ float lane_total(int cd, float cc, int Ni, float wp, float wm, float we) {
   return cd ? (wp + wm) + (we + cc * (float)(Ni - 1)) : (wp + wm);

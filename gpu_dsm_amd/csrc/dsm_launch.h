@@ -43,7 +43,7 @@ hipError_t launch_kmc_rowpair(const KmcArgs& row, const KmcArgs& pair, bool row2
 int kmc_rowpair_occupancy(int lds_floats, bool ext, bool row2);
 // The lane form (one chain per lane, quads * 4 positions): persistent workgroups of
 // kLaneWaves waves that share the tables {SP, SM, PP, PM}[kLaneN], FR[kLaneFR].
-constexpr int kLaneN = 64, kLaneFR = 256;
+constexpr int kLaneN = 64, kLaneFR = 512;  // (FR: two strands of 63, four times each)
 constexpr int kLaneTabFloats = 4 * kLaneN + kLaneFR;
 constexpr int kLaneRecFloats = 3;  // working memory per strand slot
 constexpr int kLaneWaves = 8;
@@ -56,12 +56,25 @@ constexpr int lane_max_lanes(int quads) {
   const int odd = (s & 1) ? s : s - 1;
   return odd > 64 ? 64 : odd;
 }
-// positions a chain of nk Kuhn steps stays below in a window (three standard deviations above
-// its equilibrium Z, a binomial one)
-__host__ __device__ inline float lane_room(float nk, float beta) {
-  return (nk + beta) / (1.0f + beta) + 3.0f * sqrtf((nk - 1.0f) * beta) / (1.0f + beta);
+// positions a chain of nk Kuhn steps hardly ever exceeds in a window (`sd` standard deviations
+// above its equilibrium Z, a binomial one)
+__host__ __device__ inline float lane_room(float nk, float beta, float sd = 3.0f) {
+  return (nk + beta) / (1.0f + beta) + sd * sqrtf((nk - 1.0f) * beta) / (1.0f + beta);
 }
 hipError_t launch_kmc_lane(const KmcArgs& a, int quads, int grid, hipStream_t st);
+// The lane form under flow: `cap` positions a chain, kFlowWaves waves a workgroup.
+constexpr int kFlowWaves = 8;
+constexpr int kFlowCaps[] = {8, 12, 16, 20, 24, 28, 32, 36, 40};
+// floats of a wave's columns: {Q, w} and the length of `cap` positions, S lanes
+__host__ __device__ constexpr int flow_wave_floats(int cap, int S) {
+  return ((4 * cap + cap / 2) * S + 3) & ~3;
+}
+constexpr int flow_max_lanes(int cap) {
+  int s = 65;
+  while (s > 1 && flow_wave_floats(cap, s) > ((int)(kLaneLdsBytes / sizeof(float)) - kLaneTabFloats) / kFlowWaves) s -= 2;
+  return s > 64 ? 64 : s;
+}
+hipError_t launch_kmc_lane_flow(const KmcArgs& a, int cap, int grid, hipStream_t st);
 // The solo form (one chain per wave, `cap` positions in LDS, a multiple of 4): waves per CU,
 // and a launch of `grid` waves.
 int kmc_solo_occupancy(int cap);
