@@ -48,6 +48,11 @@ constexpr int kNumLists = 2 * kNumBins + 1;
 constexpr int kSplitList = 1, kLateList = kNumBins;
 constexpr int kMaxNk = 2047;         // Z <= Nk must fit the largest geometry after a creation
 constexpr int kDefaultWindow = 256;
+// Chains up to which one block does a pass's bookkeeping (totals, order) in a launch each
+// instead of two and four: such a pass's time is its launches (64 chains of Nk 16, one tau_K
+// and the G(t) read: 151 -> 138 us; 1000 of Nk 25, 64 tau_K: 1044 -> 1001).  The block's two
+// turns of 1024 chains at a time cost a launch's gap at about this many.
+constexpr int kOneBlock = 8192;
 constexpr int kTotalsSlot = 4;       // d_counters: [0..3] advance_impl, [4..5] chain_totals
 constexpr int kNumCounters = 6;
 constexpr int kLdsTableFloats = 2816;  // per-wave LDS budget for rate tables (Nk <= ~200)
@@ -1014,7 +1019,7 @@ int pass_bins_concurrent(dsm_engine* e, Pass& ps, dsm_run_stats* rs) {
 int pass_bins(dsm_engine* e, Pass& ps, bool plain, bool timed, dsm_run_stats* rs) {
   if (!plain && ps.concurrent) return pass_bins_concurrent(e, ps, rs);
   int* cnt = e->d_cnt;
-  HIPCHK(launch_init_counts(cnt, 2 * kNumLists + kZOrderScratch, ps.n0, e->st));  // lists, queues, order scratch
+  constexpr int kCounts = 2 * kNumLists + kZOrderScratch;  // lists, queues, order scratch
   KmcArgs a = ps.a;
   int seq[kNumBins], ns = 0;
   // batched, one ensemble: the row form takes its chains in decreasing Z, so the chains
@@ -1032,10 +1037,20 @@ int pass_bins(dsm_engine* e, Pass& ps, bool plain, bool timed, dsm_run_stats* rs
   if (ps.bin_max >= 1 || lane)  // (a lane's columns may be lower than the longest chain)
     for (int b = kLateFirst; b <= late_last(ps.bin_max); ++b) seq[ns++] = b;
   constexpr int kZList = kNumLists - 1;
-  if (zorder)
-    HIPCHK(launch_z_order(ps.range ? nullptr : e->d_work, ps.first, ps.range ? ps.n_live : ps.n0, e->ch.Z,
-                          e->ch.stall, flow ? (ps.flow_cap + 15) / 16 : lane ? (ps.lane_quads + 3) / 4 : 4, cnt + 2 * kNumLists, e->d_work + (size_t)kZList * e->d_work_cap,
-                          cnt + kZList, e->st));
+  const int width = flow ? (ps.flow_cap + 15) / 16 : lane ? (ps.lane_quads + 3) / 4 : 4;
+  int* const zlist = e->d_work + (size_t)kZList * e->d_work_cap;
+  const int* const zsrc = ps.range ? nullptr : e->d_work;
+  const int nz = ps.range ? ps.n_live : ps.n0;
+  // up to kOneBlock chains the counts and the order take one launch for four
+  if (zorder && nz > 0 && nz <= kOneBlock) {
+    HIPCHK(launch_z_order_block(zsrc, ps.first, nz, e->ch.Z, e->ch.stall, width, cnt, kCounts, ps.n0, zlist,
+                                cnt + kZList, e->st));
+  } else {
+    HIPCHK(launch_init_counts(cnt, kCounts, ps.n0, e->st));
+    if (zorder)
+      HIPCHK(launch_z_order(zsrc, ps.first, nz, e->ch.Z, e->ch.stall, width, cnt + 2 * kNumLists, zlist, cnt + kZList,
+                            e->st));
+  }
   if (small) {  // the compact ordered list feeds the wave form directly
     ns = 0;
     for (int b = kLateFirst; b <= late_last(ps.bin_max); ++b) seq[ns++] = b;
@@ -1256,9 +1271,14 @@ int advance_impl(dsm_engine* e, const std::vector<int>& ids, const std::vector<d
   // synchronisation, so the totals cost no host round trip of their own
   unsigned long long tot[4] = {0, 0, 0, 0};
   bool have_tot = false;
-  HIPCHK(launch_fill_u32(e->d_counters, 0u, 8, e->st));
-  for (int id : ids)
-    HIPCHK(launch_sum_counters(e->ch.ev, e->ch.zsum, e->ens[id].chain0, e->ens[id].n, e->d_counters, e->st));
+  if (ids.size() == 1 && e->ens[ids[0]].n <= kOneBlock) {
+    const Ens& E = e->ens[ids[0]];
+    HIPCHK(launch_set_counters(e->ch.ev, e->ch.zsum, E.chain0, E.n, e->d_counters, 4, e->st));
+  } else {
+    HIPCHK(launch_fill_u32(e->d_counters, 0u, 8, e->st));
+    for (int id : ids)
+      HIPCHK(launch_sum_counters(e->ch.ev, e->ch.zsum, e->ens[id].chain0, e->ens[id].n, e->d_counters, e->st));
+  }
   auto aborted = [&]() {
     unsigned long long before[2] = {0, 0};
     if (hipMemcpy(before, e->d_counters, sizeof(before), hipMemcpyDeviceToHost) == hipSuccess)

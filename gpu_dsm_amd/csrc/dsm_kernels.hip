@@ -132,8 +132,10 @@ __global__ void fill_u32_kernel(uint32_t* p, uint32_t v, int64_t n) {
 }
 
 // one block: out[0] += sum of ev, out[1] += sum of zsum over a chain range
+// SET: one block, out[0..1] the sums, out[2..n_zero) zero; otherwise added to out[0..1].
+template <bool SET>
 __global__ void __launch_bounds__(1024) sum_counters_kernel(const uint64_t* ev, const uint64_t* zsum, int chain0,
-                                                             int n, unsigned long long* out) {
+                                                             int n, unsigned long long* out, int n_zero) {
   __shared__ unsigned long long r0[1024], r1[1024];
   unsigned long long a0 = 0, a1 = 0;
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
@@ -147,7 +149,11 @@ __global__ void __launch_bounds__(1024) sum_counters_kernel(const uint64_t* ev, 
     if ((int)threadIdx.x < h) { r0[threadIdx.x] += r0[threadIdx.x + h]; r1[threadIdx.x] += r1[threadIdx.x + h]; }
     __syncthreads();
   }
-  if (threadIdx.x == 0) { atomicAdd(out, r0[0]); atomicAdd(out + 1, r1[0]); }
+  if constexpr (SET) {
+    if (threadIdx.x < (unsigned)n_zero) out[threadIdx.x] = threadIdx.x == 0 ? r0[0] : (threadIdx.x == 1 ? r1[0] : 0ull);
+  } else {
+    if (threadIdx.x == 0) { atomicAdd(out, r0[0]); atomicAdd(out + 1, r1[0]); }
+  }
 }
 
 __global__ void set_ev_stop_kernel(const uint64_t* ev, uint64_t* ev_stop, int chain0, int n, uint64_t add) {
@@ -268,6 +274,33 @@ __global__ void __launch_bounds__(1024) zscatter_kernel(const int* src, int firs
       const int b = zbucket(Z, stall, width, c);
       dst[base[b] + atomicAdd(lh + b, 1)] = c;
     }
+  }
+}
+
+// The whole of it, and the counts of a sequential pass (init_counts_kernel), in one block:
+// short lists, where a pass's time is its launches.
+__global__ void __launch_bounds__(1024) zorder_block_kernel(const int* src, int first, int n, const int* Z,
+                                                            const int* stall, int width, int* cnt, int n_cnt, int n0,
+                                                            int* dst, int* n_out) {
+  __shared__ int lh[kZBuckets], at[kZBuckets];
+  for (int i = threadIdx.x; i < n_cnt; i += 1024) cnt[i] = i == 0 ? n0 : 0;
+  if (threadIdx.x < kZBuckets) lh[threadIdx.x] = 0;
+  __syncthreads();
+  for (int i = threadIdx.x; i < n; i += 1024) {
+    const int c = src ? src[i] : first + i;
+    if (c >= 0) atomicAdd(lh + zbucket(Z, stall, width, c), 1);
+  }
+  __syncthreads();
+  if (threadIdx.x < kZBuckets) {
+    int before = 0;
+    for (int b = 0; b < (int)threadIdx.x; ++b) before += lh[b];
+    at[threadIdx.x] = before;
+    if (threadIdx.x == kZBuckets - 1) *n_out = before + lh[kZBuckets - 1];  // (behind the counts' zeros)
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < n; i += 1024) {
+    const int c = src ? src[i] : first + i;
+    if (c >= 0) dst[atomicAdd(at + zbucket(Z, stall, width, c), 1)] = c;
   }
 }
 
@@ -913,7 +946,12 @@ hipError_t launch_sum_counters(const uint64_t* ev, const uint64_t* zsum, int cha
                                hipStream_t st) {
   if (n <= 0) return hipSuccess;
   const int grid = n > 256 * 4096 ? 256 : (n + 4095) / 4096;  // integer sums: the order does not matter
-  hipLaunchKernelGGL(sum_counters_kernel, dim3(grid), dim3(1024), 0, st, ev, zsum, chain0, n, out);
+  hipLaunchKernelGGL((sum_counters_kernel<false>), dim3(grid), dim3(1024), 0, st, ev, zsum, chain0, n, out, 0);
+  return hipGetLastError();
+}
+hipError_t launch_set_counters(const uint64_t* ev, const uint64_t* zsum, int chain0, int n, unsigned long long* out,
+                               int n_zero, hipStream_t st) {
+  hipLaunchKernelGGL((sum_counters_kernel<true>), dim3(1), dim3(1024), 0, st, ev, zsum, chain0, n, out, n_zero);
   return hipGetLastError();
 }
 
@@ -927,6 +965,13 @@ hipError_t launch_split_geoms(const int* src, int n, const ChainArrays& ch, cons
 
 hipError_t launch_init_counts(int* cnt, int n, int n0, hipStream_t st) {
   hipLaunchKernelGGL(init_counts_kernel, dim3((n + 255) / 256), dim3(256), 0, st, cnt, n, n0);
+  return hipGetLastError();
+}
+
+hipError_t launch_z_order_block(const int* src, int first, int n, const int* Z, const int* stall, int width, int* cnt,
+                                int n_cnt, int n0, int* dst, int* n_out, hipStream_t st) {
+  hipLaunchKernelGGL(zorder_block_kernel, dim3(1), dim3(1024), 0, st, src, first, n, Z, stall, width, cnt, n_cnt, n0,
+                     dst, n_out);
   return hipGetLastError();
 }
 

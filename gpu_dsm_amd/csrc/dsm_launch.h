@@ -90,6 +90,9 @@ hipError_t launch_iota(int* p, int start, int n, hipStream_t st);
 constexpr int kZOrderScratch = 17;
 hipError_t launch_z_order(const int* src, int first, int n, const int* Z, const int* stall, int width, int* scratch,
                           int* dst, int* n_out, hipStream_t st);
+// the same with launch_init_counts(cnt, n_cnt, n0) before it, in one block (n_out within cnt)
+hipError_t launch_z_order_block(const int* src, int first, int n, const int* Z, const int* stall, int width, int* cnt,
+                                int n_cnt, int n0, int* dst, int* n_out, hipStream_t st);
 // cnt[0] = n0, cnt[1..n) = 0
 hipError_t launch_init_counts(int* cnt, int n, int n0, hipStream_t st);
 hipError_t launch_split_geoms(const int* src, int n, const ChainArrays& ch, const EnsParams* ens, int* lists, int cap,
@@ -97,6 +100,9 @@ hipError_t launch_split_geoms(const int* src, int n, const ChainArrays& ch, cons
 // out[0] += sum ev[chain0..chain0+n), out[1] += sum zsum[...]
 hipError_t launch_sum_counters(const uint64_t* ev, const uint64_t* zsum, int chain0, int n, unsigned long long* out,
                                hipStream_t st);
+// out[0..1] = the sums, out[2..n_zero) = 0, in one block
+hipError_t launch_set_counters(const uint64_t* ev, const uint64_t* zsum, int chain0, int n, unsigned long long* out,
+                               int n_zero, hipStream_t st);
 hipError_t launch_set_ev_stop(const uint64_t* ev, uint64_t* ev_stop, int chain0, int n, uint64_t add,
                               hipStream_t st);
 // out[row][9]; part: nrows * flow_reduce_parts(nch) * 9 doubles
