@@ -1158,22 +1158,17 @@ int finish_stats(dsm_engine* e, const std::vector<int>& ids, const unsigned long
 }
 
 // The device work of one window after its parameters are set: staging fills, the KMC
-// pass and the sample consumers (correlator update, flow-row reduction).  Parameters come
-// from the host (eager: uploaded) or, in a captured pass, from the pinned block h_win
-// through stage_window_kernel at the head of the graph.
+// pass and the sample consumers (correlator update, flow-row reduction).  The window's
+// parameters come from the pinned block h_win (window_block) through stage_window_kernel:
+// all others have been on the device since the ensemble was added.  (Uploading them from
+// pageable memory took two copies and a host wait before the pass.)
 int window_launches(dsm_engine* e, const std::vector<int>& act, const std::vector<int64_t>& cnt_off,
                     const std::vector<int64_t>& row_off, const std::vector<int>& cnt, int mode, dsm_run_stats* rs,
                     Pass* timed) {
   int rc;
-  if (e->capturing) {
-    const WinParam* wp = (const WinParam*)e->h_win;
-    HIPCHK(launch_stage_window(wp, (int)act.size(), e->d_ens, (const int*)(wp + act.size()), e->d_corr_cnt,
-                               (int)cnt.size(), e->st));
-  } else {
-    if ((rc = upload_ens(e))) return rc;
-    if (!cnt.empty())
-      HIPCHK(hipMemcpyAsync(e->d_corr_cnt, cnt.data(), sizeof(int) * cnt.size(), hipMemcpyHostToDevice, e->st));
-  }
+  const WinParam* wp = (const WinParam*)e->h_win;
+  HIPCHK(launch_stage_window(wp, (int)act.size(), e->d_ens, (const int*)(wp + act.size()), e->d_corr_cnt,
+                             (int)cnt.size(), e->st));
   for (int id : act) {
     Ens& E = e->ens[id];
     if (E.P.k_end > E.P.k0)
@@ -1190,6 +1185,33 @@ int window_launches(dsm_engine* e, const std::vector<int>& act, const std::vecto
     else
       HIPCHK(launch_flow_reduce(e->d_stage + E.P.stage_off, E.n, rows, e->d_row_part, e->d_rows + row_off[q], e->st));
   }
+  return DSM_OK;
+}
+
+// The pinned block of a window's parameters, at least `need` bytes.
+int window_grow(dsm_engine* e, size_t need) {
+  if (e->h_win && need <= e->h_win_cap) return DSM_OK;
+  e->gen++;
+  if (e->h_win) HIPCHK(hipHostFree(e->h_win));
+  e->h_win = nullptr;
+  e->h_win_cap = 0;
+  const size_t cap = std::max<size_t>(4096, 2 * need);
+  HIPCHK(hipHostMalloc(&e->h_win, cap, hipHostMallocCoherent));
+  e->h_win_cap = cap;
+  return DSM_OK;
+}
+
+// The window's parameters into it.  (Every window ends with a wait for the stream, so no
+// launch reads the last one's any more.)
+int window_block(dsm_engine* e, const std::vector<int>& act, const std::vector<int>& cnt) {
+  const int rc = window_grow(e, sizeof(WinParam) * act.size() + sizeof(int) * cnt.size());
+  if (rc) return rc;
+  WinParam* wp = (WinParam*)e->h_win;
+  for (size_t q = 0; q < act.size(); ++q) {
+    const Ens& E = e->ens[act[q]];
+    wp[q] = WinParam{act[q], 0, E.P.t_end, E.P.k0, E.P.k_end};
+  }
+  if (!cnt.empty()) std::memcpy(wp + act.size(), cnt.data(), sizeof(int) * cnt.size());
   return DSM_OK;
 }
 
@@ -1379,24 +1401,9 @@ int advance_impl(dsm_engine* e, const std::vector<int>& ids, const std::vector<d
     }
     Pass timed;
     bool graph_timed = false;
+    if ((rc = window_block(e, act, cnt))) return rc;
     if (e->opt.graph && mode == DSM_MODE_BATCHED) {
-      // captured pass: window parameters through the pinned block, the launches replayed
-      const size_t need = sizeof(WinParam) * act.size() + sizeof(int) * cnt.size();
-      if (need > e->h_win_cap) {
-        e->gen++;
-        if (e->h_win) HIPCHK(hipHostFree(e->h_win));
-        e->h_win = nullptr;
-        e->h_win_cap = 0;
-        const size_t cap = std::max<size_t>(4096, 2 * need);
-        HIPCHK(hipHostMalloc(&e->h_win, cap, hipHostMallocCoherent));
-        e->h_win_cap = cap;
-      }
-      WinParam* wp = (WinParam*)e->h_win;
-      for (size_t q = 0; q < act.size(); ++q) {
-        const Ens& E = e->ens[act[q]];
-        wp[q] = WinParam{act[q], 0, E.P.t_end, E.P.k0, E.P.k_end};
-      }
-      if (!cnt.empty()) std::memcpy(wp + act.size(), cnt.data(), sizeof(int) * cnt.size());
+      // captured pass: the launches replayed
       std::vector<int64_t> key{(int64_t)e->gen};
       for (int id : act) {
         key.push_back(id);
@@ -1411,7 +1418,10 @@ int advance_impl(dsm_engine* e, const std::vector<int>& ids, const std::vector<d
       rs.kmc_launches++;
       rs.first_launches++;
     } else {
-      if ((rc = window_launches(e, act, cnt_off, row_off, cnt, mode, &rs, &timed))) return rc;
+      if ((rc = window_launches(e, act, cnt_off, row_off, cnt, mode, &rs, &timed))) {
+        (void)hipStreamSynchronize(e->st);  // what was launched reads the block
+        return rc;
+      }
     }
     // consume the window's samples: every reduction is queued, then one synchronisation
     std::vector<double> flow_host((size_t)flow_doubles);
@@ -1510,7 +1520,7 @@ int dsm_create(int32_t device_id, dsm_engine** out) {
   for (auto& ev : e->ev_bin) HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
   int rc;
   if ((rc = dev_alloc(&e->d_cnt, 2 * kNumLists + kZOrderScratch + 1)) || (rc = dev_alloc(&e->d_counters, kNumCounters)) ||
-      (rc = dev_alloc(&e->d_part, (size_t)kStressBlocks * 9))) {
+      (rc = dev_alloc(&e->d_part, (size_t)kStressBlocks * 9)) || (rc = window_grow(e, 0))) {
     dsm_destroy(e);
     return rc;
   }
