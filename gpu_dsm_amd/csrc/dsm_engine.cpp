@@ -675,6 +675,22 @@ bool solo_capable(const dsm_engine* e, const std::vector<int>& ids) {
   return e->opt.solo != 0;
 }
 
+// The solo form under flow (dsm_solo_flow.h) takes the place of the wave forms to 512
+// positions in sequential passes with flow, whatever else they hold but MSD sampling: a jump
+// of a chain alone on its SIMD takes 0.6 of the time (300 chains of Nk 100, 4 tau_K: 0.29
+// against 0.49 ms; 64 of Nk 30: 0.15 / 0.24; start-up of extension, 3001 chains of Nk 30, a whole
+// pass 0.94 / 1.01).  Beside the other forms of a concurrent pass, where the SIMDs are full,
+// the two are level (bursts of 12 and 24 mixed requests to Nk 512: 53.8 / 51.0, 93.2 / 97.9
+// ms), so those keep the wave forms.
+bool solo_flow_capable(const dsm_engine* e, const std::vector<int>& ids) {
+  bool flow = false;
+  for (int id : ids) {
+    flow = flow || e->ens[id].P.flow;
+    if (e->ens[id].P.sample_mode == kSampleMsd) return false;
+  }
+  return flow && e->opt.solo != 0;
+}
+
 // Its working memory: a record per strand slot, allocated when a pass first can use it,
 // and its rate tables for short strands.  It gives way to anything else: not taken beyond
 // a quarter of the free device memory, and given back when an allocation fails (the other
@@ -689,7 +705,7 @@ void release_lane(dsm_engine* e) {
 }
 int ensure_lane(dsm_engine* e, const std::vector<int>& ids) {
   const bool lanes = lane_quads(e, ids) || lane_share(e, ids);
-  if (!lanes && !solo_capable(e, ids) && !flow_cap(e, ids)) return DSM_OK;
+  if (!lanes && !solo_capable(e, ids) && !flow_cap(e, ids) && !solo_flow_capable(e, ids)) return DSM_OK;
   if (!e->d_lane_tab) {
     std::vector<float> t, out((size_t)kLaneTabFloats, 0.0f);
     build_tables(t, kLaneN, 1.0f, 0, 0.0f);
@@ -814,6 +830,7 @@ struct Pass {
   int flow_cap = 0;         // > 0: the lane form under flow with this many positions a chain
   int n_lane = 0;           // concurrent: chains that run in the lane form first
   bool solo = false;        // the solo form instead of the wave forms
+  bool solo_flow = false;   // the same under flow, bins 2 and 3 of a sequential pass
   int nmax = 0;
   bool concurrent = false;  // batched passes only: split by Z, geometries side by side
   int n_ens = 0;
@@ -853,6 +870,7 @@ int pass_setup(dsm_engine* e, const std::vector<int>& ids, bool use_ev_stop, Pas
                                          : (bin_max >= 3 || (bin_max >= 1 && z_est >= 56.0 * n_all));
   ps.flow_cap = batched && e->d_lane_tab ? flow_cap(e, ids) : 0;
   if (ps.lane_quads || ps.flow_cap) ps.concurrent = false;
+  ps.solo_flow = batched && !ps.concurrent && e->d_lane_tab && solo_flow_capable(e, ids);
   ps.n_lane = ps.concurrent && batched && e->d_rec_cap >= e->nstr ? lane_share(e, ids) : 0;
   if (n0 == 0) return DSM_OK;
   ps.range = batched && !ps.concurrent && ids.size() == 1;
@@ -880,8 +898,12 @@ int pass_setup(dsm_engine* e, const std::vector<int>& ids, bool use_ev_stop, Pas
 constexpr int kLateFirst = 2;
 int late_last(int bin_max) { return std::max(bin_max, kLateFirst); }
 
-// Launches bin b >= kLateFirst of a batched pass: the solo form, or the wave form `geom`.
+// Launches bin b >= kLateFirst of a batched pass: a solo form, or the wave form `geom`.
 hipError_t launch_wave(dsm_engine* e, const Pass& ps, const KmcArgs& a, int b, int geom, hipStream_t st) {
+  if (ps.solo_flow && b <= 3) {
+    const int cap = kmc_geom_capacity(b);
+    return launch_kmc_solo_flow(a, cap, std::min(ps.n0, kmc_solo_flow_occupancy(cap) * e->n_cu), st);
+  }
   if (!ps.solo) return launch_kmc(a, geom, false, device_blocks(e, geom, false, a.lds_floats, a.ext != 0), st);
   const int cap = kmc_geom_capacity(b);
   return launch_kmc_solo(a, cap, std::min(ps.n0, kmc_solo_occupancy(cap) * e->n_cu), st);

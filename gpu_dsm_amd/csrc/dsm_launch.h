@@ -79,6 +79,9 @@ hipError_t launch_kmc_lane_flow(const KmcArgs& a, int cap, int grid, hipStream_t
 // and a launch of `grid` waves.
 int kmc_solo_occupancy(int cap);
 hipError_t launch_kmc_solo(const KmcArgs& a, int cap, int grid, hipStream_t st);
+// The solo form for passes with flow, cap 256 or 512.
+int kmc_solo_flow_occupancy(int cap);
+hipError_t launch_kmc_solo_flow(const KmcArgs& a, int cap, int grid, hipStream_t st);
 // chains first .. first+n-1
 hipError_t launch_init_eq(const ChainArrays& ch, const EnsParams* ens, const float* tabs, int first, int n,
                           hipStream_t st);

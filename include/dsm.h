@@ -109,10 +109,10 @@ int dsm_mem_info(int32_t device_id, size_t* free_bytes, size_t* total_bytes);
 #define DSM_OPT_WIDE_PAIR 9         /* concurrent pass of one ensemble: chains with 128 <= Z < 240 run two
                                        per wave and those with 64 <= Z < 128 four (1), or one and two (0)
                                        (1) */
-#define DSM_OPT_LANE 10             /* batched equilibrium passes whose chains stay short enough run one chain
-                                       per lane: 1 by the pass's chain count, 0 never, 2 always (1) */
-#define DSM_OPT_SOLO 11             /* batched passes without flow: few or long chains run one per wave out of
-                                       LDS (1) or in the wave forms (0) (1) */
+#define DSM_OPT_LANE 10             /* batched passes, without flow or of flow alone: chains that stay short enough
+                                       run one per lane: 1 by their count, 0 never, 2 always (1) */
+#define DSM_OPT_SOLO 11             /* batched passes: few or long chains (under flow: few, to 512 positions) run
+                                       in the solo forms (1) or the wave forms (0) (1) */
 int dsm_set_option(dsm_engine* e, int32_t key, int32_t value);
 int dsm_get_option(dsm_engine* e, int32_t key, int32_t* value);
 
