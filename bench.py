@@ -6,17 +6,18 @@ chains, Nk = round(LogNormal) with number average 200 and Mw/Mn = 1.5 clipped to
 [10, 2000], beta = 1, constraint dynamics on with CD partners drawn from the melt's own
 length distribution (weight-averaged), G(t) sampled every tau_K into the multi-tau
 correlator (16 points per level, block factor 2).  One "step" advances every chain by
---window Kuhn times through the batched persistent form (chains split by Z into six
-bins whose kernels run side by side on four streams), plus the correlator update.  All inputs
+--window Kuhn times through the batched persistent form (the short chains one per lane, then
+the others, split by Z into bins whose kernels run side by side on four streams), plus the
+correlator update.  All inputs
 are synthetic (Philox-keyed equilibrium draw); the state is resident in HBM when the
 timed region starts.
 
 Printed: one JSON line.
   value        whole-job jumps/s of the headline workload (wall clock over the timed steps)
-  roofline     the KMC pass of one step (six geometry kernels, HIP events from the split
-               to the end of the late round): bound "valu" -- the kernels keep each chain
-               in registers for the whole window, so HBM sees one read and one write of a
-               chain per window and VALU issue is the limit (rocprofv3 counters).
+  roofline     the KMC pass of one step (HIP events from the split to the end of the late
+               round): bound "valu" -- the kernels keep each chain's rates in LDS or
+               registers for the whole window, and VALU issue is the limit (rocprofv3
+               counters).
                achieved = VALU wave-instructions per jump (committed rocprofv3 PMC summary
                of the same pass, profiles/) x jumps per step / pass time per step, against
                the issue peak of 256 CUs x 4 SIMDs x 2.4 GHz / 4 cycles per wave64
@@ -379,7 +380,7 @@ def main():
     pass_ms = c3["kmc_ms"] / args.steps
     rl = roofline(c3, args.steps, counters("kmc_pass_c3_counters.json"), pass_ms)
     c2 = run_c2(g, args, [])
-    rl2 = roofline(c2, args.steps, counters("kmc_row_form_c2_counters.json"), c2["first_ms"] / args.steps)
+    rl2 = roofline(c2, args.steps, counters("kmc_lane_form_c2_counters.json"), c2["first_ms"] / args.steps)
     pvb = None if args.no_plain else run_plain_vs_batched(g, args)
     copy_bytes = 1 << 30
     copy_ms = g.probe_copy(copy_bytes, 20)
@@ -417,9 +418,9 @@ def main():
         "config": {"workload": "polydisperse melt, 262144 chains, Nk log-normal (Mn 200, PDI 1.5) clipped to "
                                "[10, 2000], beta=1, CD on with melt partners, G(t) multi-tau p=16 m=2, "
                                "%d tau_K per step" % args.window,
-                   "form": "batched persistent: chains split by Z into six bins (row form 4 chains per wave "
-                           "Z<64, two-group row form 4 per wave Z<128, two-group pair form 2 per wave Z<240, "
-                           "wave form 1 per wave Z<480/960/2048) run side by side on four streams, then a late round for "
+                   "form": "batched persistent: chains that stay below 128 positions one per lane (lane form), then the "
+                           "others split by Z (two-group row form 4 per wave Z<128, solo form 1 per wave out of LDS "
+                           "Z<240/480/960/2048) side by side on four streams, then a late round for "
                            "chains that outgrew theirs",
                    "n_chains": C3["n_chains"], "nk_max": int(c3["nk"].max()), "nk_mean": float(c3["nk"].mean()),
                    "window_tau_k": args.window},
