@@ -254,15 +254,6 @@ struct RangeAlloc {
         return s0;
       }
     }
-    if (!free_.empty()) {  // a free range at the end is extended
-      auto last = std::prev(free_.end());
-      if (last->first + last->second == end) {
-        const int64_t s0 = last->first;
-        free_.erase(last);
-        end = s0 + n;
-        return s0;
-      }
-    }
     const int64_t s0 = end;
     end += n;
     return s0;
@@ -283,6 +274,10 @@ struct RangeAlloc {
       it->second += next->second;
       free_.erase(next);
     }
+    if (it->first + it->second == end) {  // nothing is taken behind it
+      end = it->first;
+      free_.erase(it);
+    }
   }
 };
 
@@ -302,8 +297,8 @@ struct Ens {
   bool live = false;
   dsm_ensemble_desc d{};
   std::vector<int> nk;
-  int chain0 = 0, n = 0, nmax = 0;
-  int64_t strand0 = 0, nstrand = 0;
+  int chain0 = -1, n = 0, nmax = 0;  // (-1: no chains taken)
+  int64_t strand0 = -1, nstrand = 0;
   EnsParams P{};
   int bin_max = 0;      // largest geometry bin a chain of this ensemble can need
   int n_lane = 0;          // its chains that stay within the lane form's largest columns
@@ -379,7 +374,6 @@ struct dsm_engine {
   };
   std::vector<TabSlot> tab_slots;
   std::vector<int64_t> stage_off;  // per ensemble
-  int64_t stage_used = 0;
   RangeAlloc chain_space, strand_space, stage_space;
   float* d_stage = nullptr;
   int64_t d_stage_cap = 0;
@@ -439,6 +433,32 @@ int grow(T** p, int64_t n_old, int64_t n_new, hipStream_t st) {
   return DSM_OK;
 }
 
+// Room for `need` elements in a device array of *cap whose contents need not be kept (*lost:
+// they were not).  When memory is short the old array makes way for the new one; should even
+// that fail, the engine goes on with an array of the old size.
+template <typename T, typename N>
+int reserve(dsm_engine* e, T** p, N* cap, int64_t need, bool* lost = nullptr) {
+  if (need <= (int64_t)*cap && (*p || need == 0)) return DSM_OK;
+  e->gen++;
+  T* q = nullptr;
+  int rc = dev_alloc(&q, (size_t)need);
+  if (rc == DSM_OK || *p) {
+    HIPCHK(hipStreamSynchronize(e->st));
+    if (lost) *lost = true;
+    if (*p) (void)hipFree(*p);
+    *p = nullptr;
+    const int64_t old = (int64_t)*cap;
+    *cap = 0;
+    if (rc) rc = dev_alloc(&q, (size_t)need);
+    if (rc && old > 0 && dev_alloc(&q, (size_t)old) == DSM_OK) need = old;
+    if (q) {
+      *p = q;
+      *cap = (N)need;
+    }
+  }
+  return rc;
+}
+
 // capacity after growth to `need`: half again the current capacity, so that a stream of
 // additions copies each element a bounded number of times, unless the extra would take
 // more than a quarter of the free device memory (then exactly `need`)
@@ -456,7 +476,7 @@ constexpr size_t kStrandBytes = 5 * 4;                             // Qx Qy Qz N
 int grow_chains(dsm_engine* e, int n_need, int64_t s_need) {
   ChainArrays& c = e->ch;
   int rc = 0;
-  e->gen++;  // chain arrays or work lists may move
+  e->gen++;  // chain arrays may move
   if (n_need > e->nch) {
     const int n0 = e->nch;
     const int n_new = (int)std::min<int64_t>(grown_capacity(n0, n_need, kChainBytes), INT32_MAX / 2);
@@ -480,53 +500,44 @@ int grow_chains(dsm_engine* e, int n_need, int64_t s_need) {
       return rc;
     e->nstr = s_new;
   }
-  // bin 0 pads every live ensemble to whole quads; one spare list past the last bin
-  int live = 1;
-  for (const Ens& E : e->ens) live += E.live ? 1 : 0;
-  const int need = e->nch + 4 * (live + 2);
-  if (need > e->d_work_cap) {
-    if (e->d_work) HIPCHK(hipFree(e->d_work));
-    e->d_work = nullptr;
-    e->d_work_cap = 0;
-    const int cap = need + need / 8 + 1024;
-    if ((rc = dev_alloc(&e->d_work, (size_t)kNumLists * cap))) return rc;
-    e->d_work_cap = cap;
-  }
   return DSM_OK;
 }
 
+// Work lists for a pass over all ensembles and `more` to come, each of as many entries as
+// there are chains, padded to whole quads by ensemble, and a spare list past the last bin.
+int ensure_work(dsm_engine* e, int more) {
+  int live = more;
+  for (const Ens& E : e->ens) live += E.live ? 1 : 0;
+  const int64_t need = e->chain_space.end + 4 * (live + 2);
+  if (e->d_work && need <= e->d_work_cap) return DSM_OK;
+  const int64_t room = std::max(need, (int64_t)e->nch + 4 * (live + 2));
+  int64_t floats = (int64_t)kNumLists * e->d_work_cap;
+  const int rc = reserve(e, &e->d_work, &floats, kNumLists * (room + room / 8 + 1024));
+  e->d_work_cap = (int)(floats / kNumLists);
+  return rc;
+}
+
 int upload_ens(dsm_engine* e) {
-  const int n = (int)e->ens.size();
-  if (n > e->d_ens_cap) {
-    e->gen++;
-    if (e->d_ens) HIPCHK(hipFree(e->d_ens));
-    int rc = dev_alloc(&e->d_ens, (size_t)std::max(n, 16));
-    if (rc) return rc;
-    e->d_ens_cap = std::max(n, 16);
-  }
+  const int rc = reserve(e, &e->d_ens, &e->d_ens_cap, std::max<int64_t>((int64_t)e->ens.size(), 16));
+  const int n = std::min((int)e->ens.size(), e->d_ens_cap);
   std::vector<EnsParams> h(n);
   for (int i = 0; i < n; ++i) h[i] = e->ens[i].P;
-  HIPCHK(hipMemcpyAsync(e->d_ens, h.data(), sizeof(EnsParams) * n, hipMemcpyHostToDevice, e->st));
+  if (n > 0) HIPCHK(hipMemcpyAsync(e->d_ens, h.data(), sizeof(EnsParams) * n, hipMemcpyHostToDevice, e->st));
   HIPCHK(hipStreamSynchronize(e->st));
-  return DSM_OK;
+  return rc;
 }
 
 // floats [off, off+n) of the table arena to the device (all of it when the device copy grows)
 int upload_tabs(dsm_engine* e, int64_t off, int64_t n) {
-  if (e->tabs.size() > e->d_tabs_cap) {
-    e->gen++;
-    if (e->d_tabs) HIPCHK(hipFree(e->d_tabs));
-    e->d_tabs = nullptr;
-    e->d_tabs_cap = 0;
-    const size_t cap = std::max(e->tabs.size() * 2, (size_t)4096);
-    int rc = dev_alloc(&e->d_tabs, cap);
-    if (rc) return rc;
-    e->d_tabs_cap = cap;
+  int rc = DSM_OK;
+  if (!e->d_tabs || e->tabs.size() > e->d_tabs_cap) {
+    bool lost = false;
+    rc = reserve(e, &e->d_tabs, &e->d_tabs_cap, std::max((int64_t)e->tabs.size() * 2, (int64_t)4096), &lost);
     off = 0;
-    n = (int64_t)e->tabs.size();
+    n = lost ? (int64_t)std::min(e->tabs.size(), e->d_tabs_cap) : 0;
   }
-  HIPCHK(hipMemcpy(e->d_tabs + off, e->tabs.data() + off, sizeof(float) * n, hipMemcpyHostToDevice));
-  return DSM_OK;
+  if (n > 0) HIPCHK(hipMemcpy(e->d_tabs + off, e->tabs.data() + off, sizeof(float) * n, hipMemcpyHostToDevice));
+  return rc;
 }
 
 bool same_tables(const dsm_engine::TabSlot& a, const dsm_engine::TabSlot& b) {
@@ -551,8 +562,9 @@ int take_tables(dsm_engine* e, const dsm_engine::TabSlot& key, Make make, int* s
   dsm_engine::TabSlot t = key;
   make(data, t);
   int idx = -1;
+  const size_t n_slots = e->tab_slots.size(), n_floats = e->tabs.size();
   for (size_t i = 0; i < e->tab_slots.size(); ++i)
-    if (e->tab_slots[i].refs == 0 && e->tab_slots[i].kind == key.kind && e->tab_slots[i].size == (int64_t)data.size()) {
+    if (e->tab_slots[i].refs == 0 && e->tab_slots[i].size == (int64_t)data.size()) {
       idx = (int)i;
       break;
     }
@@ -569,14 +581,45 @@ int take_tables(dsm_engine* e, const dsm_engine::TabSlot& key, Make make, int* s
   t.refs = 1;
   std::copy(data.begin(), data.end(), e->tabs.begin() + t.off);
   e->tab_slots[idx] = t;
+  const int rc = upload_tabs(e, t.off, t.size);
+  if (rc) {  // the device has no such tables: a slot that was free is no one's, a new one goes
+    if (e->tab_slots.size() > n_slots) {
+      e->tab_slots.pop_back();
+      e->tabs.resize(n_floats);
+    } else {
+      e->tab_slots[idx].kind = -1;
+      e->tab_slots[idx].refs = 0;
+    }
+    return rc;
+  }
   *slot = idx;
-  return upload_tabs(e, t.off, t.size);
+  return DSM_OK;
+}
+
+// What every pass reads, should a failed growth have left the engine without it.
+int ensure_device(dsm_engine* e) {
+  int rc = ensure_work(e, 0);
+  if (rc == DSM_OK && (!e->d_tabs || e->tabs.size() > e->d_tabs_cap)) rc = upload_tabs(e, 0, (int64_t)e->tabs.size());
+  if (rc == DSM_OK && (!e->d_ens || (int)e->ens.size() > e->d_ens_cap)) rc = upload_ens(e);
+  return rc;
+}
+
+// An ensemble's table slots, chains, strand slots and staging rows, back to the engine.
+void give_back(dsm_engine* e, Ens& E) {
+  if (E.tab_slot >= 0) e->tab_slots[E.tab_slot].refs--;
+  if (E.pd_slot >= 0) e->tab_slots[E.pd_slot].refs--;
+  E.tab_slot = E.pd_slot = -1;
+  if (E.chain0 >= 0) e->chain_space.give(E.chain0, E.n);
+  if (E.strand0 >= 0) e->strand_space.give(E.strand0, E.nstrand);
+  if (E.P.stage_off >= 0) e->stage_space.give(E.P.stage_off, E.stage_floats);
+  E.chain0 = -1;
+  E.strand0 = E.P.stage_off = -1;
 }
 
 int ensure_stage(dsm_engine* e) {
-  if (e->stage_used > e->d_stage_cap) {  // keeps the rows of live ensembles (last_samples)
+  if (e->stage_space.end > e->d_stage_cap) {  // keeps the rows of live ensembles (last_samples)
     e->gen++;
-    const int64_t cap = grown_capacity(e->d_stage_cap, e->stage_used, sizeof(float));
+    const int64_t cap = grown_capacity(e->d_stage_cap, e->stage_space.end, sizeof(float));
     int rc = grow(&e->d_stage, e->d_stage_cap, cap, e->st);
     if (rc) return rc;
     e->d_stage_cap = cap;
@@ -738,29 +781,36 @@ Ens* get_ens(dsm_engine* e, int id) {
   return &e->ens[id];
 }
 
-// correlator memory, sized when the level count is known
+// correlator memory, sized when the level count is known; all of it or none
+void corr_free(Ens& E) {
+  for (double** p : {&E.dD, &E.dA, &E.dC}) {
+    if (*p) (void)hipFree(*p);
+    *p = nullptr;
+  }
+  E.s = 0;
+}
 int corr_alloc(dsm_engine* e, Ens& E, int s) {
   if (E.s == s && E.dD) return DSM_OK;
   e->gen++;
-  if (E.dD) { (void)hipFree(E.dD); (void)hipFree(E.dA); (void)hipFree(E.dC); E.dD = E.dA = E.dC = nullptr; }
-  E.s = s;
-  const size_t n = (size_t)E.n;
+  corr_free(E);
+  const size_t n = (size_t)E.n, nD = (size_t)s * E.p * 3 * n, nA = (size_t)s * 3 * n, nC = (size_t)s * E.p * n;
   int rc;
-  if ((rc = dev_alloc(&E.dD, (size_t)s * E.p * 3 * n)) || (rc = dev_alloc(&E.dA, (size_t)s * 3 * n)) ||
-      (rc = dev_alloc(&E.dC, (size_t)s * E.p * n)))
+  if ((rc = dev_alloc(&E.dD, nD)) || (rc = dev_alloc(&E.dA, nA)) || (rc = dev_alloc(&E.dC, nC))) {
+    corr_free(E);
     return rc;
-  HIPCHK(hipMemsetAsync(E.dD, 0, sizeof(double) * s * E.p * 3 * n, e->st));
-  HIPCHK(hipMemsetAsync(E.dA, 0, sizeof(double) * s * 3 * n, e->st));
-  HIPCHK(hipMemsetAsync(E.dC, 0, sizeof(double) * s * E.p * n, e->st));
+  }
+  hipError_t he = hipMemsetAsync(E.dD, 0, sizeof(double) * nD, e->st);
+  if (he == hipSuccess) he = hipMemsetAsync(E.dA, 0, sizeof(double) * nA, e->st);
+  if (he == hipSuccess) he = hipMemsetAsync(E.dC, 0, sizeof(double) * nC, e->st);
+  if (he == hipSuccess) he = hipStreamSynchronize(e->st);
+  if (he != hipSuccess) {
+    corr_free(E);
+    return fail(DSM_ERR_DEVICE, "correlator memory: %s", hipGetErrorString(he));
+  }
+  E.s = s;
   E.ins.assign(s, 0);
   E.macc.assign(s, 0);
   E.nins.assign(s, 0);
-  if (3 * s > e->d_corr_cnt_cap) {
-    if (e->d_corr_cnt) HIPCHK(hipFree(e->d_corr_cnt));
-    if ((rc = dev_alloc(&e->d_corr_cnt, (size_t)3 * s))) return rc;
-    e->d_corr_cnt_cap = 3 * s;
-  }
-  HIPCHK(hipStreamSynchronize(e->st));
   return DSM_OK;
 }
 
@@ -1309,7 +1359,7 @@ int advance_impl(dsm_engine* e, const std::vector<int>& ids, const std::vector<d
   Timer T;
   dsm_run_stats rs{};
   int rc = set_device(e);
-  if (rc) return rc;
+  if (rc || (rc = ensure_device(e))) return rc;
   // jump and Z totals before (d_counters[0..1]) and after (d_counters[2..3]) the call,
   // summed on the device: the "after" sums and their copy ride on the last window's
   // synchronisation, so the totals cost no host round trip of their own
@@ -1345,9 +1395,6 @@ int advance_impl(dsm_engine* e, const std::vector<int>& ids, const std::vector<d
         if ((rc = corr_alloc(e, E, s))) {
           if (rc != DSM_ERR_MEMORY || !e->d_rec) return rc;
           release_lane(e);
-          if (E.dD) (void)hipFree(E.dD);
-          if (E.dA) (void)hipFree(E.dA);
-          E.dD = E.dA = E.dC = nullptr;
           if ((rc = corr_alloc(e, E, s))) return rc;
         }
       }
@@ -1401,26 +1448,10 @@ int advance_impl(dsm_engine* e, const std::vector<int>& ids, const std::vector<d
         row_parts = std::max(row_parts, (E.P.k_end - E.P.k0) * 9 * flow_reduce_parts(E.n));
       }
     }
-    if ((int)cnt.size() > e->d_corr_cnt_cap) {
-      e->gen++;
-      if (e->d_corr_cnt) HIPCHK(hipFree(e->d_corr_cnt));
-      if ((rc = dev_alloc(&e->d_corr_cnt, cnt.size()))) return rc;
-      e->d_corr_cnt_cap = (int)cnt.size();
-    }
-    if (flow_doubles > e->d_rows_cap) {
-      e->gen++;
-      if (e->d_rows) HIPCHK(hipFree(e->d_rows));
-      if ((rc = dev_alloc(&e->d_rows, (size_t)flow_doubles))) return rc;
-      e->d_rows_cap = flow_doubles;
-    }
-    if (row_parts > e->d_row_part_cap) {
-      e->gen++;
-      if (e->d_row_part) HIPCHK(hipFree(e->d_row_part));
-      e->d_row_part = nullptr;
-      e->d_row_part_cap = 0;
-      if ((rc = dev_alloc(&e->d_row_part, (size_t)row_parts))) return rc;
-      e->d_row_part_cap = row_parts;
-    }
+    if ((rc = reserve(e, &e->d_corr_cnt, &e->d_corr_cnt_cap, (int64_t)cnt.size())) ||
+        (rc = reserve(e, &e->d_rows, &e->d_rows_cap, flow_doubles)) ||
+        (rc = reserve(e, &e->d_row_part, &e->d_row_part_cap, row_parts)))
+      return rc;
     Pass timed;
     bool graph_timed = false;
     if ((rc = window_block(e, act, cnt))) return rc;
@@ -1601,6 +1632,12 @@ int dsm_add_ensemble(dsm_engine* e, const dsm_ensemble_desc* d, int32_t* ens_id)
   if (rc) return rc;
   e->gen++;
   Ens E;
+  E.P.stage_off = -1;
+  struct Undo {  // what a call that fails has taken
+    dsm_engine* e;
+    Ens* E;
+    ~Undo() { if (E) give_back(e, *E); }
+  } undo{e, &E};
   E.d = *d;
   E.d.nk_per_chain = nullptr;
   E.n = d->n_chains;
@@ -1708,7 +1745,6 @@ int dsm_add_ensemble(dsm_engine* e, const dsm_ensemble_desc* d, int32_t* ens_id)
   if (E.p % E.m != 0 && eq_sampling(d->sample_mode)) return fail(DSM_ERR_ARG, "corr_p must be a multiple of corr_m");
   E.stage_floats = ((int64_t)E.window * E.n * E.ncomp + 3) & ~(int64_t)3;  // rows start on 16 bytes
   P.stage_off = e->stage_space.take(E.stage_floats);
-  e->stage_used = std::max(e->stage_used, e->stage_space.end);
   if ((rc = ensure_stage(e))) {
     if (rc != DSM_ERR_MEMORY || !e->d_rec) return rc;
     release_lane(e);
@@ -1720,10 +1756,14 @@ int dsm_add_ensemble(dsm_engine* e, const dsm_ensemble_desc* d, int32_t* ens_id)
   for (int i = 0; i < E.n; ++i) E.nstrand += cap_of(E.nk[i]);
   P.chain0 = E.chain0;
   E.strand0 = e->strand_space.take(E.nstrand);
-  if ((rc = grow_chains(e, (int)e->chain_space.end, e->strand_space.end))) {
+  auto room = [&]() {
+    const int r = grow_chains(e, (int)e->chain_space.end, e->strand_space.end);
+    return r ? r : ensure_work(e, 1);
+  };
+  if ((rc = room())) {
     if (rc != DSM_ERR_MEMORY || !e->d_rec) return rc;
     release_lane(e);
-    if ((rc = grow_chains(e, (int)e->chain_space.end, e->strand_space.end))) return rc;
+    if ((rc = room())) return rc;
   }
   {
     const int id = (int)e->ens.size();
@@ -1753,7 +1793,12 @@ int dsm_add_ensemble(dsm_engine* e, const dsm_ensemble_desc* d, int32_t* ens_id)
     HIPCHK(hipMemcpy(e->ch.next_sample + c0, hns.data(), 8 * E.n, hipMemcpyHostToDevice));
     E.live = true;
     e->ens.push_back(std::move(E));
-    if ((rc = upload_ens(e))) return rc;
+    if ((rc = upload_ens(e))) {
+      E = std::move(e->ens.back());
+      e->ens.pop_back();
+      return rc;
+    }
+    undo.E = nullptr;
     if (ens_id) *ens_id = id;
   }
   return DSM_OK;
@@ -1764,17 +1809,11 @@ int dsm_remove_ensemble(dsm_engine* e, int32_t ens) {
   if (!E) return fail(DSM_ERR_ARG, "no ensemble %d", ens);
   (void)set_device(e);
   e->gen++;
-  if (E->dD) { (void)hipFree(E->dD); (void)hipFree(E->dA); (void)hipFree(E->dC); E->dD = E->dA = E->dC = nullptr; }
+  corr_free(*E);
   E->live = false;
   E->flow_rows.clear();
   E->flow_rows.shrink_to_fit();
-  // its chains, strand slots and staging rows go back to the engine's free ranges
-  if (E->tab_slot >= 0) e->tab_slots[E->tab_slot].refs--;
-  if (E->pd_slot >= 0) e->tab_slots[E->pd_slot].refs--;
-  E->tab_slot = E->pd_slot = -1;
-  e->chain_space.give(E->chain0, E->n);
-  e->strand_space.give(E->strand0, E->nstrand);
-  e->stage_space.give(E->P.stage_off, E->stage_floats);
+  give_back(e, *E);
   return DSM_OK;
 }
 
@@ -1782,7 +1821,7 @@ int dsm_init_equilibrium(dsm_engine* e, int32_t ens) {
   Ens* E = get_ens(e, ens);
   if (!E) return fail(DSM_ERR_ARG, "no ensemble %d", ens);
   int rc = set_device(e);
-  if (rc) return rc;
+  if (rc || (rc = ensure_device(e))) return rc;
   HIPCHK(launch_init_eq(e->ch, e->d_ens, e->d_tabs, E->chain0, E->n, e->st));
   HIPCHK(hipStreamSynchronize(e->st));
   E->k_cur = E->P.sample_mode == kSampleFlow ? 1 : 0;
@@ -1935,7 +1974,7 @@ int dsm_advance_events(dsm_engine* e, int32_t ens, int64_t n_events, int32_t mod
   if (!E) return fail(DSM_ERR_ARG, "no ensemble %d", ens);
   if (n_events < 0) return fail(DSM_ERR_ARG, "negative event count");
   int rc = set_device(e);
-  if (rc) return rc;
+  if (rc || (rc = ensure_device(e))) return rc;
   Timer T;
   dsm_run_stats rs{};
   if (mode == DSM_MODE_BATCHED && (rc = ensure_lane(e, {ens}))) return rc;
@@ -2073,13 +2112,7 @@ int dsm_correlator_range(dsm_engine* e, int32_t ens, int32_t first, int32_t coun
   std::vector<double> sums((size_t)s * p + 1, 0.0);
   if (g && max_pts > 0) {
     const int64_t npt = (int64_t)s * p + 1, need = npt * (1 + corr_reduce_parts(count));
-    if (need > e->d_red_cap) {
-      if (e->d_red) HIPCHK(hipFree(e->d_red));
-      e->d_red = nullptr;
-      e->d_red_cap = 0;
-      if ((rc = dev_alloc(&e->d_red, (size_t)need))) return rc;
-      e->d_red_cap = need;
-    }
+    if ((rc = reserve(e, &e->d_red, &e->d_red_cap, need))) return rc;
     HIPCHK(launch_corr_reduce(E->dC, E->n, e->ch.stall, E->chain0, first, count, p, m, s, E->nins.data(),
                               e->d_red + npt, e->d_red, e->st));
     HIPCHK(hipMemcpyAsync(sums.data(), e->d_red, sizeof(double) * npt, hipMemcpyDeviceToHost, e->st));
