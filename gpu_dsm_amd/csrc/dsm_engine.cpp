@@ -561,6 +561,7 @@ int take_tables(dsm_engine* e, const dsm_engine::TabSlot& key, Make make, int* s
   std::vector<float> data;
   dsm_engine::TabSlot t = key;
   make(data, t);
+  if (data.empty()) return DSM_ERR_ARG;  // there are none for these parameters
   int idx = -1;
   const size_t n_slots = e->tab_slots.size(), n_floats = e->tabs.size();
   for (size_t i = 0; i < e->tab_slots.size(); ++i)

@@ -132,9 +132,32 @@ static void check_alloc() {
   CHECK(fake::live_bytes == 0);
 }
 
+// ------------------------------------------------------------------ refused stays refused
+static void check_refused() {
+  dsm_engine* e = nullptr;
+  CHECK(dsm_create(0, &e) == DSM_OK);
+  int32_t id = -1;
+  for (int k = 0; k < 3; ++k) {  // a background that has no quantiles
+    dsm_ensemble_desc d = desc(20, 30, DSM_SAMPLE_GT);
+    d.partner_mode = DSM_PARTNER_GEX;
+    d.gex[0] = 1.0f;
+    d.gex[1] = 0.0f;
+    d.gex[2] = 40000.0f;
+    d.gex[3] = 120.0f;
+    CHECK(dsm_add_ensemble(e, &d, &id) == DSM_ERR_ARG);
+  }
+  dsm_ensemble_desc d = desc(20, 30, DSM_SAMPLE_GT);
+  d.corr_m = 3;  // 16 points
+  for (int k = 0; k < 3; ++k) CHECK(dsm_add_ensemble(e, &d, &id) == DSM_ERR_ARG);
+  d.corr_m = 2;
+  CHECK(dsm_add_ensemble(e, &d, &id) == DSM_OK && id == 0);
+  dsm_destroy(e);
+}
+
 int main(int argc, char** argv) {
   const std::string which = argc > 1 ? argv[1] : "";
   if (which == "alloc") check_alloc();
+  else if (which == "refused") check_refused();
   else return 2;
   std::printf("engine checks (%s): %d failures\n", which.c_str(), failures);
   return failures ? 1 : 0;

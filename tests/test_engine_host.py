@@ -39,3 +39,8 @@ def test_every_allocation_may_fail(checks):
     """Each device allocation of a session fails in turn, alone or with all that follow: the
     call is refused or done, the ensembles there are go on, and the repeated call succeeds."""
     checks("alloc")
+
+
+def test_a_refused_ensemble_is_refused_again(checks):
+    """A GEX background without quantiles, and a block factor that does not divide the lags."""
+    checks("refused")
