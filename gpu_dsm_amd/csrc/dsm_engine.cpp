@@ -281,15 +281,6 @@ struct RangeAlloc {
   }
 };
 
-template <typename T>
-int dev_alloc(T** p, size_t n) {
-  *p = nullptr;
-  if (n == 0) n = 1;
-  hipError_t e = hipMalloc((void**)p, n * sizeof(T));
-  if (e != hipSuccess) return fail(DSM_ERR_MEMORY, "hipMalloc(%zu bytes): %s", n * sizeof(T), hipGetErrorString(e));
-  return DSM_OK;
-}
-
 // G(t) and MSD(t) both sample the equilibrium state every delta into a multi-tau correlator
 inline bool eq_sampling(int mode) { return mode == kSampleEq || mode == kSampleMsd; }
 
@@ -420,14 +411,41 @@ int set_device(dsm_engine* e) {
   return DSM_OK;
 }
 
+// Gives the lane form's records back (the passes then run in the other forms).
+void release_lane(dsm_engine* e) {
+  if (!e->d_rec) return;
+  e->gen++;
+  (void)hipStreamSynchronize(e->st);
+  (void)hipFree(e->d_rec);
+  e->d_rec = nullptr;
+  e->d_rec_cap = 0;
+}
+
+// n elements of device memory; the lane form's records make way for them.
+template <typename T>
+int dev_alloc(dsm_engine* e, T** p, size_t n) {
+  *p = nullptr;
+  if (n == 0) n = 1;
+  hipError_t rc = hipMalloc((void**)p, n * sizeof(T));
+  if (rc != hipSuccess && e->d_rec) {
+    (void)hipGetLastError();
+    release_lane(e);
+    rc = hipMalloc((void**)p, n * sizeof(T));
+  }
+  if (rc == hipSuccess) return DSM_OK;
+  (void)hipGetLastError();
+  *p = nullptr;
+  return fail(DSM_ERR_MEMORY, "hipMalloc(%zu bytes): %s", n * sizeof(T), hipGetErrorString(rc));
+}
+
 // grow a device array of n_old elements to n_new, preserving contents
 template <typename T>
-int grow(T** p, int64_t n_old, int64_t n_new, hipStream_t st) {
+int grow(dsm_engine* e, T** p, int64_t n_old, int64_t n_new) {
   T* q = nullptr;
-  int rc = dev_alloc(&q, (size_t)n_new);
+  int rc = dev_alloc(e, &q, (size_t)n_new);
   if (rc) return rc;
-  if (*p && n_old > 0) HIPCHK(hipMemcpyAsync(q, *p, (size_t)n_old * sizeof(T), hipMemcpyDeviceToDevice, st));
-  HIPCHK(hipStreamSynchronize(st));
+  if (*p && n_old > 0) HIPCHK(hipMemcpyAsync(q, *p, (size_t)n_old * sizeof(T), hipMemcpyDeviceToDevice, e->st));
+  HIPCHK(hipStreamSynchronize(e->st));
   if (*p) HIPCHK(hipFree(*p));
   *p = q;
   return DSM_OK;
@@ -441,7 +459,7 @@ int reserve(dsm_engine* e, T** p, N* cap, int64_t need, bool* lost = nullptr) {
   if (need <= (int64_t)*cap && (*p || need == 0)) return DSM_OK;
   e->gen++;
   T* q = nullptr;
-  int rc = dev_alloc(&q, (size_t)need);
+  int rc = dev_alloc(e, &q, (size_t)need);
   if (rc == DSM_OK || *p) {
     HIPCHK(hipStreamSynchronize(e->st));
     if (lost) *lost = true;
@@ -449,8 +467,8 @@ int reserve(dsm_engine* e, T** p, N* cap, int64_t need, bool* lost = nullptr) {
     *p = nullptr;
     const int64_t old = (int64_t)*cap;
     *cap = 0;
-    if (rc) rc = dev_alloc(&q, (size_t)need);
-    if (rc && old > 0 && dev_alloc(&q, (size_t)old) == DSM_OK) need = old;
+    if (rc) rc = dev_alloc(e, &q, (size_t)need);
+    if (rc && old > 0 && dev_alloc(e, &q, (size_t)old) == DSM_OK) need = old;
     if (q) {
       *p = q;
       *cap = (N)need;
@@ -480,23 +498,23 @@ int grow_chains(dsm_engine* e, int n_need, int64_t s_need) {
   if (n_need > e->nch) {
     const int n0 = e->nch;
     const int n_new = (int)std::min<int64_t>(grown_capacity(n0, n_need, kChainBytes), INT32_MAX / 2);
-    if ((rc = grow(&c.Z, n0, n_new, e->st)) || (rc = grow(&c.nk, n0, n_new, e->st)) ||
-        (rc = grow(&c.ens, n0, n_new, e->st)) || (rc = grow(&c.cap, n0, n_new, e->st)) ||
-        (rc = grow(&c.stall, n0, n_new, e->st)) || (rc = grow(&c.cid, n0, n_new, e->st)) ||
-        (rc = grow(&c.local, n0, n_new, e->st)) || (rc = grow(&c.base, n0, n_new, e->st)) ||
-        (rc = grow(&c.t, n0, n_new, e->st)) || (rc = grow(&c.ev, n0, n_new, e->st)) ||
-        (rc = grow(&c.dt_prev, n0, n_new, e->st)) || (rc = grow(&c.next_sample, n0, n_new, e->st)) ||
-        (rc = grow(&c.ev_stop, n0, n_new, e->st)) || (rc = grow(&c.zsum, n0, n_new, e->st)) ||
-        (rc = grow(&c.R1, 3 * (int64_t)n0, 3 * (int64_t)n_new, e->st)))
+    if ((rc = grow(e, &c.Z, n0, n_new)) || (rc = grow(e, &c.nk, n0, n_new)) ||
+        (rc = grow(e, &c.ens, n0, n_new)) || (rc = grow(e, &c.cap, n0, n_new)) ||
+        (rc = grow(e, &c.stall, n0, n_new)) || (rc = grow(e, &c.cid, n0, n_new)) ||
+        (rc = grow(e, &c.local, n0, n_new)) || (rc = grow(e, &c.base, n0, n_new)) ||
+        (rc = grow(e, &c.t, n0, n_new)) || (rc = grow(e, &c.ev, n0, n_new)) ||
+        (rc = grow(e, &c.dt_prev, n0, n_new)) || (rc = grow(e, &c.next_sample, n0, n_new)) ||
+        (rc = grow(e, &c.ev_stop, n0, n_new)) || (rc = grow(e, &c.zsum, n0, n_new)) ||
+        (rc = grow(e, &c.R1, 3 * (int64_t)n0, 3 * (int64_t)n_new)))
       return rc;
     e->nch = n_new;
   }
   if (s_need > e->nstr) {
     const int64_t s0 = e->nstr;
     const int64_t s_new = grown_capacity(s0, s_need, kStrandBytes);
-    if ((rc = grow(&c.Qx, s0, s_new, e->st)) || (rc = grow(&c.Qy, s0, s_new, e->st)) ||
-        (rc = grow(&c.Qz, s0, s_new, e->st)) || (rc = grow(&c.N, s0, s_new, e->st)) ||
-        (rc = grow(&c.w, s0, s_new, e->st)))
+    if ((rc = grow(e, &c.Qx, s0, s_new)) || (rc = grow(e, &c.Qy, s0, s_new)) ||
+        (rc = grow(e, &c.Qz, s0, s_new)) || (rc = grow(e, &c.N, s0, s_new)) ||
+        (rc = grow(e, &c.w, s0, s_new)))
       return rc;
     e->nstr = s_new;
   }
@@ -621,7 +639,7 @@ int ensure_stage(dsm_engine* e) {
   if (e->stage_space.end > e->d_stage_cap) {  // keeps the rows of live ensembles (last_samples)
     e->gen++;
     const int64_t cap = grown_capacity(e->d_stage_cap, e->stage_space.end, sizeof(float));
-    int rc = grow(&e->d_stage, e->d_stage_cap, cap, e->st);
+    int rc = grow(e, &e->d_stage, e->d_stage_cap, cap);
     if (rc) return rc;
     e->d_stage_cap = cap;
   }
@@ -735,18 +753,11 @@ bool solo_flow_capable(const dsm_engine* e, const std::vector<int>& ids) {
   return flow && e->opt.solo != 0;
 }
 
-// Its working memory: a record per strand slot, allocated when a pass first can use it,
-// and its rate tables for short strands.  It gives way to anything else: not taken beyond
-// a quarter of the free device memory, and given back when an allocation fails (the other
-// forms then run).
-void release_lane(dsm_engine* e) {
-  if (!e->d_rec) return;
-  e->gen++;
-  (void)hipStreamSynchronize(e->st);
-  (void)hipFree(e->d_rec);
-  e->d_rec = nullptr;
-  e->d_rec_cap = 0;
-}
+// The lane form's working memory: a record per strand slot, allocated when a pass first can
+// use it, and its rate tables for short strands (the solo forms', too).  The records give way
+// to anything else: not taken beyond a quarter of the free device memory, and given back when
+// an allocation of the engine would fail (dev_alloc).  Where either cannot be had, the other
+// forms run.
 int ensure_lane(dsm_engine* e, const std::vector<int>& ids) {
   const bool lanes = lane_quads(e, ids) || lane_share(e, ids);
   if (!lanes && !solo_capable(e, ids) && !flow_cap(e, ids) && !solo_flow_capable(e, ids)) return DSM_OK;
@@ -757,9 +768,14 @@ int ensure_lane(dsm_engine* e, const std::vector<int>& ids) {
     for (int N = 1; N < kLaneN; ++N)
       for (int q = 0; q < 4; ++q) out[4 * N + q] = t[(size_t)q * n + N];
     for (int x = 1; x < kLaneFR; ++x) out[4 * kLaneN + x] = 4.0f / (float)x;  // (build_tables' FR)
-    int rc = dev_alloc(&e->d_lane_tab, out.size());
-    if (rc) return rc;
-    HIPCHK(hipMemcpy(e->d_lane_tab, out.data(), sizeof(float) * out.size(), hipMemcpyHostToDevice));
+    float* tab = nullptr;
+    if (dev_alloc(e, &tab, out.size())) return DSM_OK;
+    const hipError_t he = hipMemcpy(tab, out.data(), sizeof(float) * out.size(), hipMemcpyHostToDevice);
+    if (he != hipSuccess) {
+      (void)hipFree(tab);
+      return fail(DSM_ERR_DEVICE, "rate tables: %s", hipGetErrorString(he));
+    }
+    e->d_lane_tab = tab;
   }
   if (lanes && e->nstr > e->d_rec_cap) {
     release_lane(e);
@@ -796,7 +812,7 @@ int corr_alloc(dsm_engine* e, Ens& E, int s) {
   corr_free(E);
   const size_t n = (size_t)E.n, nD = (size_t)s * E.p * 3 * n, nA = (size_t)s * 3 * n, nC = (size_t)s * E.p * n;
   int rc;
-  if ((rc = dev_alloc(&E.dD, nD)) || (rc = dev_alloc(&E.dA, nA)) || (rc = dev_alloc(&E.dC, nC))) {
+  if ((rc = dev_alloc(e, &E.dD, nD)) || (rc = dev_alloc(e, &E.dA, nA)) || (rc = dev_alloc(e, &E.dC, nC))) {
     corr_free(E);
     return rc;
   }
@@ -910,7 +926,8 @@ int pass_setup(dsm_engine* e, const std::vector<int>& ids, bool use_ev_stop, Pas
   ps.bin_max = bin_max;
   ps.n_ens = (int)ids.size();
   ps.n_live = (int)n_all;
-  ps.lane_quads = batched && e->d_rec_cap >= e->nstr ? lane_quads(e, ids) : 0;
+  const bool records = batched && e->d_lane_tab && e->d_rec && e->d_rec_cap >= e->nstr;
+  ps.lane_quads = records ? lane_quads(e, ids) : 0;
   ps.solo = batched && e->d_lane_tab && solo_capable(e, ids);
   ps.nmax = 0;
   for (int id : ids) ps.nmax = std::max(ps.nmax, e->ens[id].nmax);
@@ -922,7 +939,7 @@ int pass_setup(dsm_engine* e, const std::vector<int>& ids, bool use_ev_stop, Pas
   ps.flow_cap = batched && e->d_lane_tab ? flow_cap(e, ids) : 0;
   if (ps.lane_quads || ps.flow_cap) ps.concurrent = false;
   ps.solo_flow = batched && !ps.concurrent && e->d_lane_tab && solo_flow_capable(e, ids);
-  ps.n_lane = ps.concurrent && batched && e->d_rec_cap >= e->nstr ? lane_share(e, ids) : 0;
+  ps.n_lane = ps.concurrent && records ? lane_share(e, ids) : 0;
   if (n0 == 0) return DSM_OK;
   ps.range = batched && !ps.concurrent && ids.size() == 1;
   ps.first = e->ens[ids[0]].chain0;
@@ -1393,11 +1410,7 @@ int advance_impl(dsm_engine* e, const std::vector<int>& ids, const std::vector<d
         if (s <= 0) s = (int)std::ceil(std::log(te / E.P.delta / E.p) / std::log((double)E.m)) + 1;
         if (s < 1) s = 1;
         if (s > 40) return fail(DSM_ERR_ARG, "correlator needs %d levels (max 40)", s);
-        if ((rc = corr_alloc(e, E, s))) {
-          if (rc != DSM_ERR_MEMORY || !e->d_rec) return rc;
-          release_lane(e);
-          if ((rc = corr_alloc(e, E, s))) return rc;
-        }
+        if ((rc = corr_alloc(e, E, s))) return rc;
       }
     } else if (E.P.sample_mode == kSampleFlow) {
       k_target[q] = (int64_t)std::ceil(te / E.P.delta - 1e-12) + 1;
@@ -1573,8 +1586,8 @@ int dsm_create(int32_t device_id, dsm_engine** out) {
   HIPCHK(hipEventCreateWithFlags(&e->ev_split, hipEventDisableTiming));
   for (auto& ev : e->ev_bin) HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
   int rc;
-  if ((rc = dev_alloc(&e->d_cnt, 2 * kNumLists + kZOrderScratch + 1)) || (rc = dev_alloc(&e->d_counters, kNumCounters)) ||
-      (rc = dev_alloc(&e->d_part, (size_t)kStressBlocks * 9)) || (rc = window_grow(e, 0))) {
+  if ((rc = dev_alloc(e, &e->d_cnt, 2 * kNumLists + kZOrderScratch + 1)) || (rc = dev_alloc(e, &e->d_counters, kNumCounters)) ||
+      (rc = dev_alloc(e, &e->d_part, (size_t)kStressBlocks * 9)) || (rc = window_grow(e, 0))) {
     dsm_destroy(e);
     return rc;
   }
@@ -1746,26 +1759,14 @@ int dsm_add_ensemble(dsm_engine* e, const dsm_ensemble_desc* d, int32_t* ens_id)
   if (E.p % E.m != 0 && eq_sampling(d->sample_mode)) return fail(DSM_ERR_ARG, "corr_p must be a multiple of corr_m");
   E.stage_floats = ((int64_t)E.window * E.n * E.ncomp + 3) & ~(int64_t)3;  // rows start on 16 bytes
   P.stage_off = e->stage_space.take(E.stage_floats);
-  if ((rc = ensure_stage(e))) {
-    if (rc != DSM_ERR_MEMORY || !e->d_rec) return rc;
-    release_lane(e);
-    if ((rc = ensure_stage(e))) return rc;
-  }
+  if ((rc = ensure_stage(e))) return rc;
   // chains
   E.chain0 = (int)e->chain_space.take(E.n);
   E.nstrand = 0;
   for (int i = 0; i < E.n; ++i) E.nstrand += cap_of(E.nk[i]);
   P.chain0 = E.chain0;
   E.strand0 = e->strand_space.take(E.nstrand);
-  auto room = [&]() {
-    const int r = grow_chains(e, (int)e->chain_space.end, e->strand_space.end);
-    return r ? r : ensure_work(e, 1);
-  };
-  if ((rc = room())) {
-    if (rc != DSM_ERR_MEMORY || !e->d_rec) return rc;
-    release_lane(e);
-    if ((rc = room())) return rc;
-  }
+  if ((rc = grow_chains(e, (int)e->chain_space.end, e->strand_space.end)) || (rc = ensure_work(e, 1))) return rc;
   {
     const int id = (int)e->ens.size();
     std::vector<int> hnk(E.n), hens(E.n, id), hcap(E.n), hzero(E.n, 0), hloc(E.n);

@@ -57,7 +57,9 @@ int corr_levels(double horizon) {
 }
 
 // device bytes of one request: strand records, per-chain header, sample staging and,
-// for G(t), the FP64 correlator registers
+// for G(t), the FP64 correlator registers.  (The lane form's records, 12 bytes a strand slot,
+// are not among them: the engine takes them out of a quarter of what is left free and gives
+// them back for a request.)
 int64_t estimate_bytes(const Req& r, double horizon) {
   const int64_t n = r.nch, cap = (r.nk + 3) & ~3;
   int64_t b = n * cap * 20 + n * 96;

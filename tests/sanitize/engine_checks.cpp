@@ -132,6 +132,70 @@ static void check_alloc() {
   CHECK(fake::live_bytes == 0);
 }
 
+// ------------------------------------------------------------------ the lane form's records give way
+// With the records in memory, no single failed allocation is the caller's: they are given
+// back for it, and the next pass takes them again or runs without.
+static int64_t lanes_session(int64_t k, bool* ran) {
+  dsm_engine* e = nullptr;
+  CHECK(dsm_create(0, &e) == DSM_OK);
+  CHECK(dsm_set_option(e, DSM_OPT_LANE, 2) == DSM_OK && dsm_set_option(e, DSM_OPT_SMALL_PER_CU, 0) == DSM_OK);
+  int32_t id = -1, fl = -1, more = -1;
+  dsm_ensemble_desc d = desc(100, 30, DSM_SAMPLE_GT), f = desc(5000, 40, DSM_SAMPLE_FLOW), x = desc(700, 50, DSM_SAMPLE_MSD);
+  x.partner_mode = DSM_PARTNER_MELT;
+  CHECK(dsm_add_ensemble(e, &d, &id) == DSM_OK && dsm_init_equilibrium(e, id) == DSM_OK);
+  auto run = [&](int32_t i, double t) { CHECK(dsm_advance(e, i, t, DSM_MODE_BATCHED, nullptr, nullptr, nullptr) == DSM_OK); };
+  fake::launches.clear();
+  fake::nulls = 0;
+  run(id, 3.0);
+  *ran = fake::launches[0].name == "lane";
+  const int64_t a0 = fake::allocs;
+  if (k > 0) fake::fail_next(k);
+  double lag[80], g[80];
+  int32_t np = 0;
+  CHECK(dsm_correlator(e, id, 80, lag, g, &np) == DSM_OK);
+  CHECK(dsm_add_ensemble(e, &f, &fl) == DSM_OK && dsm_init_equilibrium(e, fl) == DSM_OK);
+  run(fl, 6.0);
+  CHECK(dsm_add_ensemble(e, &x, &more) == DSM_OK && dsm_init_equilibrium(e, more) == DSM_OK);
+  run(more, 6.0);
+  for (int i = 0; i < 16; ++i) {
+    int32_t j = -1;
+    d.salt = (uint32_t)i + 1;
+    CHECK(dsm_add_ensemble(e, &d, &j) == DSM_OK && dsm_init_equilibrium(e, j) == DSM_OK);
+    run(j, 3.0);
+  }
+  fake::fail_none();
+  fake::launches.clear();
+  run(id, 9.0);
+  CHECK(fake::launches[0].name == "lane" && fake::nulls == 0);
+  const int64_t n = fake::allocs - a0;
+  dsm_destroy(e);
+  CHECK(fake::live_bytes == 0);
+  return n;
+}
+static void check_lanes() {
+  bool ran = false;
+  const int64_t n = lanes_session(0, &ran);
+  CHECK(ran && n > 40);
+  for (int64_t k = 1; k <= n && failures < 20; ++k) lanes_session(k, &ran);
+  int without = 0;
+  for (int64_t k = 1; k <= 6; ++k) {
+    dsm_engine* e = nullptr;
+    CHECK(dsm_create(0, &e) == DSM_OK);
+    dsm_set_option(e, DSM_OPT_LANE, 2);
+    dsm_set_option(e, DSM_OPT_SMALL_PER_CU, 0);
+    int32_t id = -1;
+    dsm_ensemble_desc d = desc(100, 30, DSM_SAMPLE_NONE);
+    CHECK(dsm_add_ensemble(e, &d, &id) == DSM_OK && dsm_init_equilibrium(e, id) == DSM_OK);
+    fake::launches.clear();
+    fake::fail_next(k);
+    CHECK(dsm_advance(e, id, 3.0, DSM_MODE_BATCHED, nullptr, nullptr, nullptr) == DSM_OK);
+    without += fake::launches[0].name != "lane";
+    fake::fail_none();
+    dsm_destroy(e);
+  }
+  CHECK(without == 2);  // the tables or the records: the other forms run
+}
+
 // ------------------------------------------------------------------ refused stays refused
 static void check_refused() {
   dsm_engine* e = nullptr;
@@ -158,6 +222,7 @@ int main(int argc, char** argv) {
   const std::string which = argc > 1 ? argv[1] : "";
   if (which == "alloc") check_alloc();
   else if (which == "refused") check_refused();
+  else if (which == "lanes") check_lanes();
   else return 2;
   std::printf("engine checks (%s): %d failures\n", which.c_str(), failures);
   return failures ? 1 : 0;

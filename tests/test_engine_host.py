@@ -44,3 +44,9 @@ def test_every_allocation_may_fail(checks):
 def test_a_refused_ensemble_is_refused_again(checks):
     """A GEX background without quantiles, and a block factor that does not divide the lags."""
     checks("refused")
+
+
+def test_lane_records_give_way(checks):
+    """With the lane form's records in memory, any one failed allocation is made good by giving
+    them back; without its tables or records a pass runs in the other forms."""
+    checks("lanes")
