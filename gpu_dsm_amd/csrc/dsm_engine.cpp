@@ -855,11 +855,13 @@ struct Timer {
   }
 };
 
+// Persistent waves of a launch: as many a CU as fit, at most DSM_OPT_BLOCKS_PER_CU.
+int device_waves(const dsm_engine* e, int per_cu) {
+  if (e->opt.blocks_per_cu > 0) per_cu = std::min(per_cu, e->opt.blocks_per_cu);
+  return std::max(per_cu, 1) * e->n_cu;
+}
 int device_blocks(dsm_engine* e, int geom, bool plain, int lds_floats, bool ext) {
-  int nb = kmc_max_blocks_per_cu(geom, plain, lds_floats, ext);
-  if (e->opt.blocks_per_cu > 0) nb = std::min(nb, e->opt.blocks_per_cu);
-  if (nb <= 0) nb = 1;
-  return nb * e->n_cu;
+  return device_waves(e, kmc_max_blocks_per_cu(geom, plain, lds_floats, ext));
 }
 
 KmcArgs base_args(dsm_engine* e) {
@@ -970,11 +972,11 @@ int late_last(int bin_max) { return std::max(bin_max, kLateFirst); }
 hipError_t launch_wave(dsm_engine* e, const Pass& ps, const KmcArgs& a, int b, int geom, hipStream_t st) {
   if (ps.solo_flow && b <= 3) {
     const int cap = kmc_geom_capacity(b);
-    return launch_kmc_solo_flow(a, cap, std::min(ps.n0, kmc_solo_flow_occupancy(cap) * e->n_cu), st);
+    return launch_kmc_solo_flow(a, cap, std::min(ps.n0, device_waves(e, kmc_solo_flow_occupancy(cap))), st);
   }
   if (!ps.solo) return launch_kmc(a, geom, false, device_blocks(e, geom, false, a.lds_floats, a.ext != 0), st);
   const int cap = kmc_geom_capacity(b);
-  return launch_kmc_solo(a, cap, std::min(ps.n0, kmc_solo_occupancy(cap) * e->n_cu), st);
+  return launch_kmc_solo(a, cap, std::min(ps.n0, device_waves(e, kmc_solo_occupancy(cap))), st);
 }
 
 // Lanes of each of `waves` waves for n chains: as many, to `most`, as give every wave the
@@ -983,8 +985,17 @@ int even_lanes(int n, int most, int waves) {
   const int rounds = (n + waves * most - 1) / (waves * most);
   return std::max(1, (n + waves * rounds - 1) / (waves * rounds));
 }
-int lane_lanes(const dsm_engine* e, int quads, int n) {
-  return even_lanes(n, lane_max_lanes(quads), kLaneWaves * e->n_cu);
+// Workgroups of a launch of `waves` waves a workgroup, one a CU, and the lanes of its waves.
+int lane_groups(const dsm_engine* e, int waves) { return std::max(1, device_waves(e, waves) / waves); }
+hipError_t launch_lanes(const dsm_engine* e, KmcArgs a, int quads, int n, hipStream_t st) {
+  const int groups = lane_groups(e, kLaneWaves);
+  a.lanes = even_lanes(n, lane_max_lanes(quads), kLaneWaves * groups);
+  return launch_kmc_lane(a, quads, groups, st);
+}
+hipError_t launch_flow_lanes(const dsm_engine* e, KmcArgs a, int cap, int n, hipStream_t st) {
+  const int groups = lane_groups(e, kFlowWaves);
+  a.lanes = even_lanes(n, flow_max_lanes(cap), kFlowWaves * groups);
+  return launch_kmc_lane_flow(a, cap, groups, st);
 }
 
 // Batched pass with the geometries side by side: the chains are split by their current
@@ -1022,8 +1033,7 @@ int pass_bins_concurrent(dsm_engine* e, Pass& ps, dsm_run_stats* rs) {
     HIPCHK(launch_z_order(list(kSplitList), 0, ps.n0, e->ch.Z, e->ch.stall, kLaneMaxQuads / 4, cnt + 2 * kNumLists,
                           list(0), cnt, e->st));
     bind(0, late_of(0));
-    a.lanes = lane_lanes(e, kLaneMaxQuads, ps.n_lane);
-    HIPCHK(launch_kmc_lane(a, kLaneMaxQuads, e->n_cu, e->st));
+    HIPCHK(launch_lanes(e, a, kLaneMaxQuads, ps.n_lane, e->st));
     ++rs->kmc_launches;
   }
   HIPCHK(hipEventRecord(e->ev_split, e->st));
@@ -1074,10 +1084,9 @@ int pass_bins_concurrent(dsm_engine* e, Pass& ps, dsm_run_stats* rs) {
   const KmcArgs pair_args = a;
   bind(kSplitList, late_of(0));
   if (ps.n_lane) a.n_work = cnt + kEmpty;
-  int nb = kmc_rowpair_occupancy(a.lds_floats, a.ext != 0, wide);
-  if (e->opt.blocks_per_cu > 0) nb = std::min(nb, e->opt.blocks_per_cu);
   if (timed) HIPCHK(hipEventRecord(e->cev[1], e->xs[2]));
-  HIPCHK(launch_kmc_rowpair(a, pair_args, wide, std::max(nb, 1) * e->n_cu, e->xs[2]));
+  HIPCHK(launch_kmc_rowpair(a, pair_args, wide, device_waves(e, kmc_rowpair_occupancy(a.lds_floats, a.ext != 0, wide)),
+                            e->xs[2]));
   if (timed) HIPCHK(hipEventRecord(e->cev[2], e->xs[2]));
   // bins 0 and 1 are the only feeders of the first late list, complete when
   // their launch ends: its run follows on the same stream, beside the other geometries'
@@ -1157,11 +1166,9 @@ int pass_bins(dsm_engine* e, Pass& ps, bool plain, bool timed, dsm_run_stats* rs
     a.n_overflow = cnt + nb;
     if (timed) HIPCHK(hipEventRecord(e->lev[2 * k], e->st));
     if (k == 0 && flow) {
-      a.lanes = even_lanes(ps.n_live, flow_max_lanes(ps.flow_cap), kFlowWaves * e->n_cu);
-      HIPCHK(launch_kmc_lane_flow(a, ps.flow_cap, e->n_cu, e->st));
+      HIPCHK(launch_flow_lanes(e, a, ps.flow_cap, ps.n_live, e->st));
     } else if (k == 0 && lane) {
-      a.lanes = lane_lanes(e, ps.lane_quads, ps.n_live);
-      HIPCHK(launch_kmc_lane(a, ps.lane_quads, e->n_cu, e->st));
+      HIPCHK(launch_lanes(e, a, ps.lane_quads, ps.n_live, e->st));
     } else if (!plain && b >= kLateFirst) {
       HIPCHK(launch_wave(e, ps, a, b, b, e->st));
     } else {

@@ -196,6 +196,62 @@ static void check_lanes() {
   CHECK(without == 2);  // the tables or the records: the other forms run
 }
 
+// ------------------------------------------------------------------ options
+struct Run {  // one pass of `n` chains a piece of the ensembles given, the options set
+  std::vector<fake::Launch> l;
+  Run(const std::vector<dsm_ensemble_desc>& ds, const std::vector<std::pair<int, int>>& opts, double t = 3.0) {
+    dsm_engine* e = nullptr;
+    CHECK(dsm_create(0, &e) == DSM_OK);
+    for (auto& o : opts) CHECK(dsm_set_option(e, o.first, o.second) == DSM_OK);
+    std::vector<int32_t> ids;
+    for (auto& d : ds) {
+      int32_t id = -1;
+      CHECK(dsm_add_ensemble(e, &d, &id) == DSM_OK && dsm_init_equilibrium(e, id) == DSM_OK);
+      ids.push_back(id);
+    }
+    fake::launches.clear();
+    fake::nulls = 0;
+    const std::vector<double> te(ids.size(), t);
+    CHECK(dsm_advance_many(e, ids.data(), te.data(), (int32_t)ids.size(), DSM_MODE_BATCHED, nullptr, nullptr) == DSM_OK);
+    CHECK(fake::nulls == 0 && !fake::launches.empty());
+    l = fake::launches;
+    dsm_destroy(e);
+  }
+  bool has(const char* name) const {
+    for (auto& x : l)
+      if (x.name == name) return true;
+    return false;
+  }
+  const std::string& first() const { return l[0].name; }
+};
+
+static const int kCu = 256;
+
+static void check_waves() {
+  // DSM_OPT_BLOCKS_PER_CU bounds the waves of every form
+  const std::vector<std::vector<dsm_ensemble_desc>> passes = {
+      {desc(40000, 60, DSM_SAMPLE_GT)},                                   // lanes, then solo
+      {desc(40000, 60, DSM_SAMPLE_FLOW)},                                 // row
+      {desc(70000, 25, DSM_SAMPLE_FLOW)},                                 // lanes under flow
+      {desc(2000, 100, DSM_SAMPLE_GT)},                                   // solo
+      {desc(2000, 100, DSM_SAMPLE_FLOW)},                                 // solo under flow
+      {desc(3500, 700, DSM_SAMPLE_GT)},                                   // concurrent
+      {desc(3500, 700, DSM_SAMPLE_GT), desc(3500, 600, DSM_SAMPLE_FLOW)}  // concurrent with flow
+  };
+  std::string seen;
+  for (auto& ds : passes)
+    for (int cap : {1, 2, 3, 8, 12, 100}) {
+      const Run r(ds, {{DSM_OPT_BLOCKS_PER_CU, cap}, {DSM_OPT_LANE, 2}});
+      for (auto& x : r.l) {
+        const int per = x.name.rfind("lane", 0) == 0 ? 8 : 1;
+        if (x.grid * per > cap * kCu) std::fprintf(stderr, "%s %d: %d waves\n", x.name.c_str(), x.size, x.grid * per);
+        CHECK(x.grid >= 1 && x.grid * per <= cap * kCu);
+        seen += " " + x.name;
+      }
+    }
+  for (const char* f : {"lane", "lane_flow", "solo", "solo_flow", "rowpair", "wave"}) CHECK(seen.find(f) != std::string::npos);
+}
+
 // ------------------------------------------------------------------ refused stays refused
 static void check_refused() {
   dsm_engine* e = nullptr;
@@ -223,6 +279,7 @@ int main(int argc, char** argv) {
   if (which == "alloc") check_alloc();
   else if (which == "refused") check_refused();
   else if (which == "lanes") check_lanes();
+  else if (which == "waves") check_waves();
   else return 2;
   std::printf("engine checks (%s): %d failures\n", which.c_str(), failures);
   return failures ? 1 : 0;

@@ -50,3 +50,7 @@ def test_lane_records_give_way(checks):
     """With the lane form's records in memory, any one failed allocation is made good by giving
     them back; without its tables or records a pass runs in the other forms."""
     checks("lanes")
+
+
+def test_waves_per_cu_are_bounded_in_every_form(checks):
+    checks("waves")
