@@ -939,6 +939,7 @@ int pass_setup(dsm_engine* e, const std::vector<int>& ids, bool use_ev_stop, Pas
   ps.concurrent = e->opt.concurrent >= 0 ? (e->opt.concurrent > 0 && bin_max >= 1)
                                          : (bin_max >= 3 || (bin_max >= 1 && z_est >= 56.0 * n_all));
   ps.flow_cap = batched && e->d_lane_tab ? flow_cap(e, ids) : 0;
+  if (e->opt.concurrent > 0 && ps.concurrent) ps.lane_quads = ps.flow_cap = 0;  // (asked for)
   if (ps.lane_quads || ps.flow_cap) ps.concurrent = false;
   ps.solo_flow = batched && !ps.concurrent && e->d_lane_tab && solo_flow_capable(e, ids);
   ps.n_lane = ps.concurrent && records ? lane_share(e, ids) : 0;

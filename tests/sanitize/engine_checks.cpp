@@ -252,6 +252,21 @@ static void check_waves() {
   for (const char* f : {"lane", "lane_flow", "solo", "solo_flow", "rowpair", "wave"}) CHECK(seen.find(f) != std::string::npos);
 }
 
+static void check_concurrent() {
+  // DSM_OPT_CONCURRENT = 1: side by side wherever a chain can leave the row form, the short
+  // ones in lanes first; 0: never
+  for (int lane : {0, 1, 2}) {
+    const std::vector<std::pair<int, int>> always = {{DSM_OPT_CONCURRENT, 1}, {DSM_OPT_LANE, lane}};
+    const Run still({desc(50000, 100, DSM_SAMPLE_GT)}, always), flow({desc(20000, 70, DSM_SAMPLE_FLOW, 3.0f)}, always);
+    CHECK(still.has("rowpair") && flow.has("rowpair"));
+    CHECK(still.has("lane") == (lane > 0) && !flow.has("lane_flow"));
+    const Run in_turn({desc(50000, 700, DSM_SAMPLE_GT)}, {{DSM_OPT_CONCURRENT, 0}, {DSM_OPT_LANE, lane}});
+    CHECK(!in_turn.has("rowpair"));
+  }
+  const Run by_itself({desc(50000, 100, DSM_SAMPLE_GT)}, {});
+  CHECK(by_itself.first() == "lane" && !by_itself.has("rowpair"));
+}
+
 // ------------------------------------------------------------------ refused stays refused
 static void check_refused() {
   dsm_engine* e = nullptr;
@@ -280,6 +295,7 @@ int main(int argc, char** argv) {
   else if (which == "refused") check_refused();
   else if (which == "lanes") check_lanes();
   else if (which == "waves") check_waves();
+  else if (which == "concurrent") check_concurrent();
   else return 2;
   std::printf("engine checks (%s): %d failures\n", which.c_str(), failures);
   return failures ? 1 : 0;

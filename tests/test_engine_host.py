@@ -54,3 +54,7 @@ def test_lane_records_give_way(checks):
 
 def test_waves_per_cu_are_bounded_in_every_form(checks):
     checks("waves")
+
+
+def test_concurrent_option_is_obeyed(checks):
+    checks("concurrent")
