@@ -657,28 +657,67 @@ double equilibrium_room(const Ens& E) {
   return std::min(nk, (nk + b) / (1.0 + b) + 5.0 * std::sqrt((nk - 1.0) * b) / (1.0 + b));
 }
 
+// An ensemble's mean equilibrium Z, and the mean length of its strands.
+double mean_z(const Ens& E) { return E.z_sum_est / E.n; }
+double mean_strand(const Ens& E) { return 1.0 + E.P.beta - E.P.beta / mean_z(E); }
+
+// Jumps of a chain between two of its samples (infinite: none are taken), from the rates at
+// equilibrium: b / (1 + b + b*b/3) a strand and tau_K, and what the chain ends add (within a
+// tenth of what was counted for b = beta 1 to 30 and Nk 6 to 400, a quarter from 0.3).
+double jumps_per_sample(const Ens& E) {
+  if (E.P.sample_mode == kSampleNone) return INFINITY;
+  const double b = E.P.beta;
+  return (mean_z(E) * b / (1.0 + b + b * b / 3.0) + 3.6 / (1.0 + b * b)) * E.P.delta;
+}
+
+// How many chains of an ensemble the lane form needs to one of an ordinary one (beta 1, a
+// sample every ten jumps or more).
+//   Long strands: a pair beyond the form's tables sends a wave to the ensemble's own (`steep`
+//     a Kuhn step of the mean length above three).  130,000 chains of Nk 100 at beta 1 4.68
+//     against 2.66 ms, 90,000 of Nk 400 at beta 12 2.74 / 2.50; 40,000 of Nk 60 at beta 6 and 12
+//     2.4 / 3.4 and 1.4 / 2.4.
+//   Samples: the row form has a chain's vectors in registers, a lane's chain gathers them from
+//     memory, the more the longer it is, an MSD sample three times over.  131,072 chains of Nk
+//     100, G(t) every 1, 0.3, 0.1 and 0.03 tau_K (22 to 0.7 jumps): 6.7 / 3.7, 7.3 / 5.2, 8.9
+//     / 9.8, 15.2 / 26.4 ms; MSD every 1, 0.3, 0.1: 8.0 / 4.8, 9.3 / 8.9, 12.1 / 20.5.  With
+//     fewer than about 1.3 jumps to a sample no count pays.
+//   Below beta 1 a third more jumps split or merge strands (40,000 of Nk 50, beta 0.3: level).
+// Over 1,800 combinations of Nk 6 to 2000, beta 0.3 to 30, 10,000 to 250,000 chains and
+// delta 0.1 to 1 the routes taken are on average 1.4% slower than the better of the two, and
+// at worst 17% slower than without the lane form; by the number of chains alone they were 12%
+// and 94%.
+double lane_price(const Ens& E, double steep, double dense) {
+  double price = 1.0 + steep * std::max(0.0, mean_strand(E) - 3.0) + 0.2 * std::max(0.0, 1.0 - (double)E.P.beta);
+  const double per = jumps_per_sample(E) / ((1.0 + mean_z(E) / 120.0) * (E.P.sample_mode == kSampleMsd ? 1.6 : 1.0));
+  if (per < 1.3) return INFINITY;
+  return price * (1.0 + dense * std::max(0.0, 1.0 / per - 0.2));
+}
+
 // Quads per chain with which a batched pass over these ensembles runs in the lane form, or
 // 0 when it runs in the others.  The chains have to fit the largest size, 128 positions,
 // with five standard deviations of the equilibrium Z (binomial) to spare (one that outgrows
 // the size chosen finishes in the wave form).
 int lane_quads(const dsm_engine* e, const std::vector<int>& ids) {
   if (e->opt.lane == 0 || ids.empty()) return 0;
-  double n = 0.0, zcap = 0.0;
+  double n = 0.0, z = 0.0, worth = 0.0, zcap = 0.0;
   for (int id : ids) {
     const Ens& E = e->ens[id];
     if (!lane_capable(E)) return 0;
     n += E.n;
+    z += E.z_sum_est;
+    worth += E.n / lane_price(E, 0.125, 2.0);
     zcap = std::max(zcap, equilibrium_room(E));
   }
   int quads = 0;
   for (int q : kLaneQuads)
     if (4 * q > zcap) { quads = q; break; }
-  // A wave's step costs nearly the same for one chain as for 64, so the form needs chains:
-  // it passes the row form (four chains a wave) at about 32,000 chains (one 16 tau_K window,
-  // Nk 100: 3.36 against 3.38 ms; 24,000: 3.14 / 2.72; 48,000: 3.63 / 4.58; Nk 50 at about
-  // 38,000, Nk 25 at 30,000) and the pair form (two a wave, from Z = 64 on) at about 14,000
-  // (Nk 150: 4.38 against 4.90 ms at 16,000).
-  if (e->opt.lane == 1 && n < (quads >= 24 ? 14000 : 36000)) return 0;
+  // A wave's step costs nearly the same for one chain as for 64, so the form needs chains: it
+  // passes the row form (four chains a wave) at about 36,000 chains (one 16 tau_K window, Nk
+  // 100: 3.36 against 3.38 ms at 32,000; 24,000: 3.14 / 2.72; 48,000: 3.63 / 4.58; Nk 50 at about
+  // 38,000, Nk 25 at 30,000), the pair form (two a wave, from Z = 64 on) at about 14,000 (Nk
+  // 150: 4.38 against 4.90 ms at 16,000), and where some of the chains leave the row form for a
+  // pass of their own at 20,000 (Nk 150, beta 2).
+  if (e->opt.lane == 1 && worth < (quads < 24 ? 36000 : z < 60.0 * n ? 22000 : 14000)) return 0;
   return quads;
 }
 
@@ -714,17 +753,24 @@ int flow_cap(const dsm_engine* e, const std::vector<int>& ids) {
 // positions (Nk 200, 8 tau_K) 3.54 ms without against 4.29 ms with 15,000 such chains, 6.24 /
 // 4.81 with 30,000, 11.2 / 5.5 with 60,000; with longer ones (the polydisperse melt, 16
 // tau_K) 18.4 / 22.8 with 46,000, 26.1 / 27.0 with 69,000, 33.8 / 32.4 with 92,000, 64 / 58
-// with 184,000.
+// with 184,000.  Long strands and samples cost it more here (lane_price): the same melt at
+// beta 3, 90,000 and 200,000 chains: 4.8 / 6.0 and 5.3 / 4.5 ms, MSD every 0.3 tau_K 5.6 / 8.4
+// and 5.6 / 6.2; at beta 8 4.5 / 7.0 and 3.9 / 4.2.  Nk 200 at beta 8, 24,000 and 90,000: 2.1 /
+// 2.9 and 3.5 / 2.0.
 int lane_share(const dsm_engine* e, const std::vector<int>& ids) {
   if (e->opt.lane == 0) return 0;
-  int64_t n = 0;
   bool longer = false;
   for (int id : ids) {
     if (!lane_capable(e->ens[id])) return 0;
-    n += e->ens[id].n_lane;
     longer = longer || e->ens[id].bin_max >= 3;
   }
-  return e->opt.lane == 2 || n >= (longer ? 80000 : 22000) ? (int)n : 0;
+  int64_t n = 0;
+  double worth = 0.0;
+  for (int id : ids) {
+    n += e->ens[id].n_lane;
+    worth += e->ens[id].n_lane / lane_price(e->ens[id], longer ? 0.8 : 0.3, 3.0);
+  }
+  return e->opt.lane == 2 || worth >= (longer ? 80000 : 22000) ? (int)n : 0;
 }
 
 // The solo form (dsm_solo.h) takes the place of the wave forms (bins 2 and up) wherever no

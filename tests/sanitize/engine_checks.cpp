@@ -267,6 +267,50 @@ static void check_concurrent() {
   CHECK(by_itself.first() == "lane" && !by_itself.has("rowpair"));
 }
 
+// ------------------------------------------------------------------ routes
+static dsm_ensemble_desc every(dsm_ensemble_desc d, double delta) {
+  d.delta = delta;
+  return d;
+}
+// Which form takes the chains of a pass; the times beside a case are its former route's and
+// the lane form's, in ms.
+static void check_lane_route() {
+  const int GT = DSM_SAMPLE_GT, MSD = DSM_SAMPLE_MSD, NONE = DSM_SAMPLE_NONE;
+  auto lanes = [](const std::vector<dsm_ensemble_desc>& ds) { return Run(ds, {}, 0.01).has("lane"); };
+  CHECK(lanes({desc(131072, 100, GT)}));                  // 9.1 / 5.2
+  CHECK(lanes({desc(131072, 100, MSD)}));                 // 8.0 / 4.8
+  CHECK(lanes({desc(50021, 150, GT)}));                   // 5.7 / 2.7
+  CHECK(lanes({desc(262144, 12, GT)}));                   // 16.5 / 10.2
+  CHECK(lanes({desc(40000, 50, GT)}));                    // 1.07 times as fast
+  CHECK(lanes({desc(131072, 100, NONE, 6.0f)}));
+  CHECK(lanes({desc(70000, 100, GT), desc(70000, 60, GT)}));
+  // a sample costs the lane form several times what it costs the others
+  CHECK(!lanes({every(desc(131072, 100, GT), 0.03)}));    // 15.2 / 26.4
+  CHECK(!lanes({every(desc(131072, 100, MSD), 0.1)}));    // 12.1 / 20.5
+  CHECK(!lanes({every(desc(40000, 60, GT), 0.1)}));       // 12.8 / 15.7
+  CHECK(!lanes({desc(131072, 100, GT, 30.0f)}));          // 2.3 / 4.0 (0.4 jumps a sample)
+  // long strands
+  CHECK(!lanes({desc(40000, 1000, GT, 30.0f)}));          // 2.7 / 5.2
+  CHECK(!lanes({desc(40000, 60, GT, 6.0f)}));             // 2.4 / 3.4
+  CHECK(!lanes({desc(40000, 60, GT, 12.0f)}));            // 1.4 / 2.4
+  // of several ensembles, each counts by its own price
+  CHECK(!lanes({desc(20000, 100, GT), desc(100000, 100, GT, 30.0f)}));
+}
+static void check_share_route() {
+  // mixed lengths, the shorter chains in lanes first where they are many
+  auto mixed = [](int n, int sample, float beta, double delta) {
+    std::vector<int32_t> nk((size_t)n);
+    for (int i = 0; i < n; ++i) nk[(size_t)i] = i % 50 == 0 ? 900 : 30 + i % 170;
+    dsm_ensemble_desc d = every(desc(n, 900, sample, beta), delta);
+    d.nk_per_chain = nk.data();
+    return Run({d}, {}, 0.01).has("lane");
+  };
+  CHECK(mixed(200000, DSM_SAMPLE_GT, 1.0f, 1.0));         // the polydisperse melt's kind: 12.5 / 10.6
+  CHECK(!mixed(90000, DSM_SAMPLE_GT, 3.0f, 1.0));         // 4.8 / 6.0
+  CHECK(!mixed(200000, DSM_SAMPLE_MSD, 8.0f, 0.3));       // 5.3 / 8.4
+  CHECK(!mixed(200000, DSM_SAMPLE_GT, 20.0f, 1.0));       // 3.7 / 4.6
+}
+
 // ------------------------------------------------------------------ refused stays refused
 static void check_refused() {
   dsm_engine* e = nullptr;
@@ -296,6 +340,8 @@ int main(int argc, char** argv) {
   else if (which == "lanes") check_lanes();
   else if (which == "waves") check_waves();
   else if (which == "concurrent") check_concurrent();
+  else if (which == "route_lane") check_lane_route();
+  else if (which == "route_share") check_share_route();
   else return 2;
   std::printf("engine checks (%s): %d failures\n", which.c_str(), failures);
   return failures ? 1 : 0;

@@ -58,3 +58,9 @@ def test_waves_per_cu_are_bounded_in_every_form(checks):
 
 def test_concurrent_option_is_obeyed(checks):
     checks("concurrent")
+
+
+@pytest.mark.parametrize("rule", ["lane", "share"])
+def test_route(checks, rule):
+    """The form a pass runs in, where the two sides of the rule were measured well apart."""
+    checks("route_" + rule)
