@@ -725,25 +725,36 @@ int lane_quads(const dsm_engine* e, const std::vector<int>& ids) {
 // (dsm_lane_flow.h), or 0: to 40, at 2.75 standard deviations above the equilibrium Z (more
 // room costs lanes: at Nk 50 five per cent of the time each position; a chain that outgrows
 // it finishes in the wave form).  A lane's step costs its wave the same for one chain as for
-// 64, so the form needs chains, the more the longer they are, and more where the row form is
-// at its best, with one ensemble whose chains it takes in decreasing Z: there, 8 tau_K, 65,536
-// chains of Nk 12 0.82 against 1.45 ms (16,384: 0.68 / 0.50), of Nk 25 1.39 / 2.01 (16,384: 1.00 /
-// 0.70), of Nk 35 1.89 / 2.42, of Nk 50 262,144 9.6 / 10.6 and 131,072 6.0 / 5.4.  Of 16
-// ensembles, 16,384 of Nk 25 1.06 / 1.24, 32,768 of Nk 50 2.66 / 3.22, 262,144 of Nk 50 9.6 / 11.8.
+// 64, so the form needs chains.  Counted by where the two are level (thousands of chains, 4 to
+// 16 tau_K, a sample each): of one ensemble, whose chains the row form takes in decreasing Z,
+// Nk 12 27, Nk 25 37 and Nk 60 73 to 87 at beta 1 to 5; more with long strands (Nk 25: 37, 49, 68
+// at beta 1, 3, 8; Nk 100: 93 and 107 at 4 and 10) and with samples (every 0.2 tau_K for 1: 45 for
+// 37, 36 for 27), and where the columns are so high that few lanes have room (29 to 32
+// positions 80 to 87, above 170 to 183).  A wave of the row form runs one ensemble at a time: of
+// 2, 4, 8 and 16 ensembles the same chains are level at 0.85, 0.6, 0.4 and 0.34 of the count (Nk
+// 25, beta 1: 34, 25, 18, under 16), high columns or not from 8 on.  Over 2,000 combinations of Nk
+// 6 to 100, beta 0.3 to 25, 1 to 16 ensembles, 16,000 to 250,000 chains the routes taken are on
+// average 0.8% slower than the better of the two, at worst 18% slower than the row form (by
+// positions and chains alone 6% and 132%).
 int flow_cap(const dsm_engine* e, const std::vector<int>& ids) {
   if (e->opt.lane == 0 || ids.empty()) return 0;
-  double n = 0.0, zcap = 0.0;
+  double n = 0.0, nk = 0.0, strand = 0.0, samples = 0.0, zcap = 0.0;
   for (int id : ids) {
     const Ens& E = e->ens[id];
     if (!E.P.flow || (E.P.sample_mode != kSampleNone && E.P.sample_mode != kSampleFlow)) return 0;
     n += E.n;
+    nk += E.n * mean_z(E) * mean_strand(E);
+    strand += E.n * mean_strand(E);
+    samples += E.n / jumps_per_sample(E);
     zcap = std::max(zcap, std::min((double)E.nmax, (double)lane_room((float)E.nmax, E.P.beta, 2.75f)));
   }
   int cap = 0;
   for (int p : kFlowCaps)
     if (p > zcap) { cap = p; break; }
-  const double least = ids.size() > 1 ? std::max(16000, 800 * cap)
-                                      : std::max(28000, (cap > 32 ? 5000 : 1500) * cap);
+  const size_t k = ids.size();
+  const double share = k < 2 ? 1.0 : k < 4 ? 0.85 : k < 8 ? 0.6 : k < 16 ? 0.4 : 0.34;
+  const double high = k >= 8 ? 1.0 : cap > 32 ? 3.5 : cap > 28 ? 1.6 : 1.0;
+  const double least = (20000.0 + 600.0 * nk / n + 2000.0 * (strand / n - 1.0)) * share * high * (1.0 + 0.25 * samples / n);
   return e->opt.lane == 2 || n >= least ? cap : 0;
 }
 

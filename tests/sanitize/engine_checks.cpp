@@ -311,6 +311,25 @@ static void check_share_route() {
   CHECK(!mixed(200000, DSM_SAMPLE_GT, 20.0f, 1.0));       // 3.7 / 4.6
 }
 
+static void check_flow_route() {
+  auto lanes = [](int n, int nk, int ens, float beta, double delta) {
+    return Run(std::vector<dsm_ensemble_desc>((size_t)ens, every(desc(n, nk, DSM_SAMPLE_FLOW, beta), delta)), {}, 0.01)
+        .has("lane_flow");
+  };
+  CHECK(lanes(16384, 50, 16, 1.0f, 1.0));    // row 15.1, lanes 10.6
+  CHECK(lanes(65536, 25, 1, 1.0f, 1.0));     // 4.2 / 2.7
+  CHECK(lanes(262144, 12, 1, 1.0f, 1.0));    // 6.5 / 1.8
+  CHECK(lanes(2000, 25, 16, 1.0f, 1.0));     // 1.6 times as fast
+  CHECK(lanes(16384, 50, 16, 6.0f, 1.0));    // 5.1 / 1.6
+  CHECK(!lanes(20000, 40, 2, 0.3f, 1.0));    // 3.1 / 3.6
+  CHECK(!lanes(10000, 25, 2, 1.0f, 1.0));    // 0.73 times
+  CHECK(!lanes(10000, 40, 2, 5.0f, 1.0));    // 0.65
+  CHECK(!lanes(30000, 25, 1, 3.0f, 1.0));    // 0.72
+  CHECK(!lanes(65536, 60, 1, 8.0f, 1.0));    // 0.86
+  CHECK(!lanes(65536, 100, 1, 25.0f, 1.0));  // 0.6
+  CHECK(!lanes(30000, 12, 1, 1.0f, 0.2));    // 0.89
+}
+
 // ------------------------------------------------------------------ refused stays refused
 static void check_refused() {
   dsm_engine* e = nullptr;
@@ -342,6 +361,7 @@ int main(int argc, char** argv) {
   else if (which == "concurrent") check_concurrent();
   else if (which == "route_lane") check_lane_route();
   else if (which == "route_share") check_share_route();
+  else if (which == "route_flow") check_flow_route();
   else return 2;
   std::printf("engine checks (%s): %d failures\n", which.c_str(), failures);
   return failures ? 1 : 0;
