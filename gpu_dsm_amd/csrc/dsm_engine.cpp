@@ -786,12 +786,30 @@ int lane_share(const dsm_engine* e, const std::vector<int>& ids) {
 
 // The solo form (dsm_solo.h) takes the place of the wave forms (bins 2 and up) wherever no
 // chain flows: a jump costs it the same at any length, so it gains most on the long chains
-// (Nk 1000: 2.7 times; Nk 600: 1.8; Nk 300, against the two-chain form: 1.08) and is level
-// with the G = 1 form on short ones.
+// (Nk 1000: 2.7 times; Nk 600: 1.8; Nk 300, against the two-chain form: 1.08).
 bool solo_capable(const dsm_engine* e, const std::vector<int>& ids) {
   for (int id : ids)
     if (!lane_capable(e->ens[id])) return false;
   return e->opt.solo != 0;
+}
+
+// Whether it also takes a whole pass of few chains, many of them short.  There it is faster
+// while a SIMD has one wave or two to run, since it splits and merges strands at twice the
+// cost of the rest, short chains do that most, and three waves a SIMD wait for each other's
+// instructions: wave and solo form, 64 samples a tau_K apart, Nk 10 0.54 / 0.54 ms with 1,000
+// chains and 0.62 / 0.73 with 2,500; Nk 25 0.71 / 0.68, 0.81 / 0.90; Nk 50 1.02 / 0.87, 1.15 /
+// 1.15; Nk 100 1.39 / 1.12, 1.58 / 1.48.  A sample gathers the chain's vectors from memory (an
+// MSD sample is dear to both): every 0.1 tau_K, Nk 30 (0.8 jumps) 0.95 of the wave form's
+// speed with 64 chains, 0.90 with 1,000, 0.71 with 3,000; Nk 100 (2.2) 1.08, 1.04, 0.80.
+bool solo_pays(const dsm_engine* e, const std::vector<int>& ids) {
+  double n = 0.0, nk = 0.0, samples = 0.0;
+  for (int id : ids) {
+    const Ens& E = e->ens[id];
+    n += E.n;
+    nk += E.n * mean_z(E) * mean_strand(E);
+    samples += E.n / jumps_per_sample(E) * (E.P.sample_mode == kSampleMsd ? 0.7 : 1.0);
+  }
+  return n * n <= 45.0 * nk && samples * (0.5 + n / 1500.0) <= n;
 }
 
 // The solo form under flow (dsm_solo_flow.h) takes the place of the wave forms to 512
@@ -987,7 +1005,6 @@ int pass_setup(dsm_engine* e, const std::vector<int>& ids, bool use_ev_stop, Pas
   ps.n_live = (int)n_all;
   const bool records = batched && e->d_lane_tab && e->d_rec && e->d_rec_cap >= e->nstr;
   ps.lane_quads = records ? lane_quads(e, ids) : 0;
-  ps.solo = batched && e->d_lane_tab && solo_capable(e, ids);
   ps.nmax = 0;
   for (int id : ids) ps.nmax = std::max(ps.nmax, e->ens[id].nmax);
   // geometries side by side when chains beyond the first wave-form geometry can occur
@@ -998,6 +1015,8 @@ int pass_setup(dsm_engine* e, const std::vector<int>& ids, bool use_ev_stop, Pas
   ps.flow_cap = batched && e->d_lane_tab ? flow_cap(e, ids) : 0;
   if (e->opt.concurrent > 0 && ps.concurrent) ps.lane_quads = ps.flow_cap = 0;  // (asked for)
   if (ps.lane_quads || ps.flow_cap) ps.concurrent = false;
+  const bool few = !ps.concurrent && ps.n_live <= e->opt.small_per_cu * e->n_cu;
+  ps.solo = batched && e->d_lane_tab && solo_capable(e, ids) && (!few || solo_pays(e, ids));
   ps.solo_flow = batched && !ps.concurrent && e->d_lane_tab && solo_flow_capable(e, ids);
   ps.n_lane = ps.concurrent && records ? lane_share(e, ids) : 0;
   if (n0 == 0) return DSM_OK;
@@ -1182,10 +1201,11 @@ int pass_bins(dsm_engine* e, Pass& ps, bool plain, bool timed, dsm_run_stats* rs
   // batched, one ensemble: the row form takes its chains in decreasing Z, so the chains
   // started last, which set the end of the launch, are the shortest (several ensembles
   // keep their order: a wave runs one ensemble at a time)
-  // A pass of few chains -- at most one wave-form wave per chain at three waves per SIMD
-  // -- is latency-bound: it runs in the wave form, whose per-jump latency is the lowest
-  // (1.79 us per jump against 2.84 us per row-form step of four chains).  Measured:
-  // 1000 chains of Nk 25 +15%, of Nk 100 +92%; 4096 chains of Nk 25 -14%.
+  // A pass of few chains is latency-bound: it runs one chain a wave.  The line, 12 chains a CU
+  // (3,072), lies where the wave form's three waves a SIMD end.  Row, solo and wave form, ms,
+  // 3,000 and 3,500 chains: Nk 10 0.66, 0.75, 0.62 and 0.67, 0.83, 0.84; Nk 25 0.91, 0.90, 0.83 and
+  // 0.95, 1.03, 1.15; Nk 50 1.25, 1.18, 1.15 and 1.29, 1.35, 1.63; Nk 100, whose chains leave the
+  // row form, 2.52, 1.48, 1.57 and 2.52, 1.71, 2.25 (6,000: 2.59, 2.27, 2.77).
   const bool small = !plain && ps.n_live <= e->opt.small_per_cu * e->n_cu;
   const bool flow = !plain && ps.flow_cap > 0 && !small;
   const bool lane = flow || (!plain && ps.lane_quads > 0 && !small);

@@ -330,6 +330,25 @@ static void check_flow_route() {
   CHECK(!lanes(30000, 12, 1, 1.0f, 0.2));    // 0.89
 }
 
+static void check_solo_route() {
+  const int GT = DSM_SAMPLE_GT, MSD = DSM_SAMPLE_MSD;
+  auto first = [](const dsm_ensemble_desc& d) { return Run({d}, {}, 0.01).first(); };
+  CHECK(first(desc(64, 16, GT)) == "solo");                  // wave 0.48, solo 0.46
+  CHECK(first(desc(1000, 25, GT)) == "solo");                // 0.71 / 0.68
+  CHECK(first(desc(3000, 100, GT)) == "solo");               // 1.57 / 1.48
+  CHECK(first(desc(1500, 100, GT, 12.0f)) == "solo");        // 0.98 / 0.66
+  CHECK(first(every(desc(64, 100, GT), 0.1)) == "solo");     // 1.08 times as fast
+  CHECK(first(desc(3000, 8, GT)) == "wave");                 // 0.83
+  CHECK(first(desc(2500, 25, GT)) == "wave");                // 0.81 / 0.90
+  CHECK(first(every(desc(3000, 30, GT), 0.1)) == "wave");    // 0.71
+  CHECK(first(every(desc(1000, 30, GT), 0.1)) == "wave");    // 0.90
+  CHECK(first(every(desc(3000, 100, GT), 0.1)) == "wave");   // 0.80
+  CHECK(first(every(desc(3000, 30, MSD), 0.1)) == "wave");
+  // several ensembles count together; longer chains keep the form however few jumps a sample
+  CHECK(Run({desc(1500, 10, GT), desc(1500, 12, GT)}, {}, 0.01).first() == "wave");
+  CHECK(Run({every(desc(1500, 1000, GT), 0.03)}, {}, 0.01).has("solo"));
+}
+
 // ------------------------------------------------------------------ refused stays refused
 static void check_refused() {
   dsm_engine* e = nullptr;
@@ -362,6 +381,7 @@ int main(int argc, char** argv) {
   else if (which == "route_lane") check_lane_route();
   else if (which == "route_share") check_share_route();
   else if (which == "route_flow") check_flow_route();
+  else if (which == "route_solo") check_solo_route();
   else return 2;
   std::printf("engine checks (%s): %d failures\n", which.c_str(), failures);
   return failures ? 1 : 0;
