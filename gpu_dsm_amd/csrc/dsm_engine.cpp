@@ -818,14 +818,22 @@ bool solo_pays(const dsm_engine* e, const std::vector<int>& ids) {
 // against 0.49 ms; 64 of Nk 30: 0.15 / 0.24; start-up of extension, 3001 chains of Nk 30, a whole
 // pass 0.94 / 1.01).  Beside the other forms of a concurrent pass, where the SIMDs are full,
 // the two are level (bursts of 12 and 24 mixed requests to Nk 512: 53.8 / 51.0, 93.2 / 97.9
-// ms), so those keep the wave forms.
+// ms), so those keep the wave forms.  A chain with a strand of 32 Kuhn steps or more takes the
+// general form of the pair rates for all of its pairs at every jump, which costs more than the
+// rest gains once every other chain has one (strands that long to a chain at equilibrium, and
+// the wave form's time over this one's, 300 and 3,000 chains: 0.34 1.15 and 0.98, 0.6 0.98 and
+// 0.97, 1.3 0.88 and 0.99, 2.3 0.81 and 0.77).
 bool solo_flow_capable(const dsm_engine* e, const std::vector<int>& ids) {
   bool flow = false;
+  double n = 0.0, longs = 0.0;
   for (int id : ids) {
-    flow = flow || e->ens[id].P.flow;
-    if (e->ens[id].P.sample_mode == kSampleMsd) return false;
+    const Ens& E = e->ens[id];
+    flow = flow || E.P.flow;
+    if (E.P.sample_mode == kSampleMsd) return false;
+    n += E.n;
+    if (E.nmax >= kLaneN / 2) longs += E.z_sum_est * std::pow(E.P.beta / (1.0 + E.P.beta), kLaneN / 2 - 1);
   }
-  return flow && e->opt.solo != 0;
+  return flow && e->opt.solo != 0 && longs <= 0.5 * n;
 }
 
 // The lane form's working memory: a record per strand slot, allocated when a pass first can

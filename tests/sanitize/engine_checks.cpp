@@ -349,6 +349,17 @@ static void check_solo_route() {
   CHECK(Run({every(desc(1500, 1000, GT), 0.03)}, {}, 0.01).has("solo"));
 }
 
+static void check_solo_flow_route() {
+  auto first = [](int n, int nk, float beta) { return Run({desc(n, nk, DSM_SAMPLE_FLOW, beta)}, {}, 0.01).first(); };
+  CHECK(first(3001, 30, 1.0f) == "solo_flow");   // wave 0.94, solo 0.82
+  CHECK(first(300, 100, 1.0f) == "solo_flow");   // 1.58 times as fast
+  CHECK(first(64, 100, 8.0f) == "solo_flow");    // 1.23
+  CHECK(first(300, 30, 20.0f) == "solo_flow");   // 1.30: no strand can be long
+  CHECK(first(3000, 100, 30.0f) == "wave");      // 0.85
+  CHECK(first(300, 200, 20.0f) == "wave");       // 0.43 / 0.48
+  CHECK(first(3000, 200, 30.0f) == "wave");      // 0.78
+}
+
 // ------------------------------------------------------------------ refused stays refused
 static void check_refused() {
   dsm_engine* e = nullptr;
@@ -382,6 +393,7 @@ int main(int argc, char** argv) {
   else if (which == "route_share") check_share_route();
   else if (which == "route_flow") check_flow_route();
   else if (which == "route_solo") check_solo_route();
+  else if (which == "route_solo_flow") check_solo_flow_route();
   else return 2;
   std::printf("engine checks (%s): %d failures\n", which.c_str(), failures);
   return failures ? 1 : 0;
