@@ -982,6 +982,7 @@ struct Pass {
   int flow_cap = 0;         // > 0: the lane form under flow with this many positions a chain
   int n_lane = 0;           // concurrent: chains that run in the lane form first
   bool solo = false;        // the solo form instead of the wave forms
+  bool pair2 = false;       // ... but bin 2 two chains a wave
   bool solo_flow = false;   // the same under flow, bins 2 and 3 of a sequential pass
   int nmax = 0;
   bool concurrent = false;  // batched passes only: split by Z, geometries side by side
@@ -1025,6 +1026,12 @@ int pass_setup(dsm_engine* e, const std::vector<int>& ids, bool use_ev_stop, Pas
   if (ps.lane_quads || ps.flow_cap) ps.concurrent = false;
   const bool few = !ps.concurrent && ps.n_live <= e->opt.small_per_cu * e->n_cu;
   ps.solo = batched && e->d_lane_tab && solo_capable(e, ids) && (!few || solo_pays(e, ids));
+  // Of many chains of up to 255 positions with their mean just below bin 2's 128, few are in
+  // bin 2 at the split: the solo form's waves then hold up the row form's without ending the
+  // pass sooner.  Two chains a wave and one, 4 tau_K of 100,000 chains at beta 0.4: Nk 167 (mean
+  // 120) 8.6 / 9.7 ms, Nk 153 (110) 7.0 / 6.9, Nk 181 (130) 11.8 / 9.0; 40,000 of Nk 239 at beta 1
+  // (120) 4.06 / 4.15; 24,000 of Nk 167 level.
+  ps.pair2 = bin_max == 2 && n_all >= 30000.0 && z_est >= 117.0 * n_all && z_est < 127.0 * n_all;
   ps.solo_flow = batched && !ps.concurrent && e->d_lane_tab && solo_flow_capable(e, ids);
   ps.n_lane = ps.concurrent && records ? lane_share(e, ids) : 0;
   if (n0 == 0) return DSM_OK;
@@ -1053,13 +1060,13 @@ int pass_setup(dsm_engine* e, const std::vector<int>& ids, bool use_ev_stop, Pas
 constexpr int kLateFirst = 2;
 int late_last(int bin_max) { return std::max(bin_max, kLateFirst); }
 
-// Launches bin b >= kLateFirst of a batched pass: a solo form, or the wave form `geom`.
-hipError_t launch_wave(dsm_engine* e, const Pass& ps, const KmcArgs& a, int b, int geom, hipStream_t st) {
+// Launches bin b >= kLateFirst of a batched pass: a solo form, or the wave form.
+hipError_t launch_wave(dsm_engine* e, const Pass& ps, const KmcArgs& a, int b, hipStream_t st) {
   if (ps.solo_flow && b <= 3) {
     const int cap = kmc_geom_capacity(b);
     return launch_kmc_solo_flow(a, cap, std::min(ps.n0, device_waves(e, kmc_solo_flow_occupancy(cap))), st);
   }
-  if (!ps.solo) return launch_kmc(a, geom, false, device_blocks(e, geom, false, a.lds_floats, a.ext != 0), st);
+  if (!ps.solo) return launch_kmc(a, b, false, device_blocks(e, b, false, a.lds_floats, a.ext != 0), st);
   const int cap = kmc_geom_capacity(b);
   return launch_kmc_solo(a, cap, std::min(ps.n0, device_waves(e, kmc_solo_occupancy(cap))), st);
 }
@@ -1140,25 +1147,28 @@ int pass_bins_concurrent(dsm_engine* e, Pass& ps, dsm_run_stats* rs) {
   // runs of 21 ms); holding the bulk streams back 100 us lets them all start at once and
   // end at 21 ms, but the bulk then runs at a lower occupancy meanwhile: 114 ms.
   auto stream = [&](int k) { return k == 0 ? e->st : e->xs[k]; };  // xs[0] is not a stream
-  // bin 2 (128 <= Z < 240 at the split) runs two chains per wave in the two-group pair
-  // form unless DSM_OPT_WIDE_PAIR is 0 (a third fewer VALU instructions per jump; on the
-  // 262,144-chain melt 93.6-94.2 ms per window against 95.0-96.7 ms in the G = 1 wave
-  // form, since the strand lengths left the registers and with them most of its spills);
-  // the late round keeps one chain per wave.  Only one-ensemble passes: a wave of two
-  // chains runs one ensemble at a time, and in a serving mix of many ensembles its
-  // segments would wait for each other (the C5 serving stream at horizon 60: 6.2e8
-  // jumps/s with the two-chain form, 8.4e8 with one chain per wave; at horizon 40 the
-  // p50 latency 5.6 s against 0.38 s).  The same switch puts bin 1 (64 <= Z < 128) in the
-  // row form with two register groups, four chains per wave, where the pair form runs two
-  // (one-ensemble 262,144-chain melt: 80-82 ms per window against 89.7-90.3 ms; the C5
-  // stream at horizon 60: 7.9e8 jumps/s against 8.4e8 in the pair form)
+  // bin 2 (128 <= Z < 240 at the split), where it does not run in the solo form, runs two
+  // chains per wave in the two-group pair form unless DSM_OPT_WIDE_PAIR is 0 (a third fewer
+  // VALU instructions per jump; on the 262,144-chain melt 93.6-94.2 ms per window against
+  // 95.0-96.7 ms in the G = 1 wave form, since the strand lengths left the registers and with
+  // them most of its spills); the late round keeps one chain per wave.  Only one-ensemble
+  // passes: a wave of two chains runs one ensemble at a time, and in a serving mix of many
+  // ensembles its segments would wait for each other (the C5 serving stream at horizon 60: 6.2e8
+  // jumps/s with the two-chain form, 8.4e8 with one chain per wave; at horizon 40 the p50
+  // latency 5.6 s against 0.38 s).  The same switch puts bin 1 (64 <= Z < 128) in the row form
+  // with two register groups, four chains per wave, where the pair form runs two (one-ensemble
+  // 262,144-chain melt: 80-82 ms per window against 89.7-90.3 ms; the C5 stream at horizon 60:
+  // 7.9e8 jumps/s against 8.4e8 in the pair form)
   const bool wide = e->opt.wide_pair && ps.n_ens == 1;
   auto first = [&](int b, int k) -> hipError_t {
     if (b > ps.bin_max) return hipSuccess;
     bind(kSplitList + b, late_of(b));
     ++rs->kmc_launches;
-    const int geom = (b == 2 && wide) ? kGeomPair2 : b;
-    return launch_wave(e, ps, a, b, geom, stream(k));
+    if (b == 2 && wide && (ps.pair2 || !ps.solo)) {
+      const int waves = device_blocks(e, kGeomPair2, false, a.lds_floats, a.ext != 0);
+      return launch_kmc(a, kGeomPair2, false, waves, stream(k));
+    }
+    return launch_wave(e, ps, a, b, stream(k));
   };
   HIPCHK(first(5, 0));
   for (int k = 1; k < 4; ++k) HIPCHK(hipStreamWaitEvent(e->xs[k], e->ev_split, 0));
@@ -1178,7 +1188,7 @@ int pass_bins_concurrent(dsm_engine* e, Pass& ps, dsm_run_stats* rs) {
   // bulk, instead of after the whole first round (118-123 ms per window against 123-126
   // with the earlier stream layout)
   bind(kLateList + kLateFirst, late_of(kLateFirst));
-  HIPCHK(launch_wave(e, ps, a, kLateFirst, kLateFirst, e->xs[2]));
+  HIPCHK(launch_wave(e, ps, a, kLateFirst, e->xs[2]));
   rs->kmc_launches += 2;
   HIPCHK(first(3, 0));
   HIPCHK(first(2, 0));
@@ -1187,7 +1197,7 @@ int pass_bins_concurrent(dsm_engine* e, Pass& ps, dsm_run_stats* rs) {
   // late launches: chains that outgrew their geometry, through the larger ones in order
   for (int b = kLateFirst + 1; b <= late_last(ps.bin_max); ++b) {
     bind(kLateList + b, late_of(b));
-    HIPCHK(launch_wave(e, ps, a, b, b, e->st));
+    HIPCHK(launch_wave(e, ps, a, b, e->st));
   }
   if (timed) HIPCHK(hipEventRecord(e->cev[3], e->st));
   ps.pending = timed ? 2 : 0;  // read by pass_times after the caller's next synchronisation
@@ -1256,7 +1266,7 @@ int pass_bins(dsm_engine* e, Pass& ps, bool plain, bool timed, dsm_run_stats* rs
     } else if (k == 0 && lane) {
       HIPCHK(launch_lanes(e, a, ps.lane_quads, ps.n_live, e->st));
     } else if (!plain && b >= kLateFirst) {
-      HIPCHK(launch_wave(e, ps, a, b, b, e->st));
+      HIPCHK(launch_wave(e, ps, a, b, e->st));
     } else {
       HIPCHK(launch_kmc(a, b, plain, device_blocks(e, b, plain, a.lds_floats, a.ext != 0), e->st));
     }

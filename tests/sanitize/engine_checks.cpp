@@ -360,6 +360,21 @@ static void check_solo_flow_route() {
   CHECK(first(3000, 200, 30.0f) == "wave");      // 0.78
 }
 
+static void check_bin2_route() {
+  auto two = [](int n, int nk, float beta) {
+    const Run r({desc(n, nk, DSM_SAMPLE_GT, beta)}, {{DSM_OPT_LANE, 0}}, 0.01);
+    CHECK(r.has("rowpair"));
+    return r.has("pair2");
+  };
+  CHECK(two(100000, 168, 0.4f));   // two chains a wave 8.6, one 9.7 ms
+  CHECK(two(40000, 239, 1.0f));    // 0.98
+  CHECK(!two(16000, 168, 0.4f));   // 1.08
+  CHECK(!two(100000, 154, 0.4f));  // 1.02
+  CHECK(!two(100000, 189, 0.4f));  // 1.5
+  CHECK(!two(40000, 300, 1.0f));   // 1.13
+  CHECK(!two(20000, 600, 1.0f));
+}
+
 // ------------------------------------------------------------------ refused stays refused
 static void check_refused() {
   dsm_engine* e = nullptr;
@@ -394,6 +409,7 @@ int main(int argc, char** argv) {
   else if (which == "route_flow") check_flow_route();
   else if (which == "route_solo") check_solo_route();
   else if (which == "route_solo_flow") check_solo_flow_route();
+  else if (which == "route_bin2") check_bin2_route();
   else return 2;
   std::printf("engine checks (%s): %d failures\n", which.c_str(), failures);
   return failures ? 1 : 0;

@@ -60,7 +60,7 @@ def test_concurrent_option_is_obeyed(checks):
     checks("concurrent")
 
 
-@pytest.mark.parametrize("rule", ["lane", "share", "flow", "solo", "solo_flow"])
+@pytest.mark.parametrize("rule", ["lane", "share", "flow", "solo", "solo_flow", "bin2"])
 def test_route(checks, rule):
     """The form a pass runs in, where the two sides of the rule were measured well apart."""
     checks("route_" + rule)

@@ -86,3 +86,8 @@ def test_lanes_under_flow(n, nk):
           window=4)]], ids=["short", "msd", "long", "flow"])
 def test_waves_that_take_several_chains(ens):
     _same(_run(dict(solo=0), ens, 3.0), _run(dict(solo=1, blocks_per_cu=1), ens, 3.0))
+
+
+def test_bin_2_two_chains_a_wave_beside_the_solo_form():
+    ens = [_still(30000, 167, beta=0.4)]
+    _same(_run(dict(lane=0, solo=0), ens, 1.5), _run(dict(lane=0), ens, 1.5))
