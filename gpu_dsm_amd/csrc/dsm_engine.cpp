@@ -402,6 +402,8 @@ struct dsm_engine {
   uint64_t graph_clock = 0;
   void* h_win = nullptr;
   size_t h_win_cap = 0;
+  WinArgs win;         // the window's parameters, where they fit (win_args)
+  bool win_args = false;
 };
 
 namespace {
@@ -1352,16 +1354,20 @@ int finish_stats(dsm_engine* e, const std::vector<int>& ids, const unsigned long
 
 // The device work of one window after its parameters are set: staging fills, the KMC
 // pass and the sample consumers (correlator update, flow-row reduction).  The window's
-// parameters come from the pinned block h_win (window_block) through stage_window_kernel:
-// all others have been on the device since the ensemble was added.  (Uploading them from
-// pageable memory took two copies and a host wait before the pass.)
+// parameters come with the first launch or from the pinned block h_win (window_block): all
+// others have been on the device since the ensemble was added.  (Uploading them from pageable
+// memory took two copies and a host wait before the pass.)
 int window_launches(dsm_engine* e, const std::vector<int>& act, const std::vector<int64_t>& cnt_off,
                     const std::vector<int64_t>& row_off, const std::vector<int>& cnt, int mode, dsm_run_stats* rs,
                     Pass* timed) {
   int rc;
-  const WinParam* wp = (const WinParam*)e->h_win;
-  HIPCHK(launch_stage_window(wp, (int)act.size(), e->d_ens, (const int*)(wp + act.size()), e->d_corr_cnt,
-                             (int)cnt.size(), e->st));
+  if (e->win_args) {
+    HIPCHK(launch_stage_args(e->win, e->d_ens, e->d_corr_cnt, e->st));
+  } else {
+    const WinParam* wp = (const WinParam*)e->h_win;
+    HIPCHK(launch_stage_window(wp, (int)act.size(), e->d_ens, (const int*)(wp + act.size()), e->d_corr_cnt,
+                               (int)cnt.size(), e->st));
+  }
   for (int id : act) {
     Ens& E = e->ens[id];
     if (E.P.k_end > E.P.k0)
@@ -1394,17 +1400,24 @@ int window_grow(dsm_engine* e, size_t need) {
   return DSM_OK;
 }
 
-// The window's parameters into it.  (Every window ends with a wait for the stream, so no
-// launch reads the last one's any more.)
-int window_block(dsm_engine* e, const std::vector<int>& act, const std::vector<int>& cnt) {
-  const int rc = window_grow(e, sizeof(WinParam) * act.size() + sizeof(int) * cnt.size());
-  if (rc) return rc;
-  WinParam* wp = (WinParam*)e->h_win;
+// The window's parameters, as a kernel argument where they fit and the window is not a
+// captured one, else into the pinned block.  (Every window ends with a wait for the stream,
+// so no launch reads the last one's any more.)
+int window_block(dsm_engine* e, const std::vector<int>& act, const std::vector<int>& cnt, bool captured) {
+  e->win_args = !captured && act.size() <= (size_t)kWinArgs && cnt.size() <= (size_t)kCntArgs;
+  if (!e->win_args) {
+    const int rc = window_grow(e, sizeof(WinParam) * act.size() + sizeof(int) * cnt.size());
+    if (rc) return rc;
+  }
+  WinParam* wp = e->win_args ? e->win.win : (WinParam*)e->h_win;
+  int* to = e->win_args ? e->win.cnt : (int*)(wp + act.size());
   for (size_t q = 0; q < act.size(); ++q) {
     const Ens& E = e->ens[act[q]];
     wp[q] = WinParam{act[q], 0, E.P.t_end, E.P.k0, E.P.k_end};
   }
-  if (!cnt.empty()) std::memcpy(wp + act.size(), cnt.data(), sizeof(int) * cnt.size());
+  if (!cnt.empty()) std::memcpy(to, cnt.data(), sizeof(int) * cnt.size());
+  e->win.n_ens = (int)act.size();
+  e->win.n_cnt = (int)cnt.size();
   return DSM_OK;
 }
 
@@ -1571,8 +1584,9 @@ int advance_impl(dsm_engine* e, const std::vector<int>& ids, const std::vector<d
       return rc;
     Pass timed;
     bool graph_timed = false;
-    if ((rc = window_block(e, act, cnt))) return rc;
-    if (e->opt.graph && mode == DSM_MODE_BATCHED) {
+    const bool captured = e->opt.graph && mode == DSM_MODE_BATCHED;
+    if ((rc = window_block(e, act, cnt, captured))) return rc;
+    if (captured) {
       // captured pass: the launches replayed
       std::vector<int64_t> key{(int64_t)e->gen};
       for (int id : act) {
@@ -1690,7 +1704,7 @@ int dsm_create(int32_t device_id, dsm_engine** out) {
   for (auto& ev : e->ev_bin) HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
   int rc;
   if ((rc = dev_alloc(e, &e->d_cnt, 2 * kNumLists + kZOrderScratch + 1)) || (rc = dev_alloc(e, &e->d_counters, kNumCounters)) ||
-      (rc = dev_alloc(e, &e->d_part, (size_t)kStressBlocks * 9)) || (rc = window_grow(e, 0))) {
+      (rc = dev_alloc(e, &e->d_part, (size_t)kStressBlocks * 9))) {
     dsm_destroy(e);
     return rc;
   }

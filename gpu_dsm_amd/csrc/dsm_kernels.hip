@@ -599,14 +599,14 @@ __global__ void __launch_bounds__(256) corr_parts_kernel(const double* part, int
   out[pt] = acc;
 }
 
-// ------------------------------------------------------------------ captured passes
-// Head of a captured window pass: the window's parameters, which change every window,
-// come from a block of pinned host memory the host fills before each replay, so the
-// graph itself never changes: (t_end, k0, k_end) of every ensemble of the pass into its
-// EnsParams, then the correlator level counters.  One block.
-__global__ void __launch_bounds__(256) stage_window_kernel(const WinParam* __restrict__ wp, int n_ens,
-                                                           EnsParams* P, const int* __restrict__ cnt_src,
-                                                           int* cnt_dst, int n_cnt) {
+// ------------------------------------------------------------------ window parameters
+// Head of a window pass: (t_end, k0, k_end) of every ensemble of the pass into its
+// EnsParams, then the correlator level counters.  One block.  In a captured pass they come
+// from a block of pinned host memory the host fills before each replay, so the graph itself
+// never changes; so do those of many ensembles.  Otherwise they are the launch's argument
+// (the pinned block costs an engine 0.25 ms to have and to give back).
+__device__ __forceinline__ void stage_window(const WinParam* wp, int n_ens, EnsParams* P, const int* cnt_src,
+                                             int* cnt_dst, int n_cnt) {
   for (int i = threadIdx.x; i < n_ens; i += blockDim.x) {
     const WinParam w = wp[i];
     P[w.ens].t_end = w.t_end;
@@ -614,6 +614,14 @@ __global__ void __launch_bounds__(256) stage_window_kernel(const WinParam* __res
     P[w.ens].k_end = w.k_end;
   }
   for (int i = threadIdx.x; i < n_cnt; i += blockDim.x) cnt_dst[i] = cnt_src[i];
+}
+__global__ void __launch_bounds__(256) stage_window_kernel(const WinParam* __restrict__ wp, int n_ens,
+                                                           EnsParams* P, const int* __restrict__ cnt_src,
+                                                           int* cnt_dst, int n_cnt) {
+  stage_window(wp, n_ens, P, cnt_src, cnt_dst, n_cnt);
+}
+__global__ void __launch_bounds__(256) stage_args_kernel(WinArgs w, EnsParams* P, int* cnt_dst) {
+  stage_window(w.win, w.n_ens, P, w.cnt, cnt_dst, w.n_cnt);
 }
 
 // ------------------------------------------------------------------ ensemble stress now
@@ -1046,6 +1054,11 @@ hipError_t launch_corr_reduce(const double* C, int ld, const int* stall, int cha
 hipError_t launch_stage_window(const WinParam* wp, int n_ens, EnsParams* P, const int* cnt_src, int* cnt_dst,
                                int n_cnt, hipStream_t st) {
   hipLaunchKernelGGL(stage_window_kernel, dim3(1), dim3(256), 0, st, wp, n_ens, P, cnt_src, cnt_dst, n_cnt);
+  return hipGetLastError();
+}
+
+hipError_t launch_stage_args(const WinArgs& w, EnsParams* P, int* cnt_dst, hipStream_t st) {
+  hipLaunchKernelGGL(stage_args_kernel, dim3(1), dim3(256), 0, st, w, P, cnt_dst);
   return hipGetLastError();
 }
 

@@ -126,8 +126,9 @@ struct KappaArg {
 };
 hipError_t launch_chain_stress(const ChainArrays& ch, int chain0, int n, const float kappa[9], double* part,
                                hipStream_t st);
-// window parameters (t_end, k0, k_end per ensemble) and correlator counters of a captured
-// pass, from host-pinned memory into EnsParams and cnt_dst
+// window parameters (t_end, k0, k_end per ensemble) and correlator counters, from
+// host-pinned memory into EnsParams and cnt_dst, or given with the launch
+hipError_t launch_stage_args(const WinArgs& w, EnsParams* P, int* cnt_dst, hipStream_t st);
 hipError_t launch_stage_window(const WinParam* wp, int n_ens, EnsParams* P, const int* cnt_src, int* cnt_dst,
                                int n_cnt, hipStream_t st);
 // invariant violations of chains chain0..chain0+n-1 added to out[0..6] (see dsm_check_state)

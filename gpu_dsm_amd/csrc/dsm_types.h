@@ -63,6 +63,14 @@ struct WinParam {
   int64_t k_end;
 };
 
+// A window's parameters and correlator counters as a kernel argument: few ensembles
+constexpr int kWinArgs = 16, kCntArgs = 256;
+struct WinArgs {
+  WinParam win[kWinArgs];
+  int cnt[kCntArgs];
+  int n_ens, n_cnt;
+};
+
 struct ChainArrays {
   int* Z;
   int* nk;

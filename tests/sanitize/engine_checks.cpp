@@ -375,6 +375,25 @@ static void check_bin2_route() {
   CHECK(!two(20000, 600, 1.0f));
 }
 
+// ------------------------------------------------------------------ window parameters
+static void check_window() {
+  // a window's parameters travel with its launch: no pinned memory but for many ensembles or a
+  // captured window
+  const auto d = desc(40, 30, DSM_SAMPLE_GT);
+  fake::pinned = 0;
+  for (int k : {1, 2, 16}) Run(std::vector<dsm_ensemble_desc>((size_t)k, d), {});
+  dsm_ensemble_desc big = d;
+  big.corr_levels = 40;
+  Run({big, big}, {});
+  CHECK(fake::pinned == 0);
+  Run(std::vector<dsm_ensemble_desc>(17, d), {});
+  CHECK(fake::pinned == 1);
+  Run({big, big, big}, {});
+  CHECK(fake::pinned == 2);
+  Run({d}, {{DSM_OPT_GRAPH, 1}}, 9.0);
+  CHECK(fake::pinned == 3);
+}
+
 // ------------------------------------------------------------------ refused stays refused
 static void check_refused() {
   dsm_engine* e = nullptr;
@@ -410,6 +429,7 @@ int main(int argc, char** argv) {
   else if (which == "route_solo") check_solo_route();
   else if (which == "route_solo_flow") check_solo_flow_route();
   else if (which == "route_bin2") check_bin2_route();
+  else if (which == "window") check_window();
   else return 2;
   std::printf("engine checks (%s): %d failures\n", which.c_str(), failures);
   return failures ? 1 : 0;

@@ -17,7 +17,7 @@
 namespace fake {
 std::vector<Launch> launches;
 int nulls = 0;
-int64_t allocs = 0, fail_from = 0, fail_to = 0, live_bytes = 0, live_count = 0;
+int64_t allocs = 0, fail_from = 0, fail_to = 0, live_bytes = 0, live_count = 0, pinned = 0;
 size_t capacity = (size_t)1 << 33;
 static std::map<void*, size_t> sizes;
 static int handle;
@@ -66,7 +66,7 @@ hipError_t hipFree(void* p) {
   std::free(p);
   return hipSuccess;
 }
-hipError_t hipHostMalloc(void** p, size_t n, unsigned) { *p = std::malloc(n); return hipSuccess; }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) { ++pinned; *p = std::malloc(n); return hipSuccess; }
 hipError_t hipHostFree(void* p) { std::free(p); return hipSuccess; }
 hipError_t hipMemGetInfo(size_t* f, size_t* t) {
   *t = capacity;
@@ -285,6 +285,9 @@ hipError_t launch_stage_window(const WinParam* wp, int n_ens, EnsParams* P, cons
   }
   if (use(cnt_dst, n_cnt)) for (int i = 0; i < n_cnt; ++i) cnt_dst[i] = cnt_src[i];
   return hipSuccess;
+}
+hipError_t launch_stage_args(const WinArgs& w, EnsParams* P, int* cnt_dst, hipStream_t st) {
+  return launch_stage_window(w.win, w.n_ens, P, w.cnt, cnt_dst, w.n_cnt, st);
 }
 hipError_t launch_copy_probe(const void*, void*, size_t, int, hipStream_t) { return hipSuccess; }
 hipError_t launch_scan_probe(const float*, float*, int, int, hipStream_t) { return hipSuccess; }

@@ -20,6 +20,7 @@ extern int nulls;                     // launches that were given a null pointer
 extern int64_t allocs;                // hipMalloc calls so far
 extern int64_t fail_from, fail_to;    // the calls (counted from 1) in this range fail
 extern int64_t live_bytes, live_count;
+extern int64_t pinned;                // hipHostMalloc calls so far
 extern size_t capacity;               // device memory; a call beyond it fails
 inline void fail_next(int64_t k, int64_t n = 1) { fail_from = allocs + k; fail_to = fail_from + n - 1; }
 inline void fail_none() { fail_from = fail_to = 0; }

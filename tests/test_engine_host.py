@@ -64,3 +64,7 @@ def test_concurrent_option_is_obeyed(checks):
 def test_route(checks, rule):
     """The form a pass runs in, where the two sides of the rule were measured well apart."""
     checks("route_" + rule)
+
+
+def test_window_parameters_need_no_pinned_memory(checks):
+    checks("window")
