@@ -631,39 +631,77 @@ __global__ void __launch_bounds__(256) stage_args_kernel(WinArgs w, EnsParams* P
 // pending from the chain's last jump (dt_prev; the reference applies it with olddt).
 // Chains that have stalled are left out.  A fixed grid of kStressBlocks blocks strides
 // over the chains, one wave a chain, one lane a strand (the arrays are read in whole
-// lines; one thread a chain took 85 us for 20,011 chains of Z ~ 100); block b writes its
-// partial sums to part[9b .. 9b+8] (xx yy zz xy yz zx Lpp Z count), which the host adds in
+// lines; one thread a chain took 101 us for 20,011 chains of Z ~ 100, call included, this 42).
+// A wave looks at 16 chains a turn (four lanes each; their headers' latency once) and does
+// them together where none is longer than 16, else four at a time, 16 lanes a chain, where
+// none of the four is longer than 64 (200,000 chains of Nk 6: 39 us a thread a chain, 98 a
+// wave a chain, 38 so; 60,000 of Nk 12 31, 40, 31; 131,072 of Nk 100 281, 83, 59).  Block b writes
+// its partial sums to part[9b .. 9b+8] (xx yy zz xy yz zx Lpp Z count), which the host adds in
 // block order, so the result does not depend on timing.
 constexpr int kStressWaves = 16;
+struct StressSum {
+  double v[9];
+  __device__ __forceinline__ void add(const ChainArrays& ch, const KappaArg& K, int64_t s, double dt) {
+    double x = ch.Qx[s], y = ch.Qy[s], z = ch.Qz[s];
+    if (dt != 0.0) {
+      const double x1 = x + dt * ((double)K.k[0] * x + (double)K.k[1] * y + (double)K.k[2] * z);
+      const double y1 = y + dt * ((double)K.k[3] * x + (double)K.k[4] * y + (double)K.k[5] * z);
+      const double z1 = z + dt * ((double)K.k[6] * x + (double)K.k[7] * y + (double)K.k[8] * z);
+      x = x1; y = y1; z = z1;
+    }
+    const double t3 = 3.0 / (double)ch.N[s];
+    v[0] -= t3 * x * x; v[1] -= t3 * y * y; v[2] -= t3 * z * z;
+    v[3] -= t3 * x * y; v[4] -= t3 * y * z; v[5] -= t3 * x * z;
+    v[6] += sqrt(x * x + y * y + z * z);
+  }
+};
 __global__ void __launch_bounds__(64 * kStressWaves) chain_stress_kernel(ChainArrays ch, int chain0, int n, KappaArg K,
                                                                          double* part) {
   __shared__ double red[9][kStressWaves];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  double acc[9];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = lane >> 4, rl = lane & 15, ql = lane & 3;
+  if ((int)blockIdx.x * kStressWaves >= n) {  // no chain is left for it
+    if (threadIdx.x < 9) part[blockIdx.x * 9 + threadIdx.x] = 0.0;
+    return;
+  }
+  StressSum S;
+  double (&acc)[9] = S.v;
 #pragma unroll
   for (int q = 0; q < 9; ++q) acc[q] = 0.0;
-  for (int i = blockIdx.x * kStressWaves + wave; i < n; i += gridDim.x * kStressWaves) {
-    const int c = chain0 + i;
-    if (ch.stall[c] != 0) continue;
-    const int Z = ch.Z[c];
-    const int64_t b = ch.base[c];
-    const double dt = (double)ch.dt_prev[c];
-    for (int k = lane; k < Z; k += 64) {
-      double x = ch.Qx[b + k], y = ch.Qy[b + k], z = ch.Qz[b + k];
-      if (dt != 0.0) {
-        const double x1 = x + dt * ((double)K.k[0] * x + (double)K.k[1] * y + (double)K.k[2] * z);
-        const double y1 = y + dt * ((double)K.k[3] * x + (double)K.k[4] * y + (double)K.k[5] * z);
-        const double z1 = z + dt * ((double)K.k[6] * x + (double)K.k[7] * y + (double)K.k[8] * z);
-        x = x1; y = y1; z = z1;
+  const int stride = gridDim.x * kStressWaves;
+  for (int i0 = blockIdx.x * kStressWaves + wave; i0 < n; i0 += 16 * stride) {
+    // lanes 4g .. 4g+3 have chain i0 + g * stride
+    const int i = i0 + (lane >> 2) * stride, c = chain0 + i;
+    int Z = 0;
+    int64_t b = 0;
+    float dt = 0.0f;
+    if (i < n && ch.stall[c] == 0) {
+      Z = ch.Z[c];
+      b = ch.base[c];
+      dt = ch.dt_prev[c];
+      if (ql == 0) {
+        acc[7] += (double)Z;
+        acc[8] += 1.0;
       }
-      const double t3 = 3.0 / (double)ch.N[b + k];
-      acc[0] -= t3 * x * x; acc[1] -= t3 * y * y; acc[2] -= t3 * z * z;
-      acc[3] -= t3 * x * y; acc[4] -= t3 * y * z; acc[5] -= t3 * x * z;
-      acc[6] += sqrt(x * x + y * y + z * z);
     }
-    if (lane == 0) {
-      acc[7] += (double)Z;
-      acc[8] += 1.0;
+    if (i0 + stride < n && !__ballot(Z > 16)) {
+      for (int k = ql; k < Z; k += 4) S.add(ch, K, b + k, (double)dt);
+      continue;
+    }
+    for (int h = 0; h < 4 && i0 + 4 * h * stride < n; ++h) {
+      const int Zr = __shfl(Z, 16 * h + 4 * row);
+      const int64_t br = __shfl(b, 16 * h + 4 * row);
+      const float dr = __shfl(dt, 16 * h + 4 * row);
+      if (i0 + (4 * h + 1) * stride < n && !__ballot(Zr > 64)) {
+        for (int k = rl; k < Zr; k += 16) S.add(ch, K, br + k, (double)dr);
+      } else {
+        for (int r = 0; r < 4; ++r) {
+          const int Zc = __shfl(Zr, 16 * r);
+          if (Zc == 0) continue;
+          const int64_t bc = __shfl(br, 16 * r);
+          const double dc = (double)__shfl(dr, 16 * r);
+          for (int k = lane; k < Zc; k += 64) S.add(ch, K, bc + k, dc);
+        }
+      }
     }
   }
 #pragma unroll
@@ -685,40 +723,86 @@ __global__ void __launch_bounds__(64 * kStressWaves) chain_stress_kernel(ChainAr
 // out[2] sum of N != Nk, out[3] an end strand (index 0 or Z-1, Z > 1) with Q != 0,
 // out[4] a non-finite Q or CD rate, out[5] stalled chains, out[6] chains whose clock is
 // below t_min.  The counters (7 x uint64) must be zero on entry.  One wave a chain, one lane
-// a strand (one thread a chain took 121 us for 20,011 chains of Z ~ 100).
+// a strand (one thread a chain took 130 us for 20,011 chains of Z ~ 100, call included, this
+// 42), or 16 or four shorter chains at a time as above (200,000 of Nk 6: 41, 124, 41 us; 60,000
+// of Nk 12 32, 53, 33; 131,072 of Nk 100 572, 97, 72).
+struct StrandChecks {
+  long long all;
+  bool n, f, e;
+  __device__ __forceinline__ void add(const ChainArrays& ch, int64_t b, int k, int Z) {
+    const int N = ch.N[b + k];
+    n = n || N < 1;
+    all += N;
+    const float x = ch.Qx[b + k], y = ch.Qy[b + k], z = ch.Qz[b + k];
+    f = f || !isfinite(x) || !isfinite(y) || !isfinite(z) || (k < Z - 1 && !isfinite(ch.w[b + k]));
+    if (Z > 1 && (k == 0 || k == Z - 1)) e = e || x != 0.f || y != 0.f || z != 0.f;
+  }
+  // the findings of the lanes of `mask` (all: their sum), to be counted by one of them
+  __device__ __forceinline__ void count(uint64_t mask, bool mine, int nk, unsigned int (&v)[7]) const {
+    const bool bn = (__ballot(n) & mask) != 0, bf = (__ballot(f) & mask) != 0, be = (__ballot(e) & mask) != 0;
+    if (mine) {
+      v[1] += bn;
+      v[2] += all != nk;
+      v[3] += be;
+      v[4] += bf;
+    }
+  }
+};
 __global__ void __launch_bounds__(256) check_state_kernel(ChainArrays ch, int chain0, int n, double t_min,
                                                           unsigned long long* out) {
   __shared__ unsigned int tot[7];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = lane >> 4, rl = lane & 15, ql = lane & 3;
   if (threadIdx.x < 7) tot[threadIdx.x] = 0;
   __syncthreads();
-  unsigned int v[7] = {0, 0, 0, 0, 0, 0, 0};  // the same on every lane of a wave
-  for (int i = blockIdx.x * 4 + wave; i < n; i += gridDim.x * 4) {
-    const int c = chain0 + i;
-    const int Z = ch.Z[c], nk = ch.nk[c];
-    if (ch.stall[c] != 0) v[5]++;
-    if (!(ch.t[c] >= t_min)) v[6]++;
-    if (Z < 1 || Z > nk || Z > ch.cap[c]) { v[0]++; continue; }
-    const int64_t b = ch.base[c];
-    long long all = 0;
-    bool bad_n = false, bad_f = false, bad_e = false;
-    for (int k = lane; k < Z; k += 64) {
-      const int N = ch.N[b + k];
-      bad_n = bad_n || N < 1;
-      all += N;
-      const float x = ch.Qx[b + k], y = ch.Qy[b + k], z = ch.Qz[b + k];
-      bad_f = bad_f || !isfinite(x) || !isfinite(y) || !isfinite(z) || (k < Z - 1 && !isfinite(ch.w[b + k]));
-      if (Z > 1 && (k == 0 || k == Z - 1)) bad_e = bad_e || x != 0.f || y != 0.f || z != 0.f;
+  unsigned int v[7] = {0, 0, 0, 0, 0, 0, 0};  // on every fourth lane
+  const int stride = gridDim.x * 4;
+  for (int i0 = blockIdx.x * 4 + wave; i0 < n; i0 += 16 * stride) {
+    const int i = i0 + (lane >> 2) * stride, c = chain0 + i;  // lanes 4g .. 4g+3: chain i0 + g * stride
+    int Z = 0, nk = 0;
+    int64_t b = 0;
+    if (i < n) {
+      Z = ch.Z[c];
+      nk = ch.nk[c];
+      b = ch.base[c];
+      const bool in = Z >= 1 && Z <= nk && Z <= ch.cap[c];
+      if (ql == 0) {
+        v[0] += !in;
+        v[5] += ch.stall[c] != 0;
+        v[6] += !(ch.t[c] >= t_min);
+      }
+      Z = in ? Z : 0;
     }
-    for (int d = 32; d > 0; d >>= 1) all += __shfl_xor(all, d, 64);
-    if (__ballot(bad_n)) v[1]++;
-    if (all != nk) v[2]++;
-    if (__ballot(bad_e)) v[3]++;
-    if (__ballot(bad_f)) v[4]++;
+    if (i0 + stride < n && !__ballot(Z > 16)) {
+      StrandChecks s{0, false, false, false};
+      for (int k = ql; k < Z; k += 4) s.add(ch, b, k, Z);
+      for (int d = 2; d > 0; d >>= 1) s.all += __shfl_xor(s.all, d, 64);
+      s.count(0xfull << (lane & ~3), ql == 0 && Z > 0, nk, v);
+      continue;
+    }
+    for (int h = 0; h < 4 && i0 + 4 * h * stride < n; ++h) {
+      const int Zr = __shfl(Z, 16 * h + 4 * row), nr = __shfl(nk, 16 * h + 4 * row);
+      const int64_t br = __shfl(b, 16 * h + 4 * row);
+      if (i0 + (4 * h + 1) * stride < n && !__ballot(Zr > 64)) {
+        StrandChecks s{0, false, false, false};
+        for (int k = rl; k < Zr; k += 16) s.add(ch, br, k, Zr);
+        for (int d = 8; d > 0; d >>= 1) s.all += __shfl_xor(s.all, d, 64);
+        s.count(0xffffull << (16 * row), rl == 0 && Zr > 0, nr, v);
+      } else {
+        for (int r = 0; r < 4; ++r) {
+          const int Zc = __shfl(Zr, 16 * r);
+          if (Zc == 0) continue;
+          const int64_t bc = __shfl(br, 16 * r);
+          StrandChecks s{0, false, false, false};
+          for (int k = lane; k < Zc; k += 64) s.add(ch, bc, k, Zc);
+          for (int d = 32; d > 0; d >>= 1) s.all += __shfl_xor(s.all, d, 64);
+          s.count(~0ull, lane == 16 * r, nr, v);
+        }
+      }
+    }
   }
 #pragma unroll
   for (int q = 0; q < 7; ++q)
-    if (lane == 0 && v[q]) atomicAdd(tot + q, v[q]);
+    if (ql == 0 && v[q]) atomicAdd(tot + q, v[q]);
   __syncthreads();
   if (threadIdx.x < 7 && tot[threadIdx.x]) atomicAdd(out + threadIdx.x, (unsigned long long)tot[threadIdx.x]);
 }
