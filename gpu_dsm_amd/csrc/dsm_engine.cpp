@@ -1941,7 +1941,8 @@ int dsm_init_equilibrium(dsm_engine* e, int32_t ens) {
   if (!E) return fail(DSM_ERR_ARG, "no ensemble %d", ens);
   int rc = set_device(e);
   if (rc || (rc = ensure_device(e))) return rc;
-  HIPCHK(launch_init_eq(e->ch, e->d_ens, e->d_tabs, E->chain0, E->n, e->st));
+  // (level between Z of 10, few chains, and 16, many)
+  HIPCHK(launch_init_eq(e->ch, e->d_ens, e->d_tabs, E->chain0, E->n, mean_z(*E) <= 10.0 ? 4 : 16, e->st));
   HIPCHK(hipStreamSynchronize(e->st));
   E->k_cur = E->P.sample_mode == kSampleFlow ? 1 : 0;
   E->flow_rows.clear();

@@ -25,7 +25,7 @@
 namespace dsm {
 
 // ------------------------------------------------------------------ equilibrium init
-// A 16-lane row per chain of first .. first+n-1.  Inner Kuhn-step boundary i (1 <= i < nk)
+// G lanes (a 16-lane row, or four) per chain of first .. first+n-1.  Inner Kuhn-step boundary i (1 <= i < nk)
 // carries an entanglement iff Philox word (i-1) < 2^32/(1+beta): Z-1 ~ Binomial(nk-1,
 // 1/(1+beta)) and N|Z uniform over compositions (the laws of common/chain.cu:38-88).
 // Internal strands get Q ~ N(0, N/3) per component (common/chain.cu:90-102), links get CD
@@ -33,12 +33,36 @@ namespace dsm {
 // the background distribution when there is one (:141-149).  A lane has the four words of
 // one Philox call in each part; a cut's strand index is the count of cuts before it, and
 // the cut positions are kept in the strand-length array until the lengths are their
-// differences.  (One thread a chain, all of it in turn: 66 us for 16,384 chains of Nk 50,
-// 3,379 us for the 262,144-chain melt.)
+// differences.  One thread a chain, all of it in turn, a row and a quad of lanes, 262,144 chains,
+// us: Nk 100 1039, 225, 324; Nk 30 362, 108, 100; Nk 12 106, 90, 49; Nk 6 55, 85, 42; Nk 4 31, 76, 34;
+// 20,000 of Nk 20 43, 22, 24.
+// inclusive sums over the G lanes of a chain, and their last lane's value
+template <int G>
+__device__ __forceinline__ int lanes_scan(int v, int gl) {
+  if constexpr (G == 16) {
+    v += dppi<kRowShr1>(v, 0);
+    v += dppi<kRowShr2>(v, 0);
+    v += dppi<kRowShr4>(v, 0);
+    v += dppi<kRowShr8>(v, 0);
+  } else {
+    const int a = dppi<kRowShr1>(v, 0);
+    v += gl >= 1 ? a : 0;
+    const int b = dppi<kRowShr2>(v, 0);
+    v += gl >= 2 ? b : 0;
+  }
+  return v;
+}
+template <int G>
+__device__ __forceinline__ int lanes_last(int v) {
+  if constexpr (G == 16) return row_last(v);
+  else return dppi<0xFF>(v, 0);  // quad_perm 3 3 3 3
+}
+template <int G>
 __global__ void __launch_bounds__(256) init_eq_kernel(ChainArrays ch, const EnsParams* ens, const float* tabs,
                                                         int first, int n) {
-  const int rl = threadIdx.x & 15;
-  const int idx = blockIdx.x * 16 + (threadIdx.x >> 4);
+  static_assert(G == 16 || G == 4, "a row of lanes, or a quad");
+  const int rl = threadIdx.x & (G - 1);
+  const int idx = blockIdx.x * (256 / G) + threadIdx.x / G;
   const bool on = idx < n;  // rows past the end run along, without a store
   const int c = first + (on ? idx : 0);
   const EnsParams& P = ens[ch.ens[c]];
@@ -47,7 +71,7 @@ __global__ void __launch_bounds__(256) init_eq_kernel(ChainArrays ch, const EnsP
   const uint32_t cid = ch.cid[c];
   const int64_t b = ch.base[c];
   int Z = 0;
-  for (int w0 = 0; __ballot(w0 < nk); w0 += 64) {
+  for (int w0 = 0; __ballot(w0 < nk); w0 += 4 * G) {
     const int wi = w0 + 4 * rl;  // words wi..wi+3: boundaries wi+1..wi+4; boundary nk always ends a strand
     uint4 x = make_uint4(0, 0, 0, 0);
     if (wi < nk - 1) x = philox4x32_10(make_uint4((uint32_t)(wi >> 2), 0u, cid, kPurposeInitCut), k0, k1);
@@ -59,12 +83,8 @@ __global__ void __launch_bounds__(256) init_eq_kernel(ChainArrays ch, const EnsP
       cut[k] = i == nk || (i < nk && word[k] < P.cut_threshold) ? 1 : 0;
       cnt += cut[k];
     }
-    int before = cnt;  // inclusive count over the row
-    before += dppi<kRowShr1>(before, 0);
-    before += dppi<kRowShr2>(before, 0);
-    before += dppi<kRowShr4>(before, 0);
-    before += dppi<kRowShr8>(before, 0);
-    const int total = row_last(before);
+    const int before = lanes_scan<G>(cnt, rl);  // inclusive
+    const int total = lanes_last<G>(before);
     int at = Z + before - cnt;
 #pragma unroll
     for (int k = 0; k < 4; ++k)
@@ -75,10 +95,10 @@ __global__ void __launch_bounds__(256) init_eq_kernel(ChainArrays ch, const EnsP
     Z += total;
   }
   // The lanes' cut positions are complete (same wave, in issue order); lengths from the
-  // last block of 16 strands down, each read before the strand below is rewritten
+  // last block of G strands down, each read before the strand below is rewritten
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   const int zmax = Z;
-  for (int s0 = (zmax - 1) & ~15; __ballot(s0 >= 0); s0 -= 16) {
+  for (int s0 = (zmax - 1) & ~(G - 1); __ballot(s0 >= 0); s0 -= G) {
     const int k = s0 + rl;
     const bool in = s0 >= 0 && k < Z;
     int N = 0;
@@ -99,7 +119,7 @@ __global__ void __launch_bounds__(256) init_eq_kernel(ChainArrays ch, const EnsP
     }
   }
   const float* pd = tabs + P.pd_off;
-  for (int s0 = 0; __ballot(s0 < Z); s0 += 64) {
+  for (int s0 = 0; __ballot(s0 < Z); s0 += 4 * G) {
     const int k = s0 + 4 * rl;
     if (k >= Z || !on) continue;
     uint4 x = make_uint4(0, 0, 0, 0), y = x;
@@ -1015,9 +1035,12 @@ int kmc_max_blocks_per_cu(int geom, bool plain, int lds_floats, bool ext) {
 
 
 hipError_t launch_init_eq(const ChainArrays& ch, const EnsParams* ens, const float* tabs, int first, int n,
-                          hipStream_t st) {
+                          int lanes, hipStream_t st) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(init_eq_kernel, dim3((n + 15) / 16), dim3(256), 0, st, ch, ens, tabs, first, n);
+  if (lanes == 16)
+    hipLaunchKernelGGL(init_eq_kernel<16>, dim3((n + 15) / 16), dim3(256), 0, st, ch, ens, tabs, first, n);
+  else
+    hipLaunchKernelGGL(init_eq_kernel<4>, dim3((n + 63) / 64), dim3(256), 0, st, ch, ens, tabs, first, n);
   return hipGetLastError();
 }
 

@@ -82,8 +82,8 @@ hipError_t launch_kmc_solo(const KmcArgs& a, int cap, int grid, hipStream_t st);
 // The solo form for passes with flow, cap 256 or 512.
 int kmc_solo_flow_occupancy(int cap);
 hipError_t launch_kmc_solo_flow(const KmcArgs& a, int cap, int grid, hipStream_t st);
-// chains first .. first+n-1
-hipError_t launch_init_eq(const ChainArrays& ch, const EnsParams* ens, const float* tabs, int first, int n,
+// chains first .. first+n-1, `lanes` (4 or 16) lanes a chain
+hipError_t launch_init_eq(const ChainArrays& ch, const EnsParams* ens, const float* tabs, int first, int n, int lanes,
                           hipStream_t st);
 hipError_t launch_fill_u32(void* p, uint32_t v, int64_t n, hipStream_t st);
 hipError_t launch_iota(int* p, int start, int n, hipStream_t st);

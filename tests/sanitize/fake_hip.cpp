@@ -168,7 +168,9 @@ hipError_t launch_kmc_solo_flow(const KmcArgs& a, int cap, int grid, hipStream_t
   jumps(a, Launch{"solo_flow", cap, grid, 0, false, false});
   return hipSuccess;
 }
-hipError_t launch_init_eq(const ChainArrays& ch, const EnsParams* ens, const float* tabs, int first, int n, hipStream_t) {
+hipError_t launch_init_eq(const ChainArrays& ch, const EnsParams* ens, const float* tabs, int first, int n, int lanes,
+                          hipStream_t) {
+  if (lanes != 4 && lanes != 16) return hipErrorInvalidValue;
   chains(ch, first, n);
   for (int c = first; c < first + n; ++c) {
     const EnsParams* P = ens + ch.ens[c];
