@@ -4,17 +4,21 @@ The reference fixes its launch shape at compile time (threads per block and chai
 call, common/textures_surfaces.h:22-24, common/ensemble.cu:47; sync interval,
 common/ensemble_kernel.cu:41-42).  Here the per-pass layout is chosen per workload:
 
-  small_per_cu      passes of few chains run in the wave form (lowest per-jump latency)
-                    instead of the row/pair forms (most jumps per instruction);
-  concurrent        geometries side by side on four streams or one after another;
+  small_per_cu      passes of few chains run one chain per wave (the solo or the wave form:
+                    lowest per-jump latency) instead of in the row/pair forms (most jumps per
+                    instruction);
+  concurrent        geometries side by side on four streams or one after another (1 also
+                    keeps a pass out of the lane forms but for a concurrent pass's short chains);
   split_margin      how close to a wave-form geometry's capacity a chain may start in it;
   lds_table_floats  rate tables staged in LDS (one copy per wave) or read from global memory;
   blocks_per_cu     persistent waves per CU (occupancy below the register limit);
   window            samples per staging window: the stress / correlator sync interval;
-  wide_pair         chains with 128 <= Z < 240 two per wave (two register groups each)
-                    instead of one per wave, and those with 64 <= Z < 128 four per wave
-                    instead of two, in concurrent passes of one ensemble.
+  wide_pair         chains with 64 <= Z < 128 four per wave (two register groups) instead of
+                    two, and those with 128 <= Z < 240 that the solo form does not take two
+                    per wave instead of one, in concurrent passes of one ensemble.
 
+The lane and solo forms (options lane, solo) are left at their defaults: the engine takes
+them by rules on counts, strands and samples, and the options above are timed under those.
 No option changes a result (every chain makes the same jumps with the same Philox
 numbers under any setting; tests/test_gpu_options.py), so tuning is free to pick on
 speed alone.  tune() builds the workload in a scratch engine from the same ensemble

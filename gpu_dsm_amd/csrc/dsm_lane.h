@@ -17,7 +17,7 @@
 // a 12-byte record {|Q|^2, w, N} per position in `rec` (L2 / Infinity Cache); Q in the
 // chain arrays; header and quad sums in registers.
 //
-// What bounds it (131,072 chains of Nk 100, one 16 tau_K window, 76 positions: 5.2 ms against
+// What bounds it (131,072 chains of Nk 100, one 16 tau_K window, 76 positions: 5.0 ms against
 // 9.0 ms in the row form plus 0.76 ms for its overflow in the wave form): per jump 35 VALU
 // instructions instead of 103, issued on about half of the cycles.  LDS holds two waves a
 // SIMD (512 lanes a CU at 76 positions), so the loads from L2 and Infinity Cache
@@ -1069,7 +1069,7 @@ __global__ void __launch_bounds__(64 * kLaneWaves) __attribute__((amdgpu_waves_p
   const int n_work = *a0.n_work;
   // The first chains go by place, the others by the queue: the list is in decreasing
   // order of work, so the workgroup's waves take far-apart parts of it, and waves w and
-  // 7 - w, which share a SIMD, opposite ones.
+  // w + 4, which share a SIMD, opposite ones (parts w and 7 - w).
   const int n_first = kLaneWaves * gridDim.x * lanes;
   const int wv = threadIdx.x >> 6, part = wv < kLaneWaves / 2 ? wv : kLaneWaves + kLaneWaves / 2 - 1 - wv;
   int first_ent = C.lane < lanes ? (part * (int)gridDim.x + (int)blockIdx.x) * lanes + C.lane : -1;

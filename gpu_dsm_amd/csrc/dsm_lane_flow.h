@@ -12,10 +12,13 @@
 // and merges move the column behind them; nothing but loading, writing back and samples'
 // rows touches memory.  Same operands in the same order as the other forms.
 //
-// What bounds it: VALU issue, about 60 instructions a position and jump on the 25 to 64 lanes
-// of a wave that LDS has room for (64 up to 16 positions, 30 at 36).  262,144 chains of 16
-// sheared ensembles, 8 tau_K: Nk 50 9.6 against 11.8 ms in the row form, Nk 25 3.4 / 7.9, Nk 12
-// 1.5 / 5.5.  Strand vectors in registers (64 lanes at 44 positions) spilled hundreds of them.
+// What bounds it: VALU issue, about 60 instructions a position and jump, on the 27 to 64
+// lanes of a wave that LDS has room for (flow_max_lanes: 64 up to 16 positions, 33 at 32, 31
+// at 36, 27 at 40), or fewer where the chains come in rounds of that many (262,144 at 36
+// positions: five rounds of 26).  262,144 chains of 16 sheared ensembles, 8 tau_K: Nk 50 9.6
+// against 11.8 ms in the row form, Nk 25 3.4 / 7.9, Nk 12 1.5 / 5.5.  A version with the strand
+// vectors in registers (64 lanes at 44 positions) spilled hundreds of them; whether it would
+// have with its elements selected by value only (dsm_solo_flow.h) was not tried.
 #pragma once
 #include "dsm_lane.h"
 

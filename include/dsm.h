@@ -73,8 +73,9 @@ typedef struct {
   uint64_t z_sum;       /* sum over jumps of the chain's Z (algorithmic byte model) */
   double kmc_ms;        /* device time of the KMC passes (HIP events: the sum of the launches of a
                            sequential pass; the span from split to late round of a concurrent one) */
-  double first_kmc_ms;  /* device time of each pass's first launch only (the row form; the wave form
-                           for a pass of few chains) */
+  double first_kmc_ms;  /* device time of one launch of each pass: the first of a sequential one (the
+                           lane, row, solo or wave form), the merged launch of the row forms of a
+                           concurrent one (which runs beside others), all of a captured window */
   double total_ms;      /* host wall time of the call */
   int64_t kmc_launches;
   int64_t first_launches;
@@ -97,23 +98,28 @@ int dsm_mem_info(int32_t device_id, size_t* free_bytes, size_t* total_bytes);
    setting -- only how passes are laid out on the device.  The autotuner
    (gpu_dsm_amd/autotune.py) sweeps them. */
 #define DSM_OPT_PLAIN_JUMPS 1       /* plain form: jumps per chain per launch (default 1, the reference's) */
-#define DSM_OPT_SMALL_PER_CU 2      /* passes of at most this many chains per CU run in the wave form (12) */
+#define DSM_OPT_SMALL_PER_CU 2      /* sequential passes of at most this many chains per CU run one chain per wave:
+                                       in the wave form, or in the solo form where that is the faster (12) */
 #define DSM_OPT_SPLIT_MARGIN 3      /* concurrent pass: chains within capacity/value of a wave-form geometry
                                        start in the next one (16; 0 = none) */
 #define DSM_OPT_LDS_TABLE_FLOATS 4  /* rate tables go to LDS when they fit this many floats per wave (2816) */
-#define DSM_OPT_CONCURRENT 5        /* geometries side by side: -1 by the pass's lengths, 0 never, 1 always */
+#define DSM_OPT_CONCURRENT 5        /* geometries side by side: -1 by the pass's lengths, 0 never, 1 always
+                                       (of passes with a chain that can leave the row form; the lane forms then
+                                       take chains only as part of such a pass) */
 #define DSM_OPT_BLOCKS_PER_CU 6     /* cap on persistent waves per CU (0 = the occupancy limit); the lane forms, with
                                        eight waves a workgroup, then have workgroups on some of the CUs alone */
 #define DSM_OPT_WINDOW 7            /* samples per staging window of ensembles added later (256) */
 #define DSM_OPT_GRAPH 8             /* 1: batched windows run as captured HIP graphs, replayed with the
                                        window's parameters in a pinned block (0) */
-#define DSM_OPT_WIDE_PAIR 9         /* concurrent pass of one ensemble: chains with 128 <= Z < 240 run two
-                                       per wave and those with 64 <= Z < 128 four (1), or one and two (0)
-                                       (1) */
+#define DSM_OPT_WIDE_PAIR 9         /* concurrent pass of one ensemble: chains with 64 <= Z < 128 run four
+                                       per wave and those with 128 <= Z < 240, where the solo form does not
+                                       take them, two (1), or two and one (0) (1) */
 #define DSM_OPT_LANE 10             /* batched passes, without flow or of flow alone: chains that stay short enough
-                                       run one per lane: 1 by their count, 0 never, 2 always (1) */
+                                       run one per lane: 1 where their count, strand lengths and samples let it
+                                       pay, 0 never, 2 always (1) */
 #define DSM_OPT_SOLO 11             /* batched passes: few or long chains (under flow: few, to 512 positions) run
-                                       in the solo forms (1) or the wave forms (0) (1) */
+                                       in the solo forms where those are the faster (1) or in the wave forms (0)
+                                       (1) */
 int dsm_set_option(dsm_engine* e, int32_t key, int32_t value);
 int dsm_get_option(dsm_engine* e, int32_t key, int32_t* value);
 
