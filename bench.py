@@ -21,11 +21,12 @@ Printed: one JSON line.
                achieved = VALU wave-instructions per jump (committed rocprofv3 PMC summary
                of the same pass, profiles/) x jumps per step / pass time per step, against
                the issue peak of 256 CUs x 4 SIMDs x 2.4 GHz / 4 cycles per wave64
-               instruction.  hbm_byte_model: the algorithmic bytes 20 Z + 32 per jump (a full
-               re-read of the chain per jump) over the same time against 8 TB/s;
-               hbm_measured: the pass's HBM bytes (PMC, FETCH_SIZE/WRITE_SIZE calibrated on
-               a copy) over the same time.
-  c2           the monodisperse melt (131,072 chains, Nk 100) as a secondary line.
+               instruction.  traffic and past_l2: the pass's bytes past the L2s (PMC,
+               FETCH_SIZE/WRITE_SIZE calibrated on a copy) and their rate over the same time;
+               the Infinity Cache serves most of them, so they are no fraction of HBM's rate.
+  c2           the monodisperse melt (131,072 chains, Nk 100) as a secondary line.  Its lane-form
+               kernel issues VALU instructions on about half of the cycles; the rest is the
+               latency of the loads and of the splits, merges and samples done by rows.
   plain_vs_batched  the 16-ensemble shear sweep (16 x 16,384 chains, Nk 50): plain = each
                ensemble in its own launch sequence, state in HBM between launches
                (1 jump per chain per launch, the reference's structure, and 16 per launch);
@@ -57,7 +58,6 @@ import numpy as np
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
-PEAK_HBM_GBS = 8000.0
 # VALU issue peak of MI355X: 256 CUs x 4 SIMDs, one wave64 instruction per 4 cycles at 2.4 GHz
 N_SIMD, CLOCK_GHZ = 1024, 2.4
 PEAK_VALU_G = N_SIMD * CLOCK_GHZ / 4.0  # G wave-instructions per second
@@ -113,26 +113,21 @@ def timed_steps(eng, ids, args, record):
     return dict(jumps=ev, z_sum=zs, wall_s=wall, kmc_ms=kmc_ms, first_ms=first_ms, t_end=t)
 
 
-def roofline(tot, steps, cnt, pass_ms):
-    """VALU roofline of the pass (bound per the counters), with both HBM views."""
+def roofline(tot, steps, cnt, kernel_ms, bound):
+    """VALU roofline of the pass or kernel timed (issue rate against its peak; `bound` per the
+    counters), with its traffic past the L2s."""
     jumps_step = tot["jumps"] / steps
-    bytes_model = (20.0 * tot["z_sum"] + 32.0 * tot["jumps"]) / steps
     valu_pj = cnt.get("valu_per_jump")
-    hbm_pj = cnt.get("hbm_bytes_per_jump")
-    achieved = valu_pj * jumps_step / (pass_ms * 1e-3) / 1e9 if valu_pj else None
-    model_gbs = bytes_model / (pass_ms * 1e-3) / 1e9
-    meas = hbm_pj * jumps_step if hbm_pj else None
-    return {"bound": "valu", "achieved": achieved, "peak": PEAK_VALU_G, "unit": "G VALU wave-instructions/s",
+    l2_pj = cnt.get("bytes_past_l2_per_jump")
+    achieved = valu_pj * jumps_step / (kernel_ms * 1e-3) / 1e9 if valu_pj else None
+    meas = l2_pj * jumps_step if l2_pj else None
+    return {"bound": bound, "achieved": achieved, "peak": PEAK_VALU_G, "unit": "G VALU wave-instructions/s",
             "frac": achieved / PEAK_VALU_G if achieved else None, "traffic": meas,
             "valu_per_jump": valu_pj, "waves_per_simd": cnt.get("waves_per_simd"),
-            "pass_ms": pass_ms, "jumps_per_pass": jumps_step,
+            "pass_ms": kernel_ms, "jumps_per_pass": jumps_step,
             "counters": cnt.get("source"),
-            "hbm_byte_model": {"bytes_per_pass": bytes_model, "achieved_GBs": model_gbs, "peak_GBs": PEAK_HBM_GBS,
-                               "frac": model_gbs / PEAK_HBM_GBS,
-                               "note": "algorithmic 20 Z + 32 bytes per jump (a full re-read of the chain per jump)"},
-            "hbm_measured": {"bytes_per_pass": meas,
-                             "achieved_GBs": meas / (pass_ms * 1e-3) / 1e9 if meas else None,
-                             "frac": meas / (pass_ms * 1e-3) / 1e9 / PEAK_HBM_GBS if meas else None}}
+            "past_l2": {"bytes_per_pass": meas,
+                        "achieved_GBs": meas / (kernel_ms * 1e-3) / 1e9 if meas else None}}
 
 
 def run_c3(g, args, record):
@@ -366,7 +361,7 @@ def main():
             json.dump({"workload": "c2", "advance_jumps": record}, open(args.record, "w"))
         copy_ms = g.probe_copy(1 << 30, 5)  # the byte counters' reference in the same profiled run
         print(json.dumps({"c2_jumps_per_s": c2["jumps"] / c2["wall_s"], "jumps": c2["jumps"],
-                          "row_kernel_ms": c2["first_ms"] / args.steps, "copy_ms": copy_ms}))
+                          "lane_kernel_ms": c2["first_ms"] / args.steps, "copy_ms": copy_ms}))
         return
     c3 = run_c3(g, args, record)
     if args.record:
@@ -378,9 +373,10 @@ def main():
         return
     value = c3["jumps"] / c3["wall_s"]
     pass_ms = c3["kmc_ms"] / args.steps
-    rl = roofline(c3, args.steps, counters("kmc_pass_c3_counters.json"), pass_ms)
+    rl = roofline(c3, args.steps, counters("kmc_pass_c3_counters.json"), pass_ms, "valu")
     c2 = run_c2(g, args, [])
-    rl2 = roofline(c2, args.steps, counters("kmc_lane_form_c2_counters.json"), c2["first_ms"] / args.steps)
+    rl2 = roofline(c2, args.steps, counters("kmc_lane_form_c2_counters.json"), c2["first_ms"] / args.steps,
+                   "valu and latency")
     pvb = None if args.no_plain else run_plain_vs_batched(g, args)
     copy_bytes = 1 << 30
     copy_ms = g.probe_copy(copy_bytes, 20)
@@ -437,7 +433,7 @@ def main():
         "c2": {"workload": "monodisperse melt, 131072 chains, Nk=100, beta=1, CD on, G(t) p=16 m=2, %d tau_K per "
                            "step" % args.window,
                "jumps_per_s": c2["jumps"] / c2["wall_s"], "ms_per_step": 1e3 * c2["wall_s"] / args.steps,
-               "row_kernel_avg_ms": c2["first_ms"] / args.steps, "roofline_row_kernel": rl2, "G0": c2["G0"]},
+               "lane_kernel_avg_ms": c2["first_ms"] / args.steps, "roofline_lane_kernel": rl2, "G0": c2["G0"]},
         "plain_vs_batched": pvb,
         "copy_probe": {"bytes": copy_bytes, "ms": copy_ms, "GBs": 2.0 * copy_bytes / (copy_ms * 1e-3) / 1e9,
                        "note": "plain 16-byte device copy, read+write bytes over time: achievable HBM rate"},
