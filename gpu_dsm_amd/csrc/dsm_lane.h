@@ -17,7 +17,7 @@
 // a 12-byte record {|Q|^2, w, N} per position in `rec` (L2 / Infinity Cache); Q in the
 // chain arrays; header and quad sums in registers.
 //
-// What bounds it (131,072 chains of Nk 100, one 16 tau_K window, 76 positions: 5.0 ms against
+// What bounds it (131,072 chains of Nk 100, one 16 tau_K window, 76 positions: 5.1 ms against
 // 9.0 ms in the row form plus 0.76 ms for its overflow in the wave form): per jump 35 VALU
 // instructions instead of 103, issued on about half of the cycles.  LDS holds two waves a
 // SIMD (512 lanes a CU at 76 positions), so the loads from L2 and Infinity Cache
